@@ -7,7 +7,9 @@
 // four waves owns one (batch, KV head) and 128 of its (position, head)
 // columns, so every K/V tile it stages in LDS serves 128 query rows.  (A
 // decode step with its key range split into short slices runs the same code
-// as one-wave blocks, one slice each.)  A wave's
+// as one-wave blocks, one slice each.  A prefill too short to fill the GPU
+// that way takes blocks of eight waves whose two or four groups divide the
+// keys of the same columns and merge in LDS: dispatch.hpp.)  A wave's
 // 32 "columns" are consecutive (position, head) pairs in position-major
 // order: 32 / G whole positions when G divides 32; any G up to 32 works (for
 // Qwen3-14B's 5 a position's heads may straddle two waves).  Per 32 keys:
@@ -33,9 +35,7 @@
 // here than leaving the overlap to the other block's wave on the same SIMD
 // (two waves per SIMD at this register count).  Tile rows are 256 bytes with
 // the 16-byte chunks XOR-swizzled by row so that the K fragment reads
-// (ds_read_b128) and the V transpose reads hit distinct LDS banks.  Prefill
-// grids are renumbered so that the query blocks of one (batch, KV head) run on
-// one XCD and share its L2.
+// (ds_read_b128) and the V transpose reads hit distinct LDS banks.
 //
 // Generic path (any head_dim <= 256, any strides): one wave per query row,
 // keys in order, lanes over the head dimension -- the reference's own
@@ -57,14 +57,10 @@ namespace q3k
         typedef __attribute__((address_space(3))) void lds_void_t;
 
         constexpr int kAttD = kAttHeadDim;
-        constexpr int kKeyTile = kAttKeyTile;                 // keys per pipeline step
         constexpr int kRowBytes = kAttD * 2;                  // one K or V row in LDS
-        constexpr int kHalfBytes = kKeyTile * kRowBytes;      // the K (or V) rows of a tile
         constexpr int kRowsPerLoad = kWave * 16 / kRowBytes;  // rows one wave-wide 16-byte load fills
         constexpr int kAhead = 2;                             // LDS fragment reads in flight ahead of use
         constexpr float kLazyMax = 8.0f;                      // log2 headroom before the softmax reference moves
-        constexpr int kAttWaves = kAttWavesPerBlock;          // waves per matrix-core block
-        constexpr int kAttBlock = kAttWaves * kWave;
         constexpr float kLog2e = 1.4426950408889634f;
 
         struct AttnArgs
@@ -82,10 +78,12 @@ namespace q3k
             int32_t D;
             int32_t qblocks;
             float scale;
-            // split-K: the key range is cut into `splits` slices of split_keys
-            // keys (a multiple of the tile); slice results (unnormalised O^T,
-            // reference max and sum) go to part_o [splits, rows, D] and part_ml
-            // [splits, rows, 2] and attn_combine_kernel merges them
+            // split-K: the key range is cut into at most `splits` slices of
+            // split_keys keys (a multiple of the tile); a query block takes the
+            // slices its causal range reaches.  With more than one, slice results
+            // (unnormalised O^T, reference max and sum) go to part_o [splits,
+            // rows, D] and part_ml [splits, rows, 2] and attn_combine_kernel
+            // merges them
             int32_t splits;
             int32_t split_keys;
             float *part_o;
@@ -142,56 +140,55 @@ namespace q3k
 
         // ---- tile operations shared by the kernels ------------------------------
 
-        // Loading a key tile's K (or V) rows into LDS from a block of WAVES
-        // waves: wave w fills rows (kKeyTile / WAVES) w .. of a buffer,
-        // kRowsPerLoad rows per load; lane j lands in slot j % 16 of row j / 16
-        // and so fetches the chunk that slot holds.  A tile's loads address from
-        // a buffer resource based at its first key, so the per-lane byte offsets
-        // (tile_offsets) stay fixed: 32-bit, checked by the launcher.  Rows past
-        // n_keys repeat the last key (finite data, later masked or weighted by
-        // zero).
-        template <int WAVES>
+        // Loading a key tile's K (or V) rows into LDS by CW waves: wave cw fills
+        // rows (KEYS / CW) cw .. of a buffer, kRowsPerLoad rows per load; lane j
+        // lands in slot j % 16 of row j / 16 and so fetches the chunk that slot
+        // holds.  A tile's loads address from a buffer resource based at its first
+        // key, so the per-lane byte offsets (tile_offsets) stay fixed: 32-bit,
+        // checked by the launcher.  Rows past n_keys repeat the last key (finite
+        // data, later masked or weighted by zero).
+        template <int CW, int KEYS>
         struct Staging
         {
-            static constexpr int kRows = kKeyTile / WAVES;      // rows of a tile per wave
+            static constexpr int kRows = KEYS / CW;             // rows of a tile per wave
             static constexpr int kLoads = kRows / kRowsPerLoad; // loads per wave per K (or V) tile
         };
 
-        template <int WAVES, typename Slot>
-        __device__ __forceinline__ void tile_offsets(int wave, int lane, int32_t byte_stride, Slot slot,
-                                                     int32_t (&voff)[Staging<WAVES>::kLoads])
+        template <int CW, int KEYS, typename Slot>
+        __device__ __forceinline__ void tile_offsets(int cw, int lane, int32_t byte_stride, Slot slot,
+                                                     int32_t (&voff)[Staging<CW, KEYS>::kLoads])
         {
-            const int st_row = Staging<WAVES>::kRows * wave + lane / 16;
+            const int st_row = Staging<CW, KEYS>::kRows * cw + lane / 16;
 #pragma unroll
-            for (int x = 0; x < Staging<WAVES>::kLoads; ++x)
+            for (int x = 0; x < Staging<CW, KEYS>::kLoads; ++x)
             {
                 const int r = st_row + kRowsPerLoad * x;
                 voff[x] = r * byte_stride + 16 * slot(r, lane % 16);
             }
         }
 
-        template <int WAVES, typename Slot>
+        template <int CW, int KEYS, typename Slot>
         __device__ __forceinline__ void load_tile_rows(int tile, unsigned char *buf, const uint16_t *base,
-                                                       int64_t row_stride, int32_t byte_stride, int32_t n_keys,
-                                                       int wave, int lane, const int32_t (&voff)[Staging<WAVES>::kLoads],
+                                                       int64_t row_stride, int32_t byte_stride, int32_t n_keys, int cw,
+                                                       int lane, const int32_t (&voff)[Staging<CW, KEYS>::kLoads],
                                                        Slot slot)
         {
-            constexpr int kRows = Staging<WAVES>::kRows;
-            const int32_t key0 = tile * kKeyTile;
+            constexpr int kRows = Staging<CW, KEYS>::kRows;
+            const int32_t key0 = tile * KEYS;
             const __amdgpu_buffer_rsrc_t rs = tile_rsrc(base + static_cast<int64_t>(key0) * row_stride);
-            unsigned char *dst = buf + kRows * wave * kRowBytes;
-            if (key0 + kKeyTile <= n_keys)
+            unsigned char *dst = buf + kRows * cw * kRowBytes;
+            if (key0 + KEYS <= n_keys)
             {
 #pragma unroll
-                for (int x = 0; x < Staging<WAVES>::kLoads; ++x)
+                for (int x = 0; x < Staging<CW, KEYS>::kLoads; ++x)
                     dma16(rs, voff[x], dst + kRowsPerLoad * x * kRowBytes);
             }
             else
             {
                 const int last = n_keys - 1 - key0;
-                const int st_row = kRows * wave + lane / 16;
+                const int st_row = kRows * cw + lane / 16;
 #pragma unroll
-                for (int x = 0; x < Staging<WAVES>::kLoads; ++x)
+                for (int x = 0; x < Staging<CW, KEYS>::kLoads; ++x)
                 {
                     const int r = st_row + kRowsPerLoad * x;
                     const int rr = r < last ? r : last;
@@ -199,24 +196,6 @@ namespace q3k
                 }
             }
         }
-
-        // both halves of the staging for one kernel: K and V bases, strides and
-        // the per-lane offsets, as lambdas over the kernel's locals
-#define Q3K_ATTN_STAGING(WAVES)                                                                                      \
-    const uint16_t *kbase = a.k + b * a.ks0 + kvh * a.ks2;                                                            \
-    const uint16_t *vbase = a.v + b * a.vs0 + kvh * a.vs2;                                                            \
-    const int32_t kstride = static_cast<int32_t>(a.ks1) * 2, vstride = static_cast<int32_t>(a.vs1) * 2;               \
-    const auto kslot = [](int r, int c) __attribute__((always_inline)) { return k_slot(r, c); };                                                     \
-    const auto vslot = [](int r, int c) __attribute__((always_inline)) { return v_slot(r, c); };                                                     \
-    int32_t k_voff[Staging<WAVES>::kLoads], v_voff[Staging<WAVES>::kLoads];                                           \
-    tile_offsets<WAVES>(wave, lane, kstride, kslot, k_voff);                                                          \
-    tile_offsets<WAVES>(wave, lane, vstride, vslot, v_voff);                                                          \
-    auto load_k = [&](int tile, unsigned char *buf) __attribute__((always_inline)) {                                                                 \
-        load_tile_rows<WAVES>(tile, buf, kbase, a.ks1, kstride, n_keys, wave, lane, k_voff, kslot);                   \
-    };                                                                                                                \
-    auto load_v = [&](int tile, unsigned char *buf) __attribute__((always_inline)) {                                                                 \
-        load_tile_rows<WAVES>(tile, buf, vbase, a.vs1, vstride, n_keys, wave, lane, v_voff, vslot);                   \
-    };
 
         // Q fragments of the lane's column.  A padding column (s_col >= S) reads
         // the last position's row instead: its scores are always masked (a wave
@@ -245,33 +224,35 @@ namespace q3k
                             8 * (tj % 2);
         }
 
-        // S^T = K Q^T for the 64 keys of a tile (sacc[hh]: keys 32 hh .. + 31).
+        // S^T = K Q^T for the 32 HH keys of a tile (sacc[hh]: keys 32 hh .. + 31).
         // The K fragment reads run kAhead steps ahead of the MFMAs that use them.
+        template <int HH>
         __device__ __forceinline__ void qk_tile(const unsigned char *k_lds, const bf16x8_t (&qf)[kAttD / 16], int li,
-                                                int lg, f32x16_t (&sacc)[2])
+                                                int lg, f32x16_t (&sacc)[HH])
         {
             auto read_k = [&](int c, int hh) __attribute__((always_inline)) {
                 return *reinterpret_cast<const Vec8 *>(k_lds + (32 * hh + li) * kRowBytes +
                                                        16 * k_slot(li, 2 * c + lg));
             };
-            sacc[0] = f32x16_t{};
-            sacc[1] = f32x16_t{};
-            Vec8 kq[kAhead + 1][2];
+#pragma unroll
+            for (int hh = 0; hh < HH; ++hh)
+                sacc[hh] = f32x16_t{};
+            Vec8 kq[kAhead + 1][HH];
 #pragma unroll
             for (int c = 0; c < kAhead; ++c)
 #pragma unroll
-                for (int hh = 0; hh < 2; ++hh)
+                for (int hh = 0; hh < HH; ++hh)
                     kq[c][hh] = read_k(c, hh);
 #pragma unroll
             for (int c = 0; c < kAttD / 16; ++c)
             {
                 if (c + kAhead < kAttD / 16)
 #pragma unroll
-                    for (int hh = 0; hh < 2; ++hh)
+                    for (int hh = 0; hh < HH; ++hh)
                         kq[(c + kAhead) % (kAhead + 1)][hh] = read_k(c + kAhead, hh);
                 __builtin_amdgcn_sched_barrier(0); // keep the reads ahead of these MFMAs
 #pragma unroll
-                for (int hh = 0; hh < 2; ++hh)
+                for (int hh = 0; hh < HH; ++hh)
                     sacc[hh] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(kq[c % (kAhead + 1)][hh]), qf[c], sacc[hh],
                                                                        0, 0, 0);
             }
@@ -279,11 +260,12 @@ namespace q3k
 
         // Scores of keys past the column's causal limit and of padding columns
         // become -inf (before the max).
-        __device__ __forceinline__ void mask_tile(f32x16_t (&sacc)[2], int32_t key0, int lg, int32_t last_key,
+        template <int HH>
+        __device__ __forceinline__ void mask_tile(f32x16_t (&sacc)[HH], int32_t key0, int lg, int32_t last_key,
                                                   bool col_ok)
         {
 #pragma unroll
-            for (int hh = 0; hh < 2; ++hh)
+            for (int hh = 0; hh < HH; ++hh)
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                 {
@@ -302,12 +284,13 @@ namespace q3k
         // not move).  An all-masked column keeps m = -inf and weight 0.  The max
         // of the raw scores times the (positive) scale is the max of the scaled
         // ones.
-        __device__ __forceinline__ float softmax_tile(const f32x16_t (&sacc)[2], float scale2, float &m, float &l,
-                                                      bf16x8_t (&phi)[2][2], bf16x8_t (&plo)[2][2])
+        template <int HH>
+        __device__ __forceinline__ float softmax_tile(const f32x16_t (&sacc)[HH], float scale2, float &m, float &l,
+                                                      bf16x8_t (&phi)[HH][2], bf16x8_t (&plo)[HH][2])
         {
             float mloc = sacc[0][0];
 #pragma unroll
-            for (int hh = 0; hh < 2; ++hh)
+            for (int hh = 0; hh < HH; ++hh)
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     mloc = fmaxf(mloc, sacc[hh][r]);
@@ -319,7 +302,7 @@ namespace q3k
             const float alpha = move ? __builtin_amdgcn_exp2f(m - m_use) : 1.0f;
             float psum = 0.0f;
 #pragma unroll
-            for (int hh = 0; hh < 2; ++hh)
+            for (int hh = 0; hh < HH; ++hh)
 #pragma unroll
                 for (int mm = 0; mm < 2; ++mm)
                 {
@@ -363,8 +346,9 @@ namespace q3k
         // O^T += V^T P^T for one tile: step i covers the 16-key chunk i / 4
         // (hh = i / 8, mm = (i / 4) % 2) and dims 32 (i % 4) .. + 31.  The
         // transpose reads run kAhead steps ahead of the MFMAs that use them.
+        template <int HH>
         __device__ __forceinline__ void pv_tile(const unsigned char *v_lds, const int (&v_off)[kAttD / 32],
-                                                const bf16x8_t (&phi)[2][2], const bf16x8_t (&plo)[2][2],
+                                                const bf16x8_t (&phi)[HH][2], const bf16x8_t (&plo)[HH][2],
                                                 f32x16_t (&o)[kAttD / 32])
         {
             auto read_v = [&](int i) __attribute__((always_inline)) {
@@ -380,9 +364,9 @@ namespace q3k
             for (int i = 0; i < kAhead; ++i)
                 vq[i] = read_v(i);
 #pragma unroll
-            for (int i = 0; i < 16; ++i)
+            for (int i = 0; i < 8 * HH; ++i)
             {
-                if (i + kAhead < 16)
+                if (i + kAhead < 8 * HH)
                     vq[(i + kAhead) % (kAhead + 1)] = read_v(i + kAhead);
                 __builtin_amdgcn_sched_barrier(0); // keep the reads ahead of these MFMAs
                 const int dt = i % 4, hh = i / 8, mm = (i / 4) % 2;
@@ -391,87 +375,105 @@ namespace q3k
             }
         }
 
-        // The lane's column of the result: bf16 O / l, or with split keys the
-        // slice's unnormalised O^T, reference max and sum for the merge.
-        __device__ __forceinline__ void store_column(const AttnArgs &a, int sp, int64_t b, int32_t s_col, int h_col,
-                                                     int lg, const f32x16_t (&o)[kAttD / 32], float m, float l)
+        // Dims 32 dt .. + 31 of the lane's column of the result: bf16 O / l, or
+        // with split keys the slice's unnormalised O^T for the merge (and, once
+        // per column, its reference max and sum: store_ml).
+        __device__ __forceinline__ void store_dims(const AttnArgs &a, bool split, int sp, int64_t row, int dt, int lg,
+                                                   const f32x16_t &o, float inv)
         {
-            if (a.splits > 1)
+            if (split)
             {
-                const int64_t slot = static_cast<int64_t>(sp) * a.rows + (b * a.S + s_col) * a.Hq + h_col;
-                float *po = a.part_o + slot * kAttD;
-#pragma unroll
-                for (int dt = 0; dt < kAttD / 32; ++dt)
-#pragma unroll
-                    for (int q4 = 0; q4 < 4; ++q4)
-                    {
-                        const float4 w = {o[dt][4 * q4], o[dt][4 * q4 + 1], o[dt][4 * q4 + 2], o[dt][4 * q4 + 3]};
-                        *reinterpret_cast<float4 *>(po + dt * 32 + 8 * q4 + 4 * lg) = w;
-                    }
-                if (lg == 0)
-                {
-                    a.part_ml[2 * slot] = m;
-                    a.part_ml[2 * slot + 1] = l;
-                }
-                return;
-            }
-            const float inv = 1.0f / l;
-            uint16_t *orow = a.out + ((b * a.S + s_col) * a.Hq + h_col) * kAttD;
-#pragma unroll
-            for (int dt = 0; dt < kAttD / 32; ++dt)
+                float *po = a.part_o + (static_cast<int64_t>(sp) * a.rows + row) * kAttD;
 #pragma unroll
                 for (int q4 = 0; q4 < 4; ++q4)
                 {
-                    const int d = dt * 32 + 8 * q4 + 4 * lg;
-                    uint2 w;
-                    w.x = pack_rne(o[dt][4 * q4] * inv, o[dt][4 * q4 + 1] * inv);
-                    w.y = pack_rne(o[dt][4 * q4 + 2] * inv, o[dt][4 * q4 + 3] * inv);
-                    *reinterpret_cast<uint2 *>(orow + d) = w;
+                    const float4 w = {o[4 * q4], o[4 * q4 + 1], o[4 * q4 + 2], o[4 * q4 + 3]};
+                    *reinterpret_cast<float4 *>(po + dt * 32 + 8 * q4 + 4 * lg) = w;
                 }
+                return;
+            }
+            uint16_t *orow = a.out + row * kAttD;
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4)
+            {
+                uint2 w;
+                w.x = pack_rne(o[4 * q4] * inv, o[4 * q4 + 1] * inv);
+                w.y = pack_rne(o[4 * q4 + 2] * inv, o[4 * q4 + 3] * inv);
+                *reinterpret_cast<uint2 *>(orow + dt * 32 + 8 * q4 + 4 * lg) = w;
+            }
+        }
+        __device__ __forceinline__ void store_ml(const AttnArgs &a, int sp, int64_t row, float m, float l)
+        {
+            reinterpret_cast<float2 *>(a.part_ml)[static_cast<int64_t>(sp) * a.rows + row] = make_float2(m, l);
         }
 
         // ---- the matrix-core kernel ---------------------------------------------
 
-        // G is the group size Hq / Hkv, or 0 for a group size that does not
-        // divide 32 (taken from the arguments at run time).  The S * G columns
-        // of one (batch, KV head), (position, head) pairs in position-major
-        // order, go 32 to a wave and 32 * WAVES to a block; for a G that
-        // divides 32 a wave thus holds 32 / G whole positions, otherwise a
-        // position's heads may straddle two waves or blocks.
-        template <int G, int WAVES>
-        __global__ __launch_bounds__(WAVES * kWave) void attn_mfma_kernel(AttnArgs a)
+        // G is the group size Hq / Hkv, or 0 for a group size taken from the
+        // arguments at run time.  The S * G columns of one (batch, KV head),
+        // (position, head) pairs in position-major order, go 32 to a wave and
+        // 32 * CW to a block; for a G that divides 32 a wave thus holds 32 / G
+        // whole positions, otherwise a position's heads may straddle two waves or
+        // blocks.  The block's KW groups of CW waves hold the same columns and
+        // take the key tiles (32 HH keys) in turn: group kw tiles kw, kw + KW, ...
+        // Their partial results meet in LDS at the end.  A wave's step is a chain
+        // (its MFMAs, then the softmax, the load wait, the barrier: 1.5 us a 64-key
+        // tile alone on a CU), so a launch of few blocks is as long as its longest
+        // chain; groups cut the chain without the global write and read of split
+        // keys (512 tokens of 32 / 8 heads: 27 us with split keys, 17.7 whole, 13.0
+        // with four groups; 2048 of 16 / 8: 61, 52, 39).
+        template <int G, int CW, int KW, int HH>
+        __global__ __launch_bounds__(CW *KW *kWave) void attn_mfma_kernel(AttnArgs a)
         {
             const int g = G > 0 ? G : a.Hq / a.Hkv;
-            constexpr int kBlockCols = 32 * WAVES;
+            constexpr int kBlockCols = 32 * CW;
+            constexpr int kKeys = 32 * HH;                     // keys of a tile
+            constexpr int kTileBytes = kKeys * kRowBytes;      // the K (or V) rows of a tile
             // K and V tiles, two buffers each.  Tile t's P V product is issued in
-            // step t + 1, beside the softmax of tile t + 1, so V(t) stays resident
-            // one step longer than K(t); V(t + 1) is loaded into V(t - 1)'s buffer
-            // once every wave has passed the barrier that ends step t.  The four
-            // buffers are separate objects and the loop below names them
-            // statically, so the compiler can tell that the LDS reads of a step do
-            // not depend on the loads in flight.
-            __shared__ __attribute__((aligned(16))) unsigned char k_a[kHalfBytes];
-            __shared__ __attribute__((aligned(16))) unsigned char k_b[kHalfBytes];
-            __shared__ __attribute__((aligned(16))) unsigned char v_a[kHalfBytes];
-            __shared__ __attribute__((aligned(16))) unsigned char v_b[kHalfBytes];
+            // the step after tile t's, beside the next tile's softmax, so a V tile
+            // stays resident one step longer than its K tile; V of the next step
+            // is loaded into the buffer of the step before once every wave has
+            // passed the barrier that ends the step.  The four buffers are separate
+            // objects and the loop below names them statically, so the compiler can
+            // tell that the LDS reads of a step do not depend on the loads in flight.
+            __shared__ __attribute__((aligned(16))) unsigned char k_a[KW * kTileBytes];
+            __shared__ __attribute__((aligned(16))) unsigned char k_b[KW * kTileBytes];
+            __shared__ __attribute__((aligned(16))) unsigned char v_a[KW * kTileBytes];
+            __shared__ __attribute__((aligned(16))) unsigned char v_b[KW * kTileBytes];
 
             const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+            const int cw = wave % CW, kw = wave / CW;
             const int lane = threadIdx.x % kWave;
             const int li = lane % 32, lg = lane / 32;
 
-            // block -> (key slice, batch, KV head, query block); the longest query
-            // blocks go first.  Workgroups are dealt to the XCDs in turn; when
-            // several query blocks read the same keys, block ids are renumbered to
-            // give each XCD a contiguous run, so the query blocks of one (batch,
-            // KV head) share that XCD's L2.  (Decode blocks share nothing and keep
-            // the plain order, which spreads each batch row over the XCDs.)
-            int bid = a.qblocks > 1 ? xcd_contiguous(blockIdx.x, gridDim.x) : static_cast<int>(blockIdx.x);
-            const int sp = bid % a.splits;
-            bid /= a.splits;
-            const int qb = a.qblocks - 1 - bid % a.qblocks;
-            bid /= a.qblocks;
-            const int kvh = bid % a.Hkv;
-            const int64_t b = bid / a.Hkv;
+            // block -> (key slice, batch, KV head, query block).  Prefill: the
+            // (batch, KV head) pair runs fastest, so with a multiple of 8 pairs
+            // every query block of a pair lands on one XCD (workgroups are dealt
+            // to the XCDs in turn) and its L2 holds that pair's K/V; the query
+            // blocks of a slice go longest first over all pairs, so that the
+            // blocks that start last are the shortest (3 x 1001 tokens of 40 / 8
+            // heads 54 us, 62 us with the pairs one after the other).  Slices
+            // are outermost: an XCD deals its workgroups to its shader engines in
+            // turn as well, and with the slice in the low bits of the id the full
+            // slices of 1 x 8192 tokens (2 / 1 heads) met on half of them.
+            // Decode: slices of a pair side by side.
+            int sp, qb, pair;
+            if (a.qblocks > 1)
+            {
+                const int pairs = static_cast<int>(gridDim.x) / (a.qblocks * a.splits);
+                pair = static_cast<int>(blockIdx.x) % pairs;
+                const int rest = static_cast<int>(blockIdx.x) / pairs;
+                sp = rest / a.qblocks;
+                qb = a.qblocks - 1 - rest % a.qblocks;
+            }
+            else
+            {
+                sp = static_cast<int>(blockIdx.x) % a.splits;
+                qb = 0;
+                pair = static_cast<int>(blockIdx.x) / a.splits;
+            }
+            const int kvh = pair % a.Hkv;
+            const int64_t b = pair / a.Hkv;
             // positions, columns and key indices fit in 32 bits (checked by the
             // launcher: B * S * Hq < 2^31)
             const int32_t S = static_cast<int32_t>(a.S), start = static_cast<int32_t>(a.start);
@@ -480,14 +482,23 @@ namespace q3k
             const int32_t block_end = static_cast<int32_t>(block_col + kBlockCols < n_cols ? block_col + kBlockCols : n_cols);
             const int32_t s_last = (block_end - 1) / g;
             const int32_t n_keys = start + s_last + 1;
-            // this block's key slice [sp * split_keys, ...) within the causal range
-            const int32_t k_begin = sp * a.split_keys;
-            const int32_t k_end = n_keys < k_begin + a.split_keys ? n_keys : k_begin + a.split_keys;
-            const int tile_begin = k_begin / kKeyTile;
-            const int ntiles = k_end > k_begin ? (k_end + kKeyTile - 1) / kKeyTile : tile_begin;
+            // this block's key slice [sp * split_keys, ...) within the causal range;
+            // slices past the range have nothing to do (the merge counts the same)
+            const int64_t slice_begin = static_cast<int64_t>(sp) * a.split_keys;
+            if (slice_begin >= n_keys)
+                return;
+            const int32_t k_begin = static_cast<int32_t>(slice_begin);
+            const bool split = n_keys > a.split_keys;
+            const int32_t k_end = n_keys - k_begin < a.split_keys ? n_keys : k_begin + a.split_keys;
+            // tiles of the block [tile0, tile_end); this group's: first, first + KW, ...
+            const int tile_end = (k_end + kKeys - 1) / kKeys;
+            const int tile0 = k_begin / kKeys;
+            const int first = tile0 + kw;
+            const int steps = (tile_end - tile0 + KW - 1) / KW;
+            const int mine = first < tile_end ? (tile_end - first + KW - 1) / KW : 0;
 
             // this lane's column
-            const int64_t wave_col = block_col + 32 * wave;
+            const int64_t wave_col = block_col + 32 * cw;
             const int64_t col = wave_col + li;
             const int32_t wave_s0 = static_cast<int32_t>(wave_col / g);  // the wave's first position
             const int32_t s_col = static_cast<int32_t>(col / g);
@@ -497,9 +508,24 @@ namespace q3k
             const bool wave_active = wave_col < n_cols;
             const bool wave_partial = wave_col + 32 > n_cols;
 
+            const uint16_t *kbase = a.k + b * a.ks0 + kvh * a.ks2;
+            const uint16_t *vbase = a.v + b * a.vs0 + kvh * a.vs2;
+            const int32_t kstride = static_cast<int32_t>(a.ks1) * 2, vstride = static_cast<int32_t>(a.vs1) * 2;
+            const auto kslot = [](int r, int c) __attribute__((always_inline)) { return k_slot(r, c); };
+            const auto vslot = [](int r, int c) __attribute__((always_inline)) { return v_slot(r, c); };
+            int32_t k_voff[Staging<CW, kKeys>::kLoads], v_voff[Staging<CW, kKeys>::kLoads];
+            tile_offsets<CW, kKeys>(cw, lane, kstride, kslot, k_voff);
+            tile_offsets<CW, kKeys>(cw, lane, vstride, vslot, v_voff);
+            auto load_k = [&](int tile, unsigned char *buf) __attribute__((always_inline)) {
+                load_tile_rows<CW, kKeys>(tile, buf + kw * kTileBytes, kbase, a.ks1, kstride, n_keys, cw, lane, k_voff,
+                                          kslot);
+            };
+            auto load_v = [&](int tile, unsigned char *buf) __attribute__((always_inline)) {
+                load_tile_rows<CW, kKeys>(tile, buf + kw * kTileBytes, vbase, a.vs1, vstride, n_keys, cw, lane, v_voff,
+                                          vslot);
+            };
             bf16x8_t qf[kAttD / 16];
             load_q(a, b, s_col, h_col, col_ok, lg, qf);
-            Q3K_ATTN_STAGING(WAVES)
             int v_off[kAttD / 32];
             v_offsets(lane, v_off);
             f32x16_t o[kAttD / 32];
@@ -508,133 +534,267 @@ namespace q3k
                 o[dt] = f32x16_t{};
             float m = -__builtin_huge_valf(), l = 0.0f;
             const float scale2 = a.scale * kLog2e;
-            bf16x8_t phi[2][2], plo[2][2]; // P of the tile whose P V is still to be issued
+            bf16x8_t phi[HH][2], plo[HH][2]; // P of the tile whose P V is still to be issued
 
-            // One step: load K(tile + 1); S^T = K(tile) Q^T; the P V of the
+            // One step: load K of the next tile; S^T = K(tile) Q^T; the P V of the
             // previous tile (WITH_PV); this tile's softmax; after the barrier,
-            // load V(tile + 1) into v_prev.
-            auto step = [&](auto with_pv, int tile, const unsigned char *k_cur, unsigned char *k_next,
-                            unsigned char *v_prev) __attribute__((always_inline)) {
-                if (tile + 1 < ntiles)
-                    load_k(tile + 1, k_next); // in flight while this tile is computed
-                if (wave_active)
+            // load V of the next tile into v_prev.  (j is the step; with KW = 1
+            // every group has a tile in every step.)
+            auto step = [&](auto with_pv, int j, unsigned char *k_cur, unsigned char *k_next, unsigned char *v_prev)
+                __attribute__((always_inline)) {
+                const int tile = first + KW * j;
+                if (j + 1 < mine)
+                    load_k(tile + KW, k_next); // in flight while this tile is computed
+                if (wave_active && (KW == 1 || j < mine))
                 {
-                    const int32_t key0 = tile * kKeyTile;
-                    f32x16_t sacc[2];
+                    const int32_t key0 = tile * kKeys;
+                    f32x16_t sacc[HH];
                     // The matrix phase (S = K Q^T, then the previous tile's P V)
                     // runs at raised wave priority, the softmax at the default:
-                    // the other block's wave on the SIMD then interleaves its
-                    // VALU work instead of competing for issue with the MFMAs
-                    // (prefill 4% faster at config 4, decode unchanged).
+                    // the other wave on the SIMD then interleaves its VALU work
+                    // instead of competing for issue with the MFMAs (prefill 4%
+                    // faster at config 4, decode unchanged).
                     __builtin_amdgcn_s_setprio(1);
-                    qk_tile(k_cur, qf, li, lg, sacc);
-                    if (key0 + kKeyTile - 1 > start + wave_s0 || wave_partial)
-                        mask_tile(sacc, key0, lg, last_key, col_ok);
+                    qk_tile<HH>(k_cur + kw * kTileBytes, qf, li, lg, sacc);
+                    if (key0 + kKeys - 1 > start + wave_s0 || wave_partial)
+                        mask_tile<HH>(sacc, key0, lg, last_key, col_ok);
                     if constexpr (decltype(with_pv)::value)
-                        pv_tile(v_prev, v_off, phi, plo, o);
+                        pv_tile<HH>(v_prev + kw * kTileBytes, v_off, phi, plo, o);
                     __builtin_amdgcn_s_setprio(0);
-                    const float alpha = softmax_tile(sacc, scale2, m, l, phi, plo);
+                    const float alpha = softmax_tile<HH>(sacc, scale2, m, l, phi, plo);
                     // o holds the tiles before this one at the previous reference
                     rescale(o, alpha);
                 }
-                // this wave's loads of K(tile + 1) and V(tile) have landed; after the
-                // barrier all have, and every wave is done with K(tile) and V(tile - 1)
+                // this wave's loads of the next K and this V have landed; after the
+                // barrier all have, and every wave is done with this K and the V before
                 __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 __syncthreads();
-                if (tile + 1 < ntiles)
-                    load_v(tile + 1, v_prev);
+                if (j + 1 < mine)
+                    load_v(tile + KW, v_prev);
             };
             using no_pv = std::integral_constant<bool, false>;
             using with_pv = std::integral_constant<bool, true>;
-            if (tile_begin < ntiles)
+            if (mine > 0)
             {
-                load_k(tile_begin, k_a);
-                load_v(tile_begin, v_a);
-                __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                __syncthreads();
-                // V(t) sits in v_a when t - tile_begin is even, else in v_b
-                step(no_pv{}, tile_begin, k_a, k_b, v_b);
-                for (int tile = tile_begin + 1; tile < ntiles; tile += 2)
-                {
-                    step(with_pv{}, tile, k_b, k_a, v_a);
-                    if (tile + 1 < ntiles)
-                        step(with_pv{}, tile + 1, k_a, k_b, v_b);
-                }
-                if (wave_active)
-                {
-                    if ((ntiles - 1 - tile_begin) % 2 == 0)
-                        pv_tile(v_a, v_off, phi, plo, o);
-                    else
-                        pv_tile(v_b, v_off, phi, plo, o);
-                }
+                load_k(first, k_a);
+                load_v(first, v_a);
             }
-            if (col_ok)
-                store_column(a, sp, b, s_col, h_col, lg, o, m, l);
-        }
-
-        // Merges the key slices of one query row per block of four waves
-        // (splits <= kMaxSplits).  Every load is issued before any is used:
-        // lane s of each wave reads slice s's reference max and sum, and wave
-        // w the unnormalised O^T of slices w, w + 4, ...  Weights
-        // 2^(m_s - max m) (the maxima are in the log2 domain), then
-        // sum_s w_s O_s / sum_s w_s l_s; lane t holds dims 2t, 2t + 1, and the
-        // four waves' partial sums meet in LDS.
-        constexpr int kMaxSplits = kAttMaxSplits;
-        constexpr int kCombineWaves = 4;
-        constexpr int kSplitsPerWave = kMaxSplits / kCombineWaves;
-
-        __global__ __launch_bounds__(kCombineWaves * kWave) void attn_combine_kernel(const float *__restrict__ part_o,
-                                                                                      const float *__restrict__ part_ml,
-                                                                                      uint16_t *__restrict__ out,
-                                                                                      int64_t rows, int32_t splits)
-        {
-            __shared__ float2 wave_acc[kCombineWaves][kWave];
-            const int64_t row = blockIdx.x;
-            const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-            const int lane = threadIdx.x % kWave;
-            float2 ml = make_float2(-__builtin_huge_valf(), 0.0f);
-            if (lane < splits)
-                ml = reinterpret_cast<const float2 *>(part_ml)[static_cast<int64_t>(lane) * rows + row];
-            float2 v[kSplitsPerWave];
-#pragma unroll
-            for (int u = 0; u < kSplitsPerWave; ++u)
-            {
-                const int sp = wave + kCombineWaves * u;
-                if (sp < splits)
-                    v[u] = reinterpret_cast<const float2 *>(part_o + (static_cast<int64_t>(sp) * rows + row) * kAttD)[lane];
-            }
-            float mx = ml.x;
-#pragma unroll
-            for (int off = kWave / 2; off > 0; off /= 2)
-                mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
-            const float w = lane < splits ? __builtin_amdgcn_exp2f(ml.x - mx) : 0.0f;
-            float a0 = 0.0f, a1 = 0.0f;
-#pragma unroll
-            for (int u = 0; u < kSplitsPerWave; ++u)
-            {
-                const int sp = wave + kCombineWaves * u;
-                if (sp < splits)
-                {
-                    const float ws = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), sp));
-                    a0 += ws * v[u].x;
-                    a1 += ws * v[u].y;
-                }
-            }
-            wave_acc[wave][lane] = make_float2(a0, a1);
-            const float lsum = group_sum<kWave>(w * ml.y);
+            __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
-            if (wave == 0)
+            // V of step j sits in v_a when j is even, else in v_b
+            step(no_pv{}, 0, k_a, k_b, v_b);
+            for (int j = 1; j < steps; j += 2)
             {
-                float2 t = wave_acc[0][lane];
-#pragma unroll
-                for (int k = 1; k < kCombineWaves; ++k)
+                step(with_pv{}, j, k_b, k_a, v_a);
+                if (j + 1 < steps)
+                    step(with_pv{}, j + 1, k_a, k_b, v_b);
+            }
+            if (wave_active && mine > 0)
+            {
+                if ((mine - 1) % 2 == 0)
+                    pv_tile<HH>(v_a + kw * kTileBytes, v_off, phi, plo, o);
+                else
+                    pv_tile<HH>(v_b + kw * kTileBytes, v_off, phi, plo, o);
+            }
+
+            const int64_t row = (b * a.S + s_col) * a.Hq + h_col;
+            if constexpr (KW == 1)
+            {
+                if (col_ok)
                 {
-                    t.x += wave_acc[k][lane].x;
-                    t.y += wave_acc[k][lane].y;
+                    const float inv = 1.0f / l;
+#pragma unroll
+                    for (int dt = 0; dt < kAttD / 32; ++dt)
+                        store_dims(a, split, sp, row, dt, lg, o[dt], inv);
+                    if (split && lg == 0)
+                        store_ml(a, sp, row, m, l);
+                }
+            }
+            else
+            {
+                // The groups' partial results of a column meet in LDS, in the tile
+                // buffers: dims 32 dt .. + 31 of all waves in buffer dt (4 KiB a
+                // wave, 16 bytes a lane, so lanes hit distinct banks).  Group kw
+                // then merges and stores 4 / KW of the four parts.
+                static_assert(kAttD / 32 == 4 && 4 % KW == 0 && CW * KW * kWave * 64 <= KW * kTileBytes, "merge buffers");
+                constexpr int kParts = 4 / KW;
+                __shared__ float2 ml[KW][kBlockCols];
+                unsigned char *const bufs[4] = {k_a, k_b, v_a, v_b};
+                __syncthreads();   // every wave is done with the V tiles
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt)
+                {
+                    float4 *dst = reinterpret_cast<float4 *>(bufs[dt]) + wave * 4 * kWave;
+#pragma unroll
+                    for (int q4 = 0; q4 < 4; ++q4)
+                        dst[q4 * kWave + lane] = {o[dt][4 * q4], o[dt][4 * q4 + 1], o[dt][4 * q4 + 2], o[dt][4 * q4 + 3]};
+                }
+                if (lg == 0)
+                    ml[kw][32 * cw + li] = make_float2(m, l);
+                __syncthreads();
+                float w[KW];
+                float mx = -__builtin_huge_valf();
+#pragma unroll
+                for (int x = 0; x < KW; ++x)
+                    mx = fmaxf(mx, ml[x][32 * cw + li].x);
+                const float m_use = mx == -__builtin_huge_valf() ? 0.0f : mx;
+                float lsum = 0.0f;
+#pragma unroll
+                for (int x = 0; x < KW; ++x)
+                {
+                    const float2 e = ml[x][32 * cw + li];
+                    w[x] = __builtin_amdgcn_exp2f(e.x - m_use);
+                    lsum += w[x] * e.y;
                 }
                 const float inv = 1.0f / lsum;
-                reinterpret_cast<uint32_t *>(out + row * kAttD)[lane] = pack_rne(t.x * inv, t.y * inv);
+#pragma unroll
+                for (int y = 0; y < kParts; ++y)
+                {
+                    f32x16_t r = f32x16_t{};
+                    const unsigned char *buf = k_a;
+                    const int dt = kw * kParts + y;
+                    if (dt == 1)
+                        buf = k_b;
+                    else if (dt == 2)
+                        buf = v_a;
+                    else if (dt == 3)
+                        buf = v_b;
+#pragma unroll
+                    for (int x = 0; x < KW; ++x)
+                    {
+                        const float4 *src = reinterpret_cast<const float4 *>(buf) + (x * CW + cw) * 4 * kWave;
+#pragma unroll
+                        for (int q4 = 0; q4 < 4; ++q4)
+                        {
+                            const float4 e = src[q4 * kWave + lane];
+                            r[4 * q4] = __builtin_fmaf(w[x], e.x, r[4 * q4]);
+                            r[4 * q4 + 1] = __builtin_fmaf(w[x], e.y, r[4 * q4 + 1]);
+                            r[4 * q4 + 2] = __builtin_fmaf(w[x], e.z, r[4 * q4 + 2]);
+                            r[4 * q4 + 3] = __builtin_fmaf(w[x], e.w, r[4 * q4 + 3]);
+                        }
+                    }
+                    if (col_ok)
+                        store_dims(a, split, sp, row, dt, lg, r, inv);
+                }
+                if (split && col_ok && lg == 0 && kw == 0)
+                    store_ml(a, sp, row, mx, lsum);
             }
+        }
+
+        // Merges the key slices of the query rows, WPR waves to a row, blocks over
+        // (heads, positions, batch rows).  Every load of a round is issued before
+        // any is used: lane s of each wave reads slice s's reference max and sum
+        // (splits <= kMaxSplits), and wave w the unnormalised O^T of slices w,
+        // w + WPR, ...  Weights 2^(m_s - max m) (the maxima are in the log2 domain),
+        // then sum_s w_s O_s / sum_s w_s l_s; lane t holds dims 2t, 2t + 1, and the
+        // waves' partial sums meet in LDS.
+        // RANGES (more than one position): a row takes the slices its own keys
+        // reach (in the others of its query block all its keys are masked), and a
+        // row whose whole query block fits one slice is already done.  The slice
+        // count is one 32-bit division before the loads; decode has none.
+        constexpr int kMaxSplits = kAttMaxSplits;
+        constexpr int kCombineWaves = 4;
+        constexpr int kCombineRound = kMaxSplits / kCombineWaves; // slices whose O^T a wave loads at once
+        // Up to this many rows a row takes a block (decode: its slices are many,
+        // their loads all in flight), above it a wave: 16384 rows of 4 slices took
+        // 13.0 us with a block each and 9.6 us with a wave each.
+        constexpr int64_t kCombineWideRows = 2048;
+
+        struct CombineArgs
+        {
+            const float *part_o;
+            const float *part_ml;
+            uint16_t *out;
+            int64_t rows;
+            int32_t splits;
+            int32_t Hq;
+            int32_t S;
+            int32_t start;
+            int32_t split_keys;
+            int32_t g;
+            int32_t block_cols;
+        };
+
+        template <int WPR, bool RANGES>
+        __global__ __launch_bounds__(kCombineWaves * kWave) void attn_combine_kernel(CombineArgs a)
+        {
+            static_assert(WPR == 1 || WPR == kCombineWaves, "waves per row");
+            __shared__ float2 wave_acc[kCombineWaves][kWave];
+            const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+            const int lane = threadIdx.x % kWave;
+            const int part = WPR == 1 ? 0 : wave;
+            const int32_t h = WPR == 1 ? static_cast<int32_t>(blockIdx.x) * kCombineWaves + wave : static_cast<int32_t>(blockIdx.x);
+            const int32_t s = RANGES ? static_cast<int32_t>(blockIdx.y) : 0;
+            if (WPR == 1 && h >= a.Hq)
+                return; // whole waves, and no barrier below
+            const int64_t row = (static_cast<int64_t>(blockIdx.z) * a.S + s) * a.Hq + h;
+            const int splits = RANGES ? static_cast<int>(static_cast<uint32_t>(a.start + s) / static_cast<uint32_t>(a.split_keys)) + 1
+                                      : a.splits;
+            float2 ml = make_float2(-__builtin_huge_valf(), 0.0f);
+            if (lane < splits)
+                ml = reinterpret_cast<const float2 *>(a.part_ml)[static_cast<int64_t>(lane) * a.rows + row];
+            float a0 = 0.0f, a1 = 0.0f, w = 0.0f;
+            auto round = [&](int s0) __attribute__((always_inline)) {
+                float2 v[kCombineRound];
+#pragma unroll
+                for (int u = 0; u < kCombineRound; ++u)
+                {
+                    const int sp = s0 + part + WPR * u;
+                    if (sp < splits)
+                        v[u] = reinterpret_cast<const float2 *>(a.part_o + (static_cast<int64_t>(sp) * a.rows + row) *
+                                                                               kAttD)[lane];
+                }
+                if (s0 == 0)
+                {
+                    float mx = ml.x;
+#pragma unroll
+                    for (int off = kWave / 2; off > 0; off /= 2)
+                        mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
+                    w = lane < splits ? __builtin_amdgcn_exp2f(ml.x - mx) : 0.0f;
+                }
+#pragma unroll
+                for (int u = 0; u < kCombineRound; ++u)
+                {
+                    const int sp = s0 + part + WPR * u;
+                    if (sp < splits)
+                    {
+                        const float ws = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), sp));
+                        a0 += ws * v[u].x;
+                        a1 += ws * v[u].y;
+                    }
+                }
+            };
+            round(0);
+            if constexpr (WPR == 1)
+                for (int s0 = kCombineRound; s0 < splits; s0 += kCombineRound)
+                    round(s0);
+            const float lsum = group_sum<kWave>(w * ml.y);
+            bool whole = false; // the row's query block wrote the result itself
+            if constexpr (RANGES)
+            {
+                const uint32_t g = static_cast<uint32_t>(a.g), cols = static_cast<uint32_t>(a.block_cols);
+                const uint32_t col = static_cast<uint32_t>(s) * g + static_cast<uint32_t>(h) % g;
+                const uint32_t last = ((col / cols + 1) * cols - 1) / g; // the block's last position, before the end of S
+                const int32_t s_last = last < static_cast<uint32_t>(a.S) ? static_cast<int32_t>(last) : a.S - 1;
+                whole = a.start + s_last < a.split_keys;
+            }
+            if constexpr (WPR > 1)
+            {
+                wave_acc[wave][lane] = make_float2(a0, a1);
+                __syncthreads();
+                if (part != 0)
+                    return;
+#pragma unroll
+                for (int k = 1; k < WPR; ++k)
+                {
+                    a0 += wave_acc[k][lane].x;
+                    a1 += wave_acc[k][lane].y;
+                }
+            }
+            if (whole)
+                return;
+            const float inv = 1.0f / lsum;
+            reinterpret_cast<uint32_t *>(a.out + row * kAttD)[lane] = pack_rne(a0 * inv, a1 * inv);
         }
 
         // Generic path: one wave per query row (b, s, h); lane t holds head
@@ -697,26 +857,60 @@ namespace q3k
             }
         }
 
-        template <int G>
-        int launch_mfma(AttnArgs a, int64_t B, int waves, hipStream_t stream)
+        template <int G, int CW, int KW, int HH>
+        int launch_mfma(AttnArgs a, int64_t B, hipStream_t stream)
         {
-            const int64_t cols = a.S * (a.Hq / a.Hkv), block_cols = 32 * kAttWaves;
-            a.qblocks = static_cast<int32_t>((cols + block_cols - 1) / block_cols);
+            constexpr int kBlockCols = 32 * CW, kThreads = CW * KW * kWave;
+            a.qblocks = static_cast<int32_t>(blocks_for(a.S * (a.Hq / a.Hkv), kBlockCols));
             const int64_t blocks = B * a.Hkv * a.qblocks * a.splits;
-            if (!launch_fits(blocks, kAttBlock) || (a.splits > 1 && !launch_fits(a.rows, kCombineWaves * kWave)))
+            // (split keys: the plan splits only grids of at most 512 blocks, so positions and
+            // batch rows fit the merge's y and z dimensions)
+            if (!launch_fits(blocks, kThreads) ||
+                (a.splits > 1 && (a.S > 65535 || B > 65535 || !launch_fits(a.rows + B * a.S * kCombineWaves, kCombineWaves * kWave))))
                 return set_error(Q3K_ERR_OVERFLOW, "GQA grid is too large");
-            if (waves == 1)
-            {
-                // one query position (at most 32 columns) per block either way, so the grid is the same
-                static_assert(G == 0 || 32 / G >= 1, "one position per wave at least");
-                attn_mfma_kernel<G, 1><<<dim3(static_cast<unsigned>(blocks)), dim3(kWave), 0, stream>>>(a);
-            }
-            else
-                attn_mfma_kernel<G, kAttWaves><<<dim3(static_cast<unsigned>(blocks)), dim3(kAttBlock), 0, stream>>>(a);
+            attn_mfma_kernel<G, CW, KW, HH><<<dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, stream>>>(a);
             if (a.splits > 1)
-                attn_combine_kernel<<<dim3(static_cast<unsigned>(a.rows)), dim3(kCombineWaves * kWave), 0, stream>>>(
-                    a.part_o, a.part_ml, a.out, a.rows, a.splits);
+            {
+                const CombineArgs c{a.part_o, a.part_ml, a.out, a.rows, a.splits, a.Hq, static_cast<int32_t>(a.S),
+                                    static_cast<int32_t>(a.start), a.split_keys, a.Hq / a.Hkv, kBlockCols};
+                const auto S = static_cast<unsigned>(a.S), batch = static_cast<unsigned>(B);
+                const auto heads = static_cast<unsigned>(a.Hq);
+                const dim3 threads(kCombineWaves * kWave);
+                if (S == 1)
+                    attn_combine_kernel<kCombineWaves, false><<<dim3(heads, 1, batch), threads, 0, stream>>>(c);
+                else if (a.rows <= kCombineWideRows)
+                    attn_combine_kernel<kCombineWaves, true><<<dim3(heads, S, batch), threads, 0, stream>>>(c);
+                else
+                    attn_combine_kernel<1, true>
+                        <<<dim3((heads + kCombineWaves - 1) / kCombineWaves, S, batch), threads, 0, stream>>>(c);
+            }
             return check_launch("grouped_query_attention");
+        }
+
+        template <int G>
+        int launch_columns(const AttnArgs &a, int64_t B, const AttnPlan &plan, hipStream_t stream)
+        {
+            if (plan.waves == 1)
+                return launch_mfma<G, 1, 1, 2>(a, B, stream); // one decode position (at most 32 columns) per block
+            return launch_mfma<G, kAttWavesPerBlock, 1, 2>(a, B, stream);
+        }
+
+        int launch_plan(const AttnArgs &a, int64_t B, const AttnPlan &plan, hipStream_t stream)
+        {
+            if (plan.split.key_groups == 2)
+                return launch_mfma<0, 4, 2, 2>(a, B, stream);
+            if (plan.split.key_groups == 4)
+                return launch_mfma<0, 2, 4, 1>(a, B, stream);
+            switch (plan.g_instance)
+            {
+            case 1: return launch_columns<1>(a, B, plan, stream);
+            case 2: return launch_columns<2>(a, B, plan, stream);
+            case 4: return launch_columns<4>(a, B, plan, stream);
+            case 8: return launch_columns<8>(a, B, plan, stream);
+            case 16: return launch_columns<16>(a, B, plan, stream);
+            case 32: return launch_columns<32>(a, B, plan, stream);
+            default: return launch_columns<0>(a, B, plan, stream);
+            }
         }
     } // namespace
 } // namespace q3k
@@ -792,16 +986,7 @@ extern "C" int q3k_gqa_attention_bf16(const uint16_t *q, const uint16_t *k_cache
             a.part_o = static_cast<float *>(workspace);
             a.part_ml = a.part_o + static_cast<int64_t>(plan.split.splits) * a.rows * kAttD;
         }
-        switch (plan.g_instance)
-        {
-        case 1: return launch_mfma<1>(a, B, plan.waves, s);
-        case 2: return launch_mfma<2>(a, B, plan.waves, s);
-        case 4: return launch_mfma<4>(a, B, plan.waves, s);
-        case 8: return launch_mfma<8>(a, B, plan.waves, s);
-        case 16: return launch_mfma<16>(a, B, plan.waves, s);
-        case 32: return launch_mfma<32>(a, B, plan.waves, s);
-        default: return launch_mfma<0>(a, B, plan.waves, s);
-        }
+        return launch_plan(a, B, plan, s);
     }
     const int64_t rows = B * S * Hq;
     const int64_t blocks = blocks_for(rows, kBlock / kWave);

@@ -7,6 +7,8 @@
 
 #include "launch_limits.hpp"
 
+#include <initializer_list>
+
 namespace q3k
 {
     // ---- RoPE and Q/K norm + RoPE over [tokens, heads, 128] rows ------------
@@ -77,15 +79,13 @@ namespace q3k
     constexpr int kAttWavesPerBlock = 4;          // waves of a matrix-core block
     constexpr int kAttColsPerWave = 32;           // (position, head) columns of a wave
     constexpr int kAttMaxSplits = 64;             // key slices the combine kernel merges
-    // Below this many blocks the grid leaves CUs idle and the key range is
-    // split; a slice keeps at least two tiles, or one for a decode step (one
-    // query position), whose slices of up to two tiles run as one-wave blocks:
-    // the four-wave block computes one position in one wave, so each slice
-    // then takes a wave of its own instead of a block (B 1 x 4096 keys: 8.7
-    // against 10.3 us; from B 4 the four-wave blocks, which share each tile's
-    // loads, are as fast or faster).
+    // A decode step (one query position) with fewer blocks than this leaves
+    // CUs idle and its key range is split; a slice keeps at least one tile, and
+    // slices of up to two tiles run as one-wave blocks: the four-wave block
+    // computes one position in one wave, so each slice then takes a wave of its
+    // own instead of a block (B 1 x 4096 keys: 8.7 against 10.3 us; from B 4 the
+    // four-wave blocks, which share each tile's loads, are as fast or faster).
     constexpr int64_t kAttSplitTargetBlocks = 512;
-    constexpr int32_t kAttMinSplitKeys = 2 * kAttKeyTile;
     constexpr int32_t kAttMinDecodeSplitKeys = kAttKeyTile;
     constexpr int32_t kAttMaxOneWaveSplitKeys = 2 * kAttKeyTile;
 
@@ -93,20 +93,154 @@ namespace q3k
     {
         int32_t splits = 1;
         int32_t split_keys = INT32_MAX;
+        int32_t key_groups = 1; // groups of waves of a block that share its columns and divide its keys (1, 2 or 4)
         int64_t bytes = 0; // workspace: unnormalised O^T, max and sum of each slice, fp32
     };
 
+    // Columns of a block and keys of a step for each number of key groups: four
+    // waves side by side and 64-key tiles with one or two groups, two waves and
+    // 32-key tiles with four (LDS: 64 KiB, two blocks a CU, or 128 KiB, one).
+    constexpr int32_t attn_block_cols(int key_groups) { return kAttColsPerWave * (key_groups == 4 ? 2 : 4); }
+
+    // Estimated time in us of a prefill or chunk (S > 1) with `key_groups` and
+    // its keys cut into slices of split_keys, from what the three kernels
+    // measured alone and side by side on a CU (1.8-2.1 GHz): a 64-key tile of a
+    // 128-column block takes 1.6 us alone on its CU and 1.25 us of CU time beside
+    // another block; with two key groups 1.4 us of CU time; with four (64
+    // columns) 0.82 us alone, 0.9 us when blocks queue.  A block costs another
+    // 3.5-5 us of start and end (Q, the first tiles, the store), which with one
+    // key group the other block on the CU hides.  Blocks start longest first, ids
+    // i and i + 256 on one CU, and their key counts fall evenly from the last
+    // query block's to the first's.  A merge costs a launch and a write and a
+    // read of the fp32 slices.
+    //
+    // Over 31 shapes the plan took within 5% of the best of the 9 to 30 forms
+    // timed for 24 of them and within 20% for all (the far ones: one KV head and
+    // long split prefills).  One group / two / four, unsplit, in us: 512 tokens of 32 / 8
+    // heads 17.7 / 17.6 / 13.0; 1000 of 16 / 8 34 / 27 / 18; 2048 of 16 / 8
+    // 52 / 45 / 39; 2048 of 32 / 8 64 / 60 / 75; 2 x 1001 of 32 / 8 41 / 38 / 51;
+    // 2048 of 64 / 8 99 / 117 / 146; 4 x 2048 of 32 / 8 200 / 241 / 304.
+    inline double attn_prefill_us(int64_t pairs, int64_t cols, int32_t G, int64_t S, int64_t cached, int key_groups,
+                                  int64_t split_keys)
+    {
+        constexpr double kCus = 256.0;
+        const int32_t block_cols = attn_block_cols(key_groups);
+        const int64_t qblocks = blocks_for(cols, block_cols);
+        // tiles of the longest and the shortest block (64 keys each)
+        const double last = static_cast<double>(cached);
+        double first = static_cast<double>(cached - S + (block_cols + G - 1) / G);
+        if (first > last)
+            first = last;
+        const bool split = split_keys < cached;
+        double longest = (last + 63.0) / 64.0, shortest = first / 64.0 + 0.5;
+        double blocks = static_cast<double>(pairs * qblocks);
+        const double mean_keys = 0.5 * (first + last);
+        double merge = 0.0;
+        if (split)
+        {
+            // slices of a block, on average: of four blocks spread over the range
+            double slices = 0.0;
+            for (int i = 0; i < 4; ++i)
+            {
+                const int64_t keys = static_cast<int64_t>(first + (last - first) * i / 3.0);
+                slices += 0.25 * static_cast<double>(blocks_for(keys, split_keys));
+            }
+            blocks *= slices;
+            longest = static_cast<double>(split_keys) / 64.0;
+            // the mean slice is the mean range over the slices
+            const double mean = mean_keys / 64.0 / slices;
+            shortest = 2.0 * mean > longest ? 2.0 * mean - longest : 0.0;
+            merge = 3.5 + slices * static_cast<double>(pairs * cols) * (kAttHeadDim * 4) / 2.0e6;
+        }
+        const double total = blocks * 0.5 * (longest + shortest);
+        auto length = [&](double rank) { return longest - (longest - shortest) * rank / blocks; };
+        double us;
+        if (key_groups == 1)
+        {
+            if (blocks <= kCus)
+                us = 4.0 + 1.6 * longest;
+            else if (blocks <= 2 * kCus)
+                us = 5.0 + 1.25 * (longest + length(kCus));
+            else
+                us = 5.0 + 1.25 * total / kCus + 0.3 * longest;
+        }
+        else
+        {
+            const double step = key_groups == 2 ? 1.4 : blocks <= kCus ? 0.82 : 0.9; // us a tile
+            const double block_us = key_groups == 2 ? 5.0 : 3.5;
+            const double rounds = blocks <= kCus ? 1.0 : blocks <= 2 * kCus ? 2.0 : blocks / kCus + 0.5;
+            double work = longest;
+            if (blocks > 2 * kCus)
+                work = total / kCus > longest ? total / kCus : longest;
+            else if (blocks > kCus && 2.0 * length(kCus) > longest)
+                work = 2.0 * length(kCus);
+            us = rounds * block_us + step * work;
+        }
+        return us + merge;
+    }
+
+    // Key groups and, when can_split, the key split of a prefill or chunk.
+    inline AttnSplit plan_attention_prefill(int64_t B, int64_t S, int32_t Hq, int32_t Hkv, int64_t cached,
+                                            bool can_split)
+    {
+        AttnSplit best;
+        const int32_t G = Hq / Hkv;
+        const int64_t cols = S * G, pairs = B * Hkv;
+        double best_us = -1.0;
+        auto consider = [&](int key_groups, int64_t split_keys) {
+            const double us = attn_prefill_us(pairs, cols, G, S, cached, key_groups, split_keys);
+            if (best_us >= 0.0 && us >= best_us)
+                return;
+            best_us = us;
+            best = AttnSplit{};
+            best.key_groups = key_groups;
+            if (split_keys < cached)
+            {
+                best.splits = static_cast<int32_t>(blocks_for(cached, split_keys));
+                best.split_keys = static_cast<int32_t>(split_keys);
+                best.bytes = best.splits * pairs * cols * (kAttHeadDim + 2) * 4;
+            }
+        };
+        // one tile of keys: nothing to divide (16 tokens of 32 / 8 heads: 6.8 us
+        // with one group, 7.5 with four)
+        if (cached <= kAttKeyTile)
+            return best;
+        for (int key_groups : {1, 2, 4})
+            consider(key_groups, cached);
+        best_us -= 0.5; // a split has to give more than the estimates' grain
+        // with a block to each CU and more a split gained nothing (2 x 700 tokens
+        // after 3000, 352 blocks: 134 us whole, 140-147 us in two to four slices)
+        const int64_t blocks = pairs * blocks_for(cols, attn_block_cols(1));
+        if (!can_split || blocks > kAttSplitTargetBlocks / 2)
+            return best;
+        for (const int slices : {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64})
+        {
+            if (slices > kAttMaxSplits || slices > kAttSplitTargetBlocks / blocks + 1)
+                break;
+            const int64_t keys = blocks_for(blocks_for(cached, slices), kAttKeyTile) * kAttKeyTile;
+            if (keys >= 2 * kAttKeyTile && keys < cached)
+                consider(1, keys);
+            const int64_t step_keys = blocks_for(blocks_for(cached, slices), 2 * kAttKeyTile) * 2 * kAttKeyTile;
+            if (step_keys < cached)
+                consider(4, step_keys);
+        }
+        return best;
+    }
+
+    // The key split the workspace is for.
     inline AttnSplit plan_attention_split(int64_t B, int64_t S, int32_t Hq, int32_t Hkv, int64_t cached)
     {
+        if (S > 1)
+        {
+            const AttnSplit p = plan_attention_prefill(B, S, Hq, Hkv, cached, true);
+            return p.splits > 1 ? p : AttnSplit{};
+        }
         AttnSplit p;
-        const int32_t G = Hq / Hkv;
-        const int64_t cols = S * G, block_cols = static_cast<int64_t>(kAttColsPerWave) * kAttWavesPerBlock;
-        const int64_t blocks = B * Hkv * blocks_for(cols, block_cols);
-        const int32_t min_keys = S == 1 ? kAttMinDecodeSplitKeys : kAttMinSplitKeys;
-        if (blocks >= kAttSplitTargetBlocks || cached < 2 * static_cast<int64_t>(min_keys))
+        const int64_t blocks = B * Hkv;
+        if (blocks >= kAttSplitTargetBlocks || cached < 2 * static_cast<int64_t>(kAttMinDecodeSplitKeys))
             return p;
         int64_t want = blocks_for(kAttSplitTargetBlocks, blocks);
-        const int64_t most = cached / min_keys;
+        const int64_t most = cached / kAttMinDecodeSplitKeys;
         if (want > most)
             want = most;
         if (want > kAttMaxSplits)
@@ -118,7 +252,7 @@ namespace q3k
         p.split_keys = static_cast<int32_t>(keys);
         if (p.splits < 2)
             return AttnSplit{};
-        p.bytes = static_cast<int64_t>(p.splits) * B * S * Hq * (kAttHeadDim + 2) * 4;
+        p.bytes = static_cast<int64_t>(p.splits) * B * Hq * (kAttHeadDim + 2) * 4;
         return p;
     }
 
@@ -127,7 +261,7 @@ namespace q3k
         bool mfma = false;   // attn_mfma_kernel; otherwise attn_generic_kernel
         int g_instance = 0;  // the compiled group size (1, 2, 4, 8, 16, 32), or 0: taken at run time
         int waves = kAttWavesPerBlock; // waves per block (1: one-wave decode slices)
-        AttnSplit split;     // splits > 1: the key range is split and attn_combine_kernel merges
+        AttnSplit split;     // key groups; splits > 1: the key range is split and attn_combine_kernel merges
     };
 
     // ks / vs: element strides (batch, position, head, dim) of the K / V
@@ -153,6 +287,8 @@ namespace q3k
         const AttnSplit split = plan_attention_split(B, S, Hq, Hkv, start + S);
         if (split.splits > 1 && split.splits <= kAttMaxSplits && workspace_bytes >= split.bytes && workspace_aligned)
             p.split = split;
+        else if (S > 1)
+            p.split = plan_attention_prefill(B, S, Hq, Hkv, start + S, false);
         if (p.split.splits > 1 && S == 1 && p.split.split_keys <= kAttMaxOneWaveSplitKeys)
             p.waves = 1;
         return p;
