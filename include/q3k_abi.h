@@ -209,9 +209,10 @@ Q3K_API int q3k_gqa_attention_bf16(const uint16_t *q, const uint16_t *k_cache,
                           q3k_stream_t stream);
 
 /*
- * Workspace bytes q3k_gqa_attention_bf16 would use to split this shape's
- * key range (0: it does not split).  No counterpart in the reference (its
- * kernel is one block per query row).
+ * Workspace bytes that let q3k_gqa_attention_bf16 split this shape's key
+ * range (0: it does not split).  A call may leave it unused where one launch
+ * is the faster way (a few hundred keys).  No counterpart in the reference
+ * (its kernel is one block per query row).
  */
 Q3K_API int64_t q3k_gqa_attention_workspace_bytes(int64_t B, int64_t S,
                           int32_t Hq, int32_t Hkv, int32_t D, int64_t cached);

@@ -6,10 +6,10 @@
 // Matrix-core path (head_dim 128, unit dim stride, 16-byte rows): a block of
 // four waves owns one (batch, KV head) and 128 of its (position, head)
 // columns, so every K/V tile it stages in LDS serves 128 query rows.  (A
-// decode step with its key range split into short slices runs the same code
-// as one-wave blocks, one slice each.  A prefill too short to fill the GPU
-// that way takes blocks of eight waves whose two or four groups divide the
-// keys of the same columns and merge in LDS: dispatch.hpp.)  A wave's
+// prefill too short to fill the GPU that way takes blocks of eight waves whose
+// two or four groups divide the keys of the same columns and merge in LDS;
+// attention of at most 32 columns, decode above all, a kernel of its own whose
+// waves share nothing: dispatch.hpp.)  A wave's
 // 32 "columns" are consecutive (position, head) pairs in position-major
 // order: 32 / G whole positions when G divides 32; any G up to 32 works (for
 // Qwen3-14B's 5 a position's heads may straddle two waves).  Per 32 keys:
@@ -136,6 +136,17 @@ namespace q3k
         {
             const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
             return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        }
+
+        // Waits until at most N of the wave's vector loads are in flight and its
+        // LDS reads are done (s_waitcnt vmcnt(N) lgkmcnt(0); 63: the LDS reads only).
+        template <int N>
+        __device__ __forceinline__ void wait_loads()
+        {
+            static_assert(N >= 0 && N < 64, "vmcnt");
+            __asm__ volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | ((N >> 4) << 14));
+            __asm__ volatile("" ::: "memory");
         }
 
         // ---- tile operations shared by the kernels ------------------------------
@@ -407,6 +418,88 @@ namespace q3k
             reinterpret_cast<float2 *>(a.part_ml)[static_cast<int64_t>(sp) * a.rows + row] = make_float2(m, l);
         }
 
+        // The whole column of one wave.
+        __device__ __forceinline__ void store_column(const AttnArgs &a, bool split, int sp, int64_t row, bool col_ok,
+                                                     int lg, const f32x16_t (&o)[kAttD / 32], float m, float l)
+        {
+            if (!col_ok)
+                return;
+            const float inv = 1.0f / l;
+#pragma unroll
+            for (int dt = 0; dt < kAttD / 32; ++dt)
+                store_dims(a, split, sp, row, dt, lg, o[dt], inv);
+            if (split && lg == 0)
+                store_ml(a, sp, row, m, l);
+        }
+
+        // The KW groups' partial results of a column meet in LDS, in the tile
+        // buffers: dims 32 dt .. + 31 of all waves in buffer dt (4 KiB a wave, 16
+        // bytes a lane, so lanes hit distinct banks).  Group kw then merges and
+        // stores 4 / KW of the four parts.
+        template <int CW, int KW>
+        __device__ __forceinline__ void merge_groups(unsigned char *b0, unsigned char *b1, unsigned char *b2,
+                                                     unsigned char *b3, const AttnArgs &a, bool split, int sp, int64_t row,
+                                                     bool col_ok, int cw, int kw, int li, int lg,
+                                                     const f32x16_t (&o)[kAttD / 32], float m, float l)
+        {
+            static_assert(kAttD / 32 == 4 && 4 % KW == 0, "parts");
+            constexpr int kParts = 4 / KW;
+            const int lane = 32 * lg + li, wave = kw * CW + cw;
+            __shared__ float2 ml[KW][32 * CW];
+            unsigned char *const bufs[4] = {b0, b1, b2, b3};
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt)
+            {
+                float4 *dst = reinterpret_cast<float4 *>(bufs[dt]) + wave * 4 * kWave;
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4)
+                    dst[q4 * kWave + lane] = {o[dt][4 * q4], o[dt][4 * q4 + 1], o[dt][4 * q4 + 2], o[dt][4 * q4 + 3]};
+            }
+            if (lg == 0)
+                ml[kw][32 * cw + li] = make_float2(m, l);
+            __syncthreads();
+            float w[KW];
+            float mx = -__builtin_huge_valf();
+#pragma unroll
+            for (int x = 0; x < KW; ++x)
+                mx = fmaxf(mx, ml[x][32 * cw + li].x);
+            const float m_use = mx == -__builtin_huge_valf() ? 0.0f : mx;
+            float lsum = 0.0f;
+#pragma unroll
+            for (int x = 0; x < KW; ++x)
+            {
+                const float2 e = ml[x][32 * cw + li];
+                w[x] = __builtin_amdgcn_exp2f(e.x - m_use);
+                lsum += w[x] * e.y;
+            }
+            const float inv = 1.0f / lsum;
+#pragma unroll
+            for (int y = 0; y < kParts; ++y)
+            {
+                const int dt = kw * kParts + y;
+                const unsigned char *buf = dt == 0 ? b0 : dt == 1 ? b1 : dt == 2 ? b2 : b3;
+                f32x16_t r = f32x16_t{};
+#pragma unroll
+                for (int x = 0; x < KW; ++x)
+                {
+                    const float4 *src = reinterpret_cast<const float4 *>(buf) + (x * CW + cw) * 4 * kWave;
+#pragma unroll
+                    for (int q4 = 0; q4 < 4; ++q4)
+                    {
+                        const float4 e = src[q4 * kWave + lane];
+                        r[4 * q4] = __builtin_fmaf(w[x], e.x, r[4 * q4]);
+                        r[4 * q4 + 1] = __builtin_fmaf(w[x], e.y, r[4 * q4 + 1]);
+                        r[4 * q4 + 2] = __builtin_fmaf(w[x], e.z, r[4 * q4 + 2]);
+                        r[4 * q4 + 3] = __builtin_fmaf(w[x], e.w, r[4 * q4 + 3]);
+                    }
+                }
+                if (col_ok)
+                    store_dims(a, split, sp, row, dt, lg, r, inv);
+            }
+            if (split && col_ok && lg == 0 && kw == 0)
+                store_ml(a, sp, row, mx, lsum);
+        }
+
         // ---- the matrix-core kernel ---------------------------------------------
 
         // G is the group size Hq / Hkv, or 0 for a group size taken from the
@@ -446,7 +539,7 @@ namespace q3k
             const int lane = threadIdx.x % kWave;
             const int li = lane % 32, lg = lane / 32;
 
-            // block -> (key slice, batch, KV head, query block).  Prefill: the
+            // block -> (key slice, batch, KV head, query block).  The
             // (batch, KV head) pair runs fastest, so with a multiple of 8 pairs
             // every query block of a pair lands on one XCD (workgroups are dealt
             // to the XCDs in turn) and its L2 holds that pair's K/V; the query
@@ -456,22 +549,10 @@ namespace q3k
             // are outermost: an XCD deals its workgroups to its shader engines in
             // turn as well, and with the slice in the low bits of the id the full
             // slices of 1 x 8192 tokens (2 / 1 heads) met on half of them.
-            // Decode: slices of a pair side by side.
-            int sp, qb, pair;
-            if (a.qblocks > 1)
-            {
-                const int pairs = static_cast<int>(gridDim.x) / (a.qblocks * a.splits);
-                pair = static_cast<int>(blockIdx.x) % pairs;
-                const int rest = static_cast<int>(blockIdx.x) / pairs;
-                sp = rest / a.qblocks;
-                qb = a.qblocks - 1 - rest % a.qblocks;
-            }
-            else
-            {
-                sp = static_cast<int>(blockIdx.x) % a.splits;
-                qb = 0;
-                pair = static_cast<int>(blockIdx.x) / a.splits;
-            }
+            const int pairs = static_cast<int>(gridDim.x) / (a.qblocks * a.splits);
+            const int pair = static_cast<int>(blockIdx.x) % pairs;
+            const int rest = static_cast<int>(blockIdx.x) / pairs;
+            const int sp = rest / a.qblocks, qb = a.qblocks - 1 - rest % a.qblocks;
             const int kvh = pair % a.Hkv;
             const int64_t b = pair / a.Hkv;
             // positions, columns and key indices fit in 32 bits (checked by the
@@ -553,7 +634,7 @@ namespace q3k
                     // runs at raised wave priority, the softmax at the default:
                     // the other wave on the SIMD then interleaves its VALU work
                     // instead of competing for issue with the MFMAs (prefill 4%
-                    // faster at config 4, decode unchanged).
+                    // faster at config 4).
                     __builtin_amdgcn_s_setprio(1);
                     qk_tile<HH>(k_cur + kw * kTileBytes, qf, li, lg, sacc);
                     if (key0 + kKeys - 1 > start + wave_s0 || wave_partial)
@@ -600,84 +681,136 @@ namespace q3k
             const int64_t row = (b * a.S + s_col) * a.Hq + h_col;
             if constexpr (KW == 1)
             {
-                if (col_ok)
-                {
-                    const float inv = 1.0f / l;
-#pragma unroll
-                    for (int dt = 0; dt < kAttD / 32; ++dt)
-                        store_dims(a, split, sp, row, dt, lg, o[dt], inv);
-                    if (split && lg == 0)
-                        store_ml(a, sp, row, m, l);
-                }
+                store_column(a, split, sp, row, col_ok, lg, o, m, l);
             }
             else
             {
-                // The groups' partial results of a column meet in LDS, in the tile
-                // buffers: dims 32 dt .. + 31 of all waves in buffer dt (4 KiB a
-                // wave, 16 bytes a lane, so lanes hit distinct banks).  Group kw
-                // then merges and stores 4 / KW of the four parts.
-                static_assert(kAttD / 32 == 4 && 4 % KW == 0 && CW * KW * kWave * 64 <= KW * kTileBytes, "merge buffers");
-                constexpr int kParts = 4 / KW;
-                __shared__ float2 ml[KW][kBlockCols];
-                unsigned char *const bufs[4] = {k_a, k_b, v_a, v_b};
-                __syncthreads();   // every wave is done with the V tiles
+                __syncthreads(); // every wave is done with the V tiles
+                merge_groups<CW, KW>(k_a, k_b, v_a, v_b, a, split, sp, row, col_ok, cw, kw, li, lg, o, m, l);
+            }
+        }
+
+        // ---- few columns: decode ---------------------------------------------
+
+        // At most 32 (position, head) columns to a (batch, KV head): one wave holds
+        // them all, so the block's KW waves divide the keys, 32 at a time, and
+        // share nothing until the merge.  Each wave streams its own tiles through
+        // two K and two V buffers with no barrier: a buffer is refilled as soon as
+        // its products are issued, and a wave waits only for the tile it needs, so
+        // about 1.5 tiles of K and V (24 KiB a wave) stay in flight throughout.  What
+        // bounds it is memory for many sequences (64 x 4096 keys of 32 / 8 heads: 184.7
+        // us, 5.8 TB/s; 193.0 with the four-wave prefill kernel, one of whose waves
+        // computed) and the latency of a launch, a tile and the merge for few (1 x 8191
+        // of 16 / 8: 12.2 -> 11.4 us; 40 x 3000 of 16 / 8: 119 -> 88; 19 x 8548 of
+        // 5 / 1: 27 -> 18; 1 x 250: 10.0 -> 6.7).
+        template <int KW>
+        __global__ __launch_bounds__(KW *kWave) void attn_decode_kernel(AttnArgs a)
+        {
+            constexpr int kKeys = 32, kTileBytes = kKeys * kRowBytes, kL = Staging<1, kKeys>::kLoads;
+            __shared__ __attribute__((aligned(16))) unsigned char k_a[KW * kTileBytes];
+            __shared__ __attribute__((aligned(16))) unsigned char k_b[KW * kTileBytes];
+            __shared__ __attribute__((aligned(16))) unsigned char v_a[KW * kTileBytes];
+            __shared__ __attribute__((aligned(16))) unsigned char v_b[KW * kTileBytes];
+            const int kw = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+            const int lane = threadIdx.x % kWave;
+            const int li = lane % 32, lg = lane / 32;
+            // slices of a pair side by side
+            const int sp = static_cast<int>(blockIdx.x) % a.splits, pair = static_cast<int>(blockIdx.x) / a.splits;
+            const int kvh = pair % a.Hkv;
+            const int64_t b = pair / a.Hkv;
+            const int32_t S = static_cast<int32_t>(a.S), start = static_cast<int32_t>(a.start);
+            const int32_t n_keys = start + S;
+            const int32_t k_begin = a.splits > 1 ? sp * a.split_keys : 0;
+            const bool split = a.splits > 1;
+            const int32_t k_end = split && n_keys - k_begin > a.split_keys ? k_begin + a.split_keys : n_keys;
+            const int first = k_begin / kKeys + kw, tile_end = (k_end + kKeys - 1) / kKeys;
+            const int mine = first < tile_end ? (tile_end - first + KW - 1) / KW : 0;
+
+            const uint16_t *kbase = a.k + b * a.ks0 + kvh * a.ks2;
+            const uint16_t *vbase = a.v + b * a.vs0 + kvh * a.vs2;
+            const int32_t kstride = static_cast<int32_t>(a.ks1) * 2, vstride = static_cast<int32_t>(a.vs1) * 2;
+            const auto kslot = [](int r, int c) __attribute__((always_inline)) { return k_slot(r, c); };
+            const auto vslot = [](int r, int c) __attribute__((always_inline)) { return v_slot(r, c); };
+            int32_t k_voff[kL], v_voff[kL];
+            tile_offsets<1, kKeys>(0, lane, kstride, kslot, k_voff);
+            tile_offsets<1, kKeys>(0, lane, vstride, vslot, v_voff);
+            auto load_k = [&](int j, unsigned char *buf) __attribute__((always_inline)) {
+                load_tile_rows<1, kKeys>(first + KW * j, buf + kw * kTileBytes, kbase, a.ks1, kstride, n_keys, 0, lane,
+                                         k_voff, kslot);
+            };
+            auto load_v = [&](int j, unsigned char *buf) __attribute__((always_inline)) {
+                load_tile_rows<1, kKeys>(first + KW * j, buf + kw * kTileBytes, vbase, a.vs1, vstride, n_keys, 0, lane,
+                                         v_voff, vslot);
+            };
+            // the lane's column; lanes past the last one repeat a row of the last position
+            const int g = a.Hq / a.Hkv;
+            const int32_t s_col = li / g;
+            const int h_col = kvh * g + li % g;
+            const bool col_ok = s_col < S;
+            bf16x8_t qf[kAttD / 16];
+            load_q(a, b, s_col, h_col, col_ok, lg, qf);
+            __asm__ volatile("" ::: "memory"); // Q first: waiting for it waits for no tile
+            if (mine > 0)
+            {
+                load_k(0, k_a);
+                load_v(0, v_a);
+            }
+            if (mine > 1)
+            {
+                load_k(1, k_b);
+                load_v(1, v_b);
+            }
+            int v_off[kAttD / 32];
+            v_offsets(lane, v_off);
+            f32x16_t o[kAttD / 32];
 #pragma unroll
-                for (int dt = 0; dt < 4; ++dt)
-                {
-                    float4 *dst = reinterpret_cast<float4 *>(bufs[dt]) + wave * 4 * kWave;
-#pragma unroll
-                    for (int q4 = 0; q4 < 4; ++q4)
-                        dst[q4 * kWave + lane] = {o[dt][4 * q4], o[dt][4 * q4 + 1], o[dt][4 * q4 + 2], o[dt][4 * q4 + 3]};
-                }
-                if (lg == 0)
-                    ml[kw][32 * cw + li] = make_float2(m, l);
-                __syncthreads();
-                float w[KW];
-                float mx = -__builtin_huge_valf();
-#pragma unroll
-                for (int x = 0; x < KW; ++x)
-                    mx = fmaxf(mx, ml[x][32 * cw + li].x);
-                const float m_use = mx == -__builtin_huge_valf() ? 0.0f : mx;
-                float lsum = 0.0f;
-#pragma unroll
-                for (int x = 0; x < KW; ++x)
-                {
-                    const float2 e = ml[x][32 * cw + li];
-                    w[x] = __builtin_amdgcn_exp2f(e.x - m_use);
-                    lsum += w[x] * e.y;
-                }
-                const float inv = 1.0f / lsum;
-#pragma unroll
-                for (int y = 0; y < kParts; ++y)
-                {
-                    f32x16_t r = f32x16_t{};
-                    const unsigned char *buf = k_a;
-                    const int dt = kw * kParts + y;
-                    if (dt == 1)
-                        buf = k_b;
-                    else if (dt == 2)
-                        buf = v_a;
-                    else if (dt == 3)
-                        buf = v_b;
-#pragma unroll
-                    for (int x = 0; x < KW; ++x)
-                    {
-                        const float4 *src = reinterpret_cast<const float4 *>(buf) + (x * CW + cw) * 4 * kWave;
-#pragma unroll
-                        for (int q4 = 0; q4 < 4; ++q4)
-                        {
-                            const float4 e = src[q4 * kWave + lane];
-                            r[4 * q4] = __builtin_fmaf(w[x], e.x, r[4 * q4]);
-                            r[4 * q4 + 1] = __builtin_fmaf(w[x], e.y, r[4 * q4 + 1]);
-                            r[4 * q4 + 2] = __builtin_fmaf(w[x], e.z, r[4 * q4 + 2]);
-                            r[4 * q4 + 3] = __builtin_fmaf(w[x], e.w, r[4 * q4 + 3]);
-                        }
-                    }
-                    if (col_ok)
-                        store_dims(a, split, sp, row, dt, lg, r, inv);
-                }
-                if (split && col_ok && lg == 0 && kw == 0)
-                    store_ml(a, sp, row, mx, lsum);
+            for (int dt = 0; dt < kAttD / 32; ++dt)
+                o[dt] = f32x16_t{};
+            float m = -__builtin_huge_valf(), l = 0.0f;
+            const float scale2 = a.scale * kLog2e;
+
+            auto step = [&](int j, unsigned char *kb, unsigned char *vb) __attribute__((always_inline)) {
+                // loads by age: K(j), V(j), K(j + 1), V(j + 1)
+                if (j + 1 < mine)
+                    wait_loads<3 * kL>();
+                else
+                    wait_loads<kL>();
+                f32x16_t sacc[1];
+                qk_tile<1>(kb + kw * kTileBytes, qf, li, lg, sacc);
+                wait_loads<63>();
+                if (j + 2 < mine)
+                    load_k(j + 2, kb);
+                const int32_t key0 = (first + KW * j) * kKeys;
+                if (key0 + kKeys - 1 > start)
+                    mask_tile<1>(sacc, key0, lg, start + s_col, true);
+                bf16x8_t phi[1][2], plo[1][2];
+                const float alpha = softmax_tile<1>(sacc, scale2, m, l, phi, plo);
+                rescale(o, alpha);
+                // V(j), then K(j + 1), V(j + 1), K(j + 2)
+                if (j + 2 < mine)
+                    wait_loads<3 * kL>();
+                else if (j + 1 < mine)
+                    wait_loads<2 * kL>();
+                else
+                    wait_loads<0>();
+                pv_tile<1>(vb + kw * kTileBytes, v_off, phi, plo, o);
+                wait_loads<63>();
+                if (j + 2 < mine)
+                    load_v(j + 2, vb);
+            };
+            for (int j = 0; j < mine; j += 2)
+            {
+                step(j, k_a, v_a);
+                if (j + 1 < mine)
+                    step(j + 1, k_b, v_b);
+            }
+            const int64_t row = (b * a.S + s_col) * a.Hq + h_col;
+            if constexpr (KW == 1)
+                store_column(a, split, sp, row, col_ok, lg, o, m, l);
+            else
+            {
+                __syncthreads(); // every wave is done with its tiles
+                merge_groups<1, KW>(k_a, k_b, v_a, v_b, a, split, sp, row, col_ok, 0, kw, li, lg, o, m, l);
             }
         }
 
@@ -857,22 +990,12 @@ namespace q3k
             }
         }
 
-        template <int G, int CW, int KW, int HH>
-        int launch_mfma(AttnArgs a, int64_t B, hipStream_t stream)
+        int launch_merge(const AttnArgs &a, int64_t B, int block_cols, hipStream_t stream)
         {
-            constexpr int kBlockCols = 32 * CW, kThreads = CW * KW * kWave;
-            a.qblocks = static_cast<int32_t>(blocks_for(a.S * (a.Hq / a.Hkv), kBlockCols));
-            const int64_t blocks = B * a.Hkv * a.qblocks * a.splits;
-            // (split keys: the plan splits only grids of at most 512 blocks, so positions and
-            // batch rows fit the merge's y and z dimensions)
-            if (!launch_fits(blocks, kThreads) ||
-                (a.splits > 1 && (a.S > 65535 || B > 65535 || !launch_fits(a.rows + B * a.S * kCombineWaves, kCombineWaves * kWave))))
-                return set_error(Q3K_ERR_OVERFLOW, "GQA grid is too large");
-            attn_mfma_kernel<G, CW, KW, HH><<<dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, stream>>>(a);
             if (a.splits > 1)
             {
                 const CombineArgs c{a.part_o, a.part_ml, a.out, a.rows, a.splits, a.Hq, static_cast<int32_t>(a.S),
-                                    static_cast<int32_t>(a.start), a.split_keys, a.Hq / a.Hkv, kBlockCols};
+                                    static_cast<int32_t>(a.start), a.split_keys, a.Hq / a.Hkv, block_cols};
                 const auto S = static_cast<unsigned>(a.S), batch = static_cast<unsigned>(B);
                 const auto heads = static_cast<unsigned>(a.Hq);
                 const dim3 threads(kCombineWaves * kWave);
@@ -887,29 +1010,52 @@ namespace q3k
             return check_launch("grouped_query_attention");
         }
 
-        template <int G>
-        int launch_columns(const AttnArgs &a, int64_t B, const AttnPlan &plan, hipStream_t stream)
+        template <int G, int CW, int KW, int HH>
+        int launch_mfma(AttnArgs a, int64_t B, hipStream_t stream)
         {
-            if (plan.waves == 1)
-                return launch_mfma<G, 1, 1, 2>(a, B, stream); // one decode position (at most 32 columns) per block
-            return launch_mfma<G, kAttWavesPerBlock, 1, 2>(a, B, stream);
+            constexpr int kBlockCols = 32 * CW, kThreads = CW * KW * kWave;
+            a.qblocks = static_cast<int32_t>(blocks_for(a.S * (a.Hq / a.Hkv), kBlockCols));
+            const int64_t blocks = B * a.Hkv * a.qblocks * a.splits;
+            // (split keys: the plan splits only grids of at most 512 blocks, so positions and
+            // batch rows fit the merge's y and z dimensions)
+            if (!launch_fits(blocks, kThreads) ||
+                (a.splits > 1 && (a.S > 65535 || B > 65535 || !launch_fits(a.rows + B * a.S * kCombineWaves, kCombineWaves * kWave))))
+                return set_error(Q3K_ERR_OVERFLOW, "GQA grid is too large");
+            attn_mfma_kernel<G, CW, KW, HH><<<dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, stream>>>(a);
+            return launch_merge(a, B, kBlockCols, stream);
+        }
+
+        template <int KW>
+        int launch_decode(const AttnArgs &a, int64_t B, hipStream_t stream)
+        {
+            const int64_t blocks = B * a.Hkv * a.splits;
+            if (!launch_fits(blocks, KW * kWave))
+                return set_error(Q3K_ERR_OVERFLOW, "GQA grid is too large");
+            attn_decode_kernel<KW><<<dim3(static_cast<unsigned>(blocks)), dim3(KW * kWave), 0, stream>>>(a);
+            return launch_merge(a, B, 32, stream);
         }
 
         int launch_plan(const AttnArgs &a, int64_t B, const AttnPlan &plan, hipStream_t stream)
         {
+            if (plan.split.decode_waves == 1)
+                return launch_decode<1>(a, B, stream);
+            if (plan.split.decode_waves == 2)
+                return launch_decode<2>(a, B, stream);
+            if (plan.split.decode_waves == 4)
+                return launch_decode<4>(a, B, stream);
             if (plan.split.key_groups == 2)
                 return launch_mfma<0, 4, 2, 2>(a, B, stream);
             if (plan.split.key_groups == 4)
                 return launch_mfma<0, 2, 4, 1>(a, B, stream);
             switch (plan.g_instance)
             {
-            case 1: return launch_columns<1>(a, B, plan, stream);
-            case 2: return launch_columns<2>(a, B, plan, stream);
-            case 4: return launch_columns<4>(a, B, plan, stream);
-            case 8: return launch_columns<8>(a, B, plan, stream);
-            case 16: return launch_columns<16>(a, B, plan, stream);
-            case 32: return launch_columns<32>(a, B, plan, stream);
-            default: return launch_columns<0>(a, B, plan, stream);
+            case 1: return launch_mfma<1, kAttWavesPerBlock, 1, 2>(a, B, stream);
+            case 2: return launch_mfma<2, kAttWavesPerBlock, 1, 2>(a, B, stream);
+            case 4: return launch_mfma<4, kAttWavesPerBlock, 1, 2>(a, B, stream);
+            case 8: return launch_mfma<8, kAttWavesPerBlock, 1, 2>(a, B, stream);
+            case 16: return launch_mfma<16, kAttWavesPerBlock, 1, 2>(a, B, stream);
+            case 32: return launch_mfma<32, kAttWavesPerBlock, 1, 2>(a, B, stream);
+            default: return launch_mfma<0, kAttWavesPerBlock, 1, 2>(a, B, stream);
             }
         }
     } // namespace

@@ -79,22 +79,19 @@ namespace q3k
     constexpr int kAttWavesPerBlock = 4;          // waves of a matrix-core block
     constexpr int kAttColsPerWave = 32;           // (position, head) columns of a wave
     constexpr int kAttMaxSplits = 64;             // key slices the combine kernel merges
-    // A decode step (one query position) with fewer blocks than this leaves
-    // CUs idle and its key range is split; a slice keeps at least one tile, and
-    // slices of up to two tiles run as one-wave blocks: the four-wave block
-    // computes one position in one wave, so each slice then takes a wave of its
-    // own instead of a block (B 1 x 4096 keys: 8.7 against 10.3 us; from B 4 the
-    // four-wave blocks, which share each tile's loads, are as fast or faster).
+    // Grids of fewer blocks leave CUs idle: their keys may be split.
     constexpr int64_t kAttSplitTargetBlocks = 512;
-    constexpr int32_t kAttMinDecodeSplitKeys = kAttKeyTile;
+    // Decode slices of up to this many keys run as one-wave blocks.
     constexpr int32_t kAttMaxOneWaveSplitKeys = 2 * kAttKeyTile;
+    constexpr int32_t kAttDecodeTile = 32; // keys of a decode wave's tile
 
     struct AttnSplit
     {
         int32_t splits = 1;
         int32_t split_keys = INT32_MAX;
         int32_t key_groups = 1; // groups of waves of a block that share its columns and divide its keys (1, 2 or 4)
-        int64_t bytes = 0; // workspace: unnormalised O^T, max and sum of each slice, fp32
+        int32_t decode_waves = 0; // waves of a decode block (1, 2 or 4); 0: not the decode kernel
+        int64_t bytes = 0; // workspace of the best split (unnormalised O^T, max and sum of each slice, fp32), taken or not
     };
 
     // Columns of a block and keys of a step for each number of key groups: four
@@ -202,8 +199,9 @@ namespace q3k
             }
         };
         // one tile of keys: nothing to divide (16 tokens of 32 / 8 heads: 6.8 us
-        // with one group, 7.5 with four)
-        if (cached <= kAttKeyTile)
+        // with one group, 7.5 with four); two tiles and few columns: as long as the
+        // groups' merge (13 tokens after 95: 7.9 us against 8.3)
+        if (cached <= kAttKeyTile || (cached <= 2 * kAttKeyTile && cols <= 2 * kAttColsPerWave))
             return best;
         for (int key_groups : {1, 2, 4})
             consider(key_groups, cached);
@@ -227,40 +225,104 @@ namespace q3k
         return best;
     }
 
+    // Estimated time in us of attention over at most 32 columns to a (batch, KV
+    // head) pair (decode), blocks of `waves` waves and slices of split_keys keys.
+    // The measurements behind it: a wave takes 0.95 us a 32-key tile when alone,
+    // c busy CUs read 8.6 c / (c + 90) TB/s together up to 5.9, and one CU 31 GB/s
+    // beside the others, so uneven CUs cost; one, two or four waves a block put
+    // four, two or one block on a CU; start and end take 2.7 us with one wave, 3.3
+    // with two and 4.5 with four (the groups' merge), another round of short blocks
+    // 2 us, the merge launch 3.8 us with its share of the host.
+    inline double attn_decode_us(int64_t pairs, int64_t cached, int waves, int64_t split_keys)
+    {
+        const int64_t keys = split_keys < cached ? split_keys : cached;
+        const int64_t slices = blocks_for(cached, keys);
+        const int64_t blocks = pairs * slices, slots = 256 * (waves == 1 ? 4 : waves == 2 ? 2 : 1);
+        const double chain = 0.95 * static_cast<double>(blocks_for(blocks_for(keys, kAttDecodeTile), waves));
+        const double bytes = static_cast<double>(keys) * (4 * kAttHeadDim);
+        auto round_us = [&](int64_t n) {
+            const double cus = static_cast<double>(n < 256 ? n : 256);
+            const double rate = 8.6e6 * cus / (cus + 90.0);
+            double us = static_cast<double>(n) * bytes / ((rate < 5.9e6 ? rate : 5.9e6) * (waves == 4 ? 1.0 : 0.95));
+            const double cu = n > 256 ? static_cast<double>(blocks_for(n, 256)) * bytes / 31.0e3 : 0.0;
+            us = us > cu ? us : cu;
+            return us > chain ? us : chain;
+        };
+        const int64_t full = blocks / slots, rest = blocks % slots;
+        double us = waves == 4 ? 4.5 : waves == 2 ? 3.3 : 2.7;
+        if (full > 0)
+            us += static_cast<double>(full) * round_us(slots);
+        if (rest > 0)
+            us += round_us(rest);
+        const int64_t more = blocks_for(blocks, slots) - 1;
+        if (more > 0 && round_us(slots) < 20.0)
+            us += 2.0 * static_cast<double>(more);
+        if (slices > 1)
+            us += 3.8 + 0.006 * static_cast<double>(slices);
+        return us;
+    }
+
+    // Waves to a block and, when can_split, the key split of a decode step (or
+    // any attention of at most 32 columns a pair).  One launch beats split and
+    // merge up to about 600 keys a pair (1 sequence of 250 keys: 6.3 us against
+    // 8.6; 16 x 300: 9.0 against 10.6; 1 x 1023: 12.0 against 9.2); 64 x 511 keys
+    // of 32 / 8 heads took 27.2 us with two waves a block and 29.6 with four, 40 x
+    // 3000 of 16 / 8 105 us whole and 88 in three slices of four-wave blocks.
+    inline AttnSplit plan_attention_decode(int64_t B, int64_t S, int32_t Hq, int32_t Hkv, int64_t cached, bool can_split)
+    {
+        const int64_t pairs = B * Hkv;
+        AttnSplit best, best_split;
+        double best_us = -1.0, best_split_us = -1.0;
+        for (const int waves : {4, 2, 1})
+        {
+            if (waves == 1 && cached > kAttDecodeTile)
+                continue;
+            const double us = attn_decode_us(pairs, cached, waves, cached);
+            if (best_us >= 0.0 && us >= best_us)
+                continue;
+            best_us = us;
+            best.decode_waves = waves;
+        }
+        if (pairs >= kAttSplitTargetBlocks || cached < 2 * kAttKeyTile)
+            return best;
+        for (const int slices : {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64})
+        {
+            const int64_t keys = blocks_for(blocks_for(cached, slices), kAttDecodeTile) * kAttDecodeTile;
+            if (keys >= cached || keys < 2 * kAttDecodeTile)
+                continue;
+            for (const int waves : {4, 2, 1})
+            {
+                if ((waves == 1) != (keys <= kAttMaxOneWaveSplitKeys))
+                    continue;
+                const double us = attn_decode_us(pairs, cached, waves, keys);
+                if (best_split_us >= 0.0 && us >= best_split_us)
+                    continue;
+                best_split_us = us;
+                best_split.decode_waves = waves;
+                best_split.split_keys = static_cast<int32_t>(keys);
+                best_split.splits = static_cast<int32_t>(blocks_for(cached, keys));
+                best_split.bytes = static_cast<int64_t>(best_split.splits) * B * S * Hq * (kAttHeadDim + 2) * 4;
+            }
+        }
+        if (can_split && best_split_us >= 0.0 && best_split_us < best_us)
+            return best_split;
+        best.bytes = best_split.bytes;
+        return best;
+    }
+
     // The key split the workspace is for.
     inline AttnSplit plan_attention_split(int64_t B, int64_t S, int32_t Hq, int32_t Hkv, int64_t cached)
     {
-        if (S > 1)
-        {
-            const AttnSplit p = plan_attention_prefill(B, S, Hq, Hkv, cached, true);
-            return p.splits > 1 ? p : AttnSplit{};
-        }
-        AttnSplit p;
-        const int64_t blocks = B * Hkv;
-        if (blocks >= kAttSplitTargetBlocks || cached < 2 * static_cast<int64_t>(kAttMinDecodeSplitKeys))
-            return p;
-        int64_t want = blocks_for(kAttSplitTargetBlocks, blocks);
-        const int64_t most = cached / kAttMinDecodeSplitKeys;
-        if (want > most)
-            want = most;
-        if (want > kAttMaxSplits)
-            want = kAttMaxSplits;
-        if (want < 2)
-            return p;
-        const int64_t keys = blocks_for(blocks_for(cached, want), kAttKeyTile) * kAttKeyTile;
-        p.splits = static_cast<int32_t>(blocks_for(cached, keys));
-        p.split_keys = static_cast<int32_t>(keys);
-        if (p.splits < 2)
-            return AttnSplit{};
-        p.bytes = static_cast<int64_t>(p.splits) * B * Hq * (kAttHeadDim + 2) * 4;
-        return p;
+        if (S * (Hq / Hkv) <= kAttColsPerWave)
+            return plan_attention_decode(B, S, Hq, Hkv, cached, true);
+        return plan_attention_prefill(B, S, Hq, Hkv, cached, true);
     }
 
     struct AttnPlan
     {
         bool mfma = false;   // attn_mfma_kernel; otherwise attn_generic_kernel
         int g_instance = 0;  // the compiled group size (1, 2, 4, 8, 16, 32), or 0: taken at run time
-        int waves = kAttWavesPerBlock; // waves per block (1: one-wave decode slices)
+        int waves = kAttWavesPerBlock; // waves that divide a block's columns or, in decode, its keys
         AttnSplit split;     // key groups; splits > 1: the key range is split and attn_combine_kernel merges
     };
 
@@ -284,13 +346,13 @@ namespace q3k
         if (!p.mfma)
             return p;
         p.g_instance = (G == 1 || G == 2 || G == 4 || G == 8 || G == 16 || G == 32) ? G : 0;
-        const AttnSplit split = plan_attention_split(B, S, Hq, Hkv, start + S);
-        if (split.splits > 1 && split.splits <= kAttMaxSplits && workspace_bytes >= split.bytes && workspace_aligned)
-            p.split = split;
-        else if (S > 1)
-            p.split = plan_attention_prefill(B, S, Hq, Hkv, start + S, false);
-        if (p.split.splits > 1 && S == 1 && p.split.split_keys <= kAttMaxOneWaveSplitKeys)
-            p.waves = 1;
+        p.split = plan_attention_split(B, S, Hq, Hkv, start + S);
+        if (p.split.splits > 1 &&
+            (p.split.splits > kAttMaxSplits || workspace_bytes < p.split.bytes || !workspace_aligned))
+            p.split = S * G <= kAttColsPerWave ? plan_attention_decode(B, S, Hq, Hkv, start + S, false)
+                                               : plan_attention_prefill(B, S, Hq, Hkv, start + S, false);
+        if (p.split.decode_waves > 0)
+            p.waves = p.split.decode_waves;
         return p;
     }
 } // namespace q3k

@@ -61,3 +61,24 @@ def test_gqa_attention_key_groups_split(q3k, hip, oracle, synth, B, S, start, Hq
     prim, lo, hi = oracle.gqa_attention(q, k, v, Hq, start, rows=rows)
     check_band(oracle, name, got.reshape(-1, D)[rows], prim, lo, hi)
     assert np.isfinite(synth.bf16_to_f32(got)).all()
+
+
+# at most 32 columns a pair (decode): one, two and four waves a block; fewer keys than one tile, waves without a
+# tile, partial tiles; several positions; slices of one wave and of several; more sequences than one round holds
+@pytest.mark.parametrize("B,S,start,Hq,Hkv,split", [
+    (1, 1, 0, 16, 8, False), (3, 1, 31, 32, 8, False), (2, 1, 32, 40, 8, False), (1, 1, 127, 32, 1, False),
+    (1, 1, 200, 32, 8, False), (2, 3, 250, 40, 8, False), (1, 8, 90, 32, 8, False), (40, 1, 161, 32, 8, False),
+    (65, 1, 100, 32, 8, False), (1, 1, 2100, 16, 8, False), (1, 1, 700, 16, 8, True), (2, 4, 1500, 32, 8, True),
+    (1, 1, 9000, 5, 1, True), (5, 1, 3001, 8, 8, True), (20, 1, 2500, 4, 2, True)])
+def test_gqa_attention_decode_waves(q3k, hip, oracle, synth, B, S, start, Hq, Hkv, split):
+    name = f"gqa_attention decode waves B={B} S={S} start={start} Hq={Hq} Hkv={Hkv} split={split}"
+    announce(name)
+    cap = start + S + 3
+    q = synth.normal_bf16(186, B, (B, S, Hq * D))
+    k = synth.normal_bf16(187, B, (B, cap, Hkv, D))
+    v = synth.normal_bf16(188, B, (B, cap, Hkv, D))
+    got = run_attention(q3k, hip, q, k, v, B, S, Hq, start, split=split)
+    rows = np.unique(np.concatenate([np.arange(min(B, 3) * S * Hq), np.arange((B - 1) * S * Hq, B * S * Hq)]))
+    prim, lo, hi = oracle.gqa_attention(q, k[:, :start + S], v[:, :start + S], Hq, start, rows=rows)
+    check_band(oracle, name, got.reshape(-1, D)[rows], prim, lo, hi)
+    assert np.isfinite(synth.bf16_to_f32(got)).all()
