@@ -7,9 +7,12 @@
 // reference's float compare treats them as equal) in the high word and
 // ~index in the low word, so "larger value, then smaller index" is a plain
 // unsigned max.  One block of 1024 threads per row (rows strided over the
-// grid): 128-bit loads when the row allows, wave max by lane shuffles, block
-// max through LDS.  When there are too few rows to fill the GPU and the
-// caller gives a workspace, each row is cut into slices of whole 8-column
+// grid): 128-bit loads of the row's aligned middle, a thread's maximum from the
+// plain bits as packed 16-bit integers (a key per thread, not per element; rows
+// without a positive value or with a NaN start over with a key per element), wave
+// and block maxima by DPP and through LDS.  When rows are longer than
+// kWholeRowColumns, too few to fill the GPU, and the caller gives a workspace,
+// each row is cut into slices of whole 8-column
 // vectors: one block per (row, slice) writes the slice's best key, and a
 // second kernel takes the maximum over the slices of each row (the key
 // order is total, so the result is the same).
@@ -35,65 +38,187 @@ namespace q3k
 
         __device__ __forceinline__ uint64_t max_u64(uint64_t a, uint64_t b) { return a > b ? a : b; }
 
-        // This thread's best key over columns [begin, end) of row r; with
-        // VEC, r is 16-byte aligned and begin a multiple of 8.
-        template <bool VEC>
-        __device__ __forceinline__ uint64_t thread_best(const uint16_t *r, int64_t begin, int64_t end)
+        // Maximum over the wave's lanes, in every lane: DPP within 16-lane rows,
+        // permlane swaps across them (VALU only, no LDS round trip).
+        __device__ __forceinline__ uint32_t wave_max(uint32_t v)
+        {
+            auto max2 = [](uint32_t x, uint32_t y) __attribute__((always_inline)) { return x > y ? x : y; };
+            v = max2(v, dpp_u<kDppQuadXor1>(v));
+            v = max2(v, dpp_u<kDppQuadXor2>(v));
+            v = max2(v, dpp_u<kDppHalfMirror>(v));
+            v = max2(v, dpp_u<kDppMirror>(v));
+            const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+            v = max2(r[0], r[1]);
+            const auto q = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+            return max2(q[0], q[1]);
+        }
+        __device__ __forceinline__ uint64_t wave_max(uint64_t key)
+        {
+            const uint32_t hi = wave_max(static_cast<uint32_t>(key >> 32));
+            const uint32_t lo = static_cast<uint32_t>(key >> 32) == hi ? static_cast<uint32_t>(key) : 0u;
+            return (static_cast<uint64_t>(hi) << 32) | wave_max(lo);
+        }
+
+        // The 16-byte aligned middle of columns [begin, end) of row r: vectors
+        // from column `first`, `count` of them; up to seven columns lie on either
+        // side, column side(t) with thread t < 16 (-1: none).
+        struct Middle
+        {
+            int64_t begin, end, first, count;
+            __device__ __forceinline__ Middle(const uint16_t *r, int64_t b, int64_t e) : begin(b), end(e)
+            {
+                const int64_t odd = (reinterpret_cast<uintptr_t>(r + b) / 2) % 8;
+                first = odd == 0 ? b : b + 8 - odd < e ? b + 8 - odd : e;
+                count = (e - first) / 8;
+            }
+            __device__ __forceinline__ int64_t side(int t) const
+            {
+                const int64_t c = t < 8 ? begin + t : first + 8 * count + t - 8;
+                return t < 16 && c < (t < 8 ? first : end) ? c : -1;
+            }
+        };
+
+        // This thread's best key over columns [begin, end) of row r: any values.
+        constexpr int kUnroll = 5;
+        __device__ uint64_t thread_best_any(const uint16_t *r, int64_t begin, int64_t end)
         {
             uint64_t best = 0; // below every candidate
-            int64_t tail = begin;
-            if constexpr (VEC)
+            const Middle mid(r, begin, end);
+            const Vec8 *rv = reinterpret_cast<const Vec8 *>(r + mid.first);
+            for (int64_t i = threadIdx.x; i < mid.count; i += kUnroll * kArgmaxBlock)
             {
-                const int64_t v_end = end / 8;
-                const Vec8 *rv = reinterpret_cast<const Vec8 *>(r);
-                // groups of four 16-byte loads per thread, the last group
-                // partial, all issued before any is used
-                constexpr int U = 4;
-                for (int64_t i = begin / 8 + threadIdx.x; i < v_end; i += U * kArgmaxBlock)
-                {
-                    Vec8 v[U];
+                Vec8 v[kUnroll];
 #pragma unroll
-                    for (int u = 0; u < U; ++u)
-                        if (i + u * kArgmaxBlock < v_end)
-                            v[u] = rv[i + u * kArgmaxBlock];
+                for (int u = 0; u < kUnroll; ++u)
+                    if (i + u * kArgmaxBlock < mid.count)
+                        v[u] = load8<false>(rv + i + u * kArgmaxBlock);
 #pragma unroll
-                    for (int u = 0; u < U; ++u)
-                        if (i + u * kArgmaxBlock < v_end)
-                        {
+                for (int u = 0; u < kUnroll; ++u)
+                    if (i + u * kArgmaxBlock < mid.count)
+                    {
+                        const uint32_t c = static_cast<uint32_t>(mid.first + 8 * (i + u * kArgmaxBlock));
 #pragma unroll
-                            for (int j = 0; j < 4; ++j)
-                            {
-                                const uint32_t idx = static_cast<uint32_t>(8 * (i + u * kArgmaxBlock) + 2 * j);
-                                best = max_u64(best, argmax_key(v[u].d[j] & 0xffffu, idx));
-                                best = max_u64(best, argmax_key(v[u].d[j] >> 16, idx + 1));
-                            }
-                        }
-                }
-                tail = v_end * 8 > begin ? v_end * 8 : begin;
+                        for (int j = 0; j < 8; ++j)
+                            best = max_u64(best, argmax_key(j % 2 == 0 ? v[u].d[j / 2] & 0xffffu : v[u].d[j / 2] >> 16, c + j));
+                    }
             }
-            for (int64_t c = tail + threadIdx.x; c < end; c += kArgmaxBlock)
-                best = max_u64(best, argmax_key(r[c], static_cast<uint32_t>(c)));
+            const int64_t side = mid.side(threadIdx.x);
+            if (side >= 0)
+                best = max_u64(best, argmax_key(r[side], static_cast<uint32_t>(side)));
             return best;
         }
 
-        // Block maximum of the threads' keys, valid in thread 0; wave_best is
-        // free again when the call returns.
-        __device__ __forceinline__ uint64_t block_best(uint64_t best, uint64_t *wave_best)
+        typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
+        __device__ __forceinline__ uint32_t max_i16x2(uint32_t a, uint32_t b)
         {
-            const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+            return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(i16x2, a), __builtin_bit_cast(i16x2, b)));
+        }
+
+        // This thread's best key over columns [begin, end) of row r when the range
+        // holds a positive finite or infinite value and no positive NaN (the bits
+        // are then in order as signed 16-bit integers: everything negative, NaN
+        // included, sorts below).  Returns the plain bits' maximum in *top: a block
+        // whose maximum is outside (0, +inf] starts over with thread_best_any.
+        //
+        // The 16-byte aligned middle of the range goes kUnroll vectors a thread at a
+        // time, all loaded before any is used; of the vectors seen only the one
+        // holding the first maximum is kept.  Two packed-max instructions do a
+        // dword pair; a 64-bit key per element made the kernel VALU-bound (64 x
+        // 151936: 7.5 us of kernel, 12 instructions an element).
+        __device__ __forceinline__ uint64_t thread_best(const uint16_t *r, int64_t begin, int64_t end, int32_t *top)
+        {
+            const Middle mid(r, begin, end);
+            const int64_t nv = mid.count;
+            const Vec8 *rv = reinterpret_cast<const Vec8 *>(r + mid.first);
+            int32_t best = INT32_MIN; // below every 16-bit value
+            int64_t at = 0;
+            Vec8 keep{};
+            for (int64_t i = threadIdx.x; i < nv; i += kUnroll * kArgmaxBlock)
+            {
+                Vec8 v[kUnroll];
 #pragma unroll
-            for (int off = 32; off > 0; off /= 2)
-                best = max_u64(best, __shfl_xor(best, off, kWave));
+                for (int u = 0; u < kUnroll; ++u)
+                    if (i + u * kArgmaxBlock < nv)
+                        v[u] = load8<false>(rv + i + u * kArgmaxBlock);
+#pragma unroll
+                for (int u = 0; u < kUnroll; ++u)
+                    if (i + u * kArgmaxBlock < nv)
+                    {
+                        const uint32_t m = max_i16x2(max_i16x2(v[u].d[0], v[u].d[1]), max_i16x2(v[u].d[2], v[u].d[3]));
+                        const int32_t lo = static_cast<int16_t>(m & 0xffffu), hi = static_cast<int32_t>(m) >> 16;
+                        const int32_t mx = lo > hi ? lo : hi;
+                        if (mx > best)
+                        {
+                            best = mx;
+                            at = i + u * kArgmaxBlock;
+                            keep = v[u];
+                        }
+                    }
+            }
+            uint32_t index = 0;
+            if (best != INT32_MIN)
+            {
+                int e = 7;
+#pragma unroll
+                for (int j = 7; j >= 0; --j)
+                {
+                    const int32_t x = static_cast<int16_t>(j % 2 == 0 ? keep.d[j / 2] & 0xffffu : keep.d[j / 2] >> 16);
+                    e = x == best ? j : e;
+                }
+                index = static_cast<uint32_t>(mid.first + 8 * at + e);
+            }
+            const int64_t side = mid.side(threadIdx.x);
+            if (side >= 0)
+            {
+                const int32_t x = static_cast<int16_t>(r[side]);
+                if (x > best || (x == best && static_cast<uint32_t>(side) < index))
+                {
+                    best = x;
+                    index = static_cast<uint32_t>(side);
+                }
+            }
+            *top = best;
+            return best > 0 ? argmax_key(static_cast<uint32_t>(best), index) : 0;
+        }
+
+        struct ArgmaxShared
+        {
+            uint64_t key[kArgmaxBlock / kWave];
+            int32_t top[kArgmaxBlock / kWave];
+        };
+
+        // The best key of columns [begin, end) of row r, in every thread of wave 0;
+        // the shared memory is free again when the call returns.
+        __device__ __forceinline__ uint64_t block_best(const uint16_t *r, int64_t begin, int64_t end, ArgmaxShared &sh)
+        {
+            constexpr int kWaves = kArgmaxBlock / kWave;
+            const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+            int32_t top;
+            uint64_t best = wave_max(thread_best(r, begin, end, &top));
+            const int32_t wave_top = static_cast<int32_t>(wave_max(static_cast<uint32_t>(top) ^ 0x80000000u) ^ 0x80000000u);
             if (lane == 0)
-                wave_best[wave] = best;
+            {
+                sh.key[wave] = best;
+                sh.top[wave] = wave_top;
+            }
+            __syncthreads();
+            const int32_t t = lane < kWaves ? sh.top[lane] : INT32_MIN;
+            const int32_t block_top = static_cast<int32_t>(wave_max(static_cast<uint32_t>(t) ^ 0x80000000u) ^ 0x80000000u);
+            if (block_top > 0 && block_top <= 0x7f80)
+            {
+                if (wave == 0)
+                    best = wave_max(lane < kWaves ? sh.key[lane] : uint64_t{0});
+                __syncthreads();
+                return best;
+            }
+            // no positive value, or a NaN
+            __syncthreads();
+            best = wave_max(thread_best_any(r, begin, end));
+            if (lane == 0)
+                sh.key[wave] = best;
             __syncthreads();
             if (wave == 0)
-            {
-                best = lane < kArgmaxBlock / kWave ? wave_best[lane] : 0;
-#pragma unroll
-                for (int off = 8; off > 0; off /= 2)
-                    best = max_u64(best, __shfl_xor(best, off, kWave));
-            }
+                best = wave_max(lane < kWaves ? sh.key[lane] : uint64_t{0});
             __syncthreads();
             return best;
         }
@@ -103,15 +228,14 @@ namespace q3k
             return static_cast<int32_t>(0xffffffffu - static_cast<uint32_t>(key));
         }
 
-        template <bool VEC>
         __global__ __launch_bounds__(kArgmaxBlock) void argmax_kernel(const uint16_t *__restrict__ x,
                                                                       int32_t *__restrict__ out, int64_t rows,
                                                                       int64_t stride, int64_t n)
         {
-            __shared__ uint64_t wave_best[kArgmaxBlock / kWave];
+            __shared__ ArgmaxShared sh;
             for (int64_t row = blockIdx.x; row < rows; row += gridDim.x)
             {
-                const uint64_t best = block_best(thread_best<VEC>(x + row * stride, 0, n), wave_best);
+                const uint64_t best = block_best(x + row * stride, 0, n, sh);
                 if (threadIdx.x == 0)
                     out[row] = key_index(best);
             }
@@ -119,17 +243,16 @@ namespace q3k
 
         // One block per (row, slice): part[row * slices + slice] = the best
         // key of columns [slice * slice_len, min(n, (slice + 1) * slice_len)).
-        template <bool VEC>
         __global__ __launch_bounds__(kArgmaxBlock) void argmax_slice_kernel(const uint16_t *__restrict__ x,
                                                                             uint64_t *__restrict__ part,
                                                                             int64_t stride, int64_t n,
                                                                             int32_t slices, int64_t slice_len)
         {
-            __shared__ uint64_t wave_best[kArgmaxBlock / kWave];
-            const int64_t row = blockIdx.x / slices;
-            const int64_t begin = (blockIdx.x % slices) * slice_len;
+            __shared__ ArgmaxShared sh;
+            const int32_t row = static_cast<int32_t>(blockIdx.x) / slices;
+            const int64_t begin = (static_cast<int32_t>(blockIdx.x) % slices) * slice_len;
             const int64_t end = begin + slice_len < n ? begin + slice_len : n;
-            const uint64_t best = block_best(thread_best<VEC>(x + row * stride, begin, end), wave_best);
+            const uint64_t best = block_best(x + row * stride, begin, end, sh);
             if (threadIdx.x == 0)
                 part[blockIdx.x] = best;
         }
@@ -143,10 +266,7 @@ namespace q3k
             if (row >= rows)
                 return;
             const int lane = threadIdx.x % kWave;
-            uint64_t best = lane < slices ? part[row * slices + lane] : 0;
-#pragma unroll
-            for (int off = 32; off > 0; off /= 2)
-                best = max_u64(best, __shfl_xor(best, off, kWave));
+            const uint64_t best = wave_max(lane < slices ? part[row * slices + lane] : uint64_t{0});
             if (lane == 0)
                 out[row] = key_index(best);
         }
@@ -156,6 +276,12 @@ namespace q3k
         constexpr int64_t kTargetBlocks = 512;
         constexpr int64_t kMinSlice = 8 * kArgmaxBlock;
         constexpr int kMaxSlices = kWave;
+
+        // Rows up to this long are searched whole, a block each: one launch.  64 x
+        // 151936 took 6.3 us whole and 7.6 as slices and merge, 1 x 151936 4.7 and
+        // 4.7 (the second launch costs the host another 1.3), 256 x 151669 13.6 and
+        // 15.6.
+        constexpr int64_t kWholeRowColumns = int64_t{1} << 18;
 
         struct SlicePlan
         {
@@ -221,26 +347,17 @@ namespace q3k
         int launch_argmax(const uint16_t *x, int32_t *out, int64_t rows, int64_t row_stride, int64_t search_size,
                           const SlicePlan &plan, uint64_t *part, hipStream_t s)
         {
-            const bool vec = aligned16(x) && row_stride % 8 == 0;
-            if (plan.slices > 1 && part != nullptr)
+            if (plan.slices > 1 && part != nullptr && search_size > kWholeRowColumns)
             {
-                const dim3 grid(static_cast<unsigned>(rows * plan.slices));
-                if (vec)
-                    argmax_slice_kernel<true><<<grid, dim3(kArgmaxBlock), 0, s>>>(x, part, row_stride, search_size,
-                                                                                  plan.slices, plan.slice_len);
-                else
-                    argmax_slice_kernel<false><<<grid, dim3(kArgmaxBlock), 0, s>>>(x, part, row_stride, search_size,
-                                                                                   plan.slices, plan.slice_len);
+                argmax_slice_kernel<<<dim3(static_cast<unsigned>(rows * plan.slices)), dim3(kArgmaxBlock), 0, s>>>(
+                    x, part, row_stride, search_size, plan.slices, plan.slice_len);
                 const int64_t per_block = kBlock / kWave;
                 argmax_merge_kernel<<<dim3(static_cast<unsigned>((rows + per_block - 1) / per_block)), dim3(kBlock), 0,
                                       s>>>(part, out, rows, plan.slices);
                 return check_launch("argmax_last_dimension");
             }
             const unsigned grid = static_cast<unsigned>(rows < 65535 ? rows : 65535);
-            if (vec)
-                argmax_kernel<true><<<dim3(grid), dim3(kArgmaxBlock), 0, s>>>(x, out, rows, row_stride, search_size);
-            else
-                argmax_kernel<false><<<dim3(grid), dim3(kArgmaxBlock), 0, s>>>(x, out, rows, row_stride, search_size);
+            argmax_kernel<<<dim3(grid), dim3(kArgmaxBlock), 0, s>>>(x, out, rows, row_stride, search_size);
             return check_launch("argmax_last_dimension");
         }
 

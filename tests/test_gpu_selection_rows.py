@@ -1,0 +1,83 @@
+"""Argmax and top-k candidates at the edges of their row kernels: rows that start off 16 bytes, lengths around a
+vector, a block's loads, the longest row kept in registers and the shortest cut into slices, rows without a positive
+value, with NaN, with signed zeros and with many ties; k around the bound rules.  Bit-exact against the oracle."""
+import numpy as np
+import pytest
+
+from gpu_util import Guarded, announce, check_exact
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [1, 7, 8, 9, 15, 100, 8191, 8193, 20000, 155649, 163840, 163841, 262144, 262145, 300001]
+
+
+def _rows(synth, n, stride):
+    """Six rows of `stride` columns, the first n of them searched: plain, all negative, zeros of both signs over
+    negatives, one positive maximum at both ends, a few values tied many times, large and tied."""
+    x = synth.normal_bf16(190, n, (6, stride), std=3.0)
+    x[1] |= 0x8000
+    x[2] |= 0x8000
+    x[2, n // 2:: 7] = 0x8000
+    x[2, n // 2 + n // 4:: 11] = 0x0000
+    x[3] |= 0x8000
+    x[3, n - 1] = x[3, 0] = 0x4000
+    levels = synth.f32_to_bf16(np.linspace(-2.0, 2.0, 9).astype(np.float32))
+    x[4] = levels[np.random.default_rng(n).integers(0, 9, stride)]
+    x[5, ::3] = 0x4120
+    return x
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("pad,offset", [(0, 0), (1, 2), (5, 14)])
+def test_argmax_row_edges(q3k, hip, oracle, synth, n, pad, offset):
+    stride = n + pad
+    name = f"argmax edges n={n} stride={stride} offset={offset}"
+    announce(name)
+    x = _rows(synth, n, stride)
+    x = np.concatenate([x, x[:2], np.full((1, stride), 0xff80, np.uint16)])
+    x[6, n // 3] = 0x7fc0                 # a NaN among positives
+    x[7, 0] = 0xffc1                      # a negative NaN first
+    rows = x.shape[0]
+    X, O = Guarded(hip, x, offset=offset), Guarded(hip, nbytes=rows * 4)
+    ws = q3k.argmax_workspace_bytes(rows, n)
+    W = Guarded(hip, nbytes=ws) if ws else None
+    q3k.argmax(X, O, rows, stride, n, workspace=W, workspace_bytes=ws)
+    hip.synchronize()
+    assert O.guards_intact() and (W is None or W.guards_intact())
+    check_exact(name, O.get(np.int32, (rows,)).view(np.uint32), oracle.argmax(x, n).view(np.uint32))
+
+
+@pytest.mark.parametrize("n,ks", [(9, (1, 9)), (100, (1, 20, 100)), (8193, (20, 192, 193)), (20000, (1, 192, 1024, 1500)),
+                                  (155649, (20, 193)), (163840, (1, 64, 192, 193, 1024)), (163841, (20, 1024)),
+                                  (262145, (20, 300))])
+@pytest.mark.parametrize("pad,offset", [(0, 0), (3, 6)])
+def test_topk_row_edges(q3k, hip, oracle, synth, n, ks, pad, offset):
+    stride = n + pad
+    x = _rows(synth, n, stride)
+    x = np.concatenate([x, x[:1]])
+    x[6, n - 1] = 0xff80                  # -inf: a non-finite row
+    rows = x.shape[0]
+    X = Guarded(hip, x, offset=offset)
+    for k in ks:
+        name = f"topk edges n={n} stride={stride} offset={offset} k={k}"
+        announce(name)
+        cap = 2048
+        C, F = Guarded(hip, nbytes=rows * 4), Guarded(hip, nbytes=rows * 4)
+        I, V = Guarded(hip, nbytes=rows * cap * 4), Guarded(hip, nbytes=rows * cap * 2)
+        ws = q3k.topk_workspace_bytes(rows, n, k)
+        W = Guarded(hip, nbytes=ws) if ws else None
+        q3k.topk_candidates(X, rows, stride, n, k, cap, C, I, V, F, workspace=W, workspace_bytes=ws)
+        hip.synchronize()
+        assert all(b.guards_intact() for b in (C, F, I, V) + ((W,) if W is not None else ()))
+        counts, flags = C.get(np.int32, (rows,)), F.get(np.int32, (rows,))
+        ids, vals = I.get(np.int32, (rows, cap)), V.get(np.uint16, (rows, cap))
+        for r in range(rows):
+            want = oracle.topk_set(x[r, :n], k)
+            if want is None:
+                assert flags[r] != 0, f"{name} row {r}: non-finite not flagged"
+                continue
+            assert flags[r] == 0 and counts[r] == want.size, (name, r, counts[r], want.size)
+            if want.size <= cap:
+                got = ids[r, :want.size]
+                check_exact(f"{name} row {r} ids", np.sort(got), np.sort(want))
+                check_exact(f"{name} row {r} logits", vals[r, :want.size], x[r, got])
