@@ -9,7 +9,9 @@
 // or above it (index and bf16 bits, any order), so the host finishes the
 // reference's steps on about k candidates instead of V logits.
 //
-// One block of 1024 threads per row (rows strided over the grid), usually
+// Rows of up to 163840 columns (every Qwen3 vocabulary) with k up to 1024: one
+// block of 1024 threads a row reads it once into its registers (topk_row_kernel,
+// below).  Longer rows, and k above 1024: one block per row (rows strided over the grid),
 // two reads of the row:
 //   1. each thread's largest logit (16-byte loads when the row is aligned)
 //      and the non-finite flag;
@@ -25,7 +27,7 @@
 // each wave counts into its own histogram.  A row with a non-finite logit is
 // flagged (the reference throws for it).
 //
-// With few rows and a caller workspace, each row is cut into slices: one
+// With few of those rows and a caller workspace, each row is cut into slices: one
 // block per (row, slice) finds the slice's bound and lists its logits at or
 // above it (steps 1-2 on the slice), and one block per row keeps the listed
 // logits at or above the largest slice bound and finishes with step 3 (or
@@ -189,6 +191,7 @@ namespace q3k
             uint32_t thread_max[kSelBlock];
             uint32_t list_bits[kCandMax];
             int32_t list_index[kCandMax];
+            int32_t group_max[kSelBlock / 4];
             uint32_t sel[3];
             uint32_t found, bad, listed, bound, overflow;
         };
@@ -341,6 +344,36 @@ namespace q3k
             return t_key == 0u ? -__builtin_huge_valf() : bf_val(key_bits(t_key));
         }
 
+        // Steps 1-3 by reading the row twice (sh.found, sh.bad and sh.listed
+        // zeroed before); ends with a barrier.
+        __device__ void select_reading(const uint16_t *r, int64_t n, uint32_t k, int64_t row, const CandOut &co, SelShared &sh)
+        {
+            // 1. per-thread maxima and the non-finite flag
+            thread_maxima(r, 0, n, sh);
+            bool exact = false;
+            // rows with a non-finite logit keep the whole-row select
+            if (k <= static_cast<uint32_t>(kSelBlock) && sh.bad == 0u)
+            {
+                // 2. lower bound and the list of logits at or above it
+                uint32_t t_key;
+                const float t_val = maxima_bound(sh, k, &t_key);
+                for_row(r, 0, n, [&](int64_t c, uint32_t b) __attribute__((always_inline)) {
+                    list_append(sh, bf_val(b) >= t_val, b, static_cast<int32_t>(c));
+                });
+                __syncthreads();
+                const uint32_t nl = sh.listed;
+                if (nl <= static_cast<uint32_t>(kCandMax))
+                {
+                    // 3. exact k-th over the list (k <= nl: the bound holds)
+                    emit_list(sh, nl, k, row, co);
+                    exact = true;
+                }
+            }
+            if (!exact)
+                whole_row_select(r, n, k, row, co, sh);
+            __syncthreads();
+        }
+
         __global__ __launch_bounds__(kSelBlock) void topk_select_kernel(const uint16_t *__restrict__ x, int64_t rows,
                                                                         int64_t stride, int64_t n, uint32_t k,
                                                                         CandOut co, int32_t *__restrict__ count,
@@ -350,7 +383,6 @@ namespace q3k
             const int tid = threadIdx.x;
             for (int64_t row = blockIdx.x; row < rows; row += gridDim.x)
             {
-                const uint16_t *r = x + row * stride;
                 if (tid == 0)
                 {
                     sh.found = 0u;
@@ -358,30 +390,247 @@ namespace q3k
                     sh.listed = 0u;
                 }
                 __syncthreads();
-                // 1. per-thread maxima and the non-finite flag
-                thread_maxima(r, 0, n, sh);
-                bool exact = false;
-                // rows with a non-finite logit keep the whole-row select
-                if (k <= static_cast<uint32_t>(kSelBlock) && sh.bad == 0u)
+                select_reading(x + row * stride, n, k, row, co, sh);
+                if (tid == 0)
                 {
-                    // 2. lower bound and the list of logits at or above it
-                    uint32_t t_key;
-                    const float t_val = maxima_bound(sh, k, &t_key);
-                    for_row(r, 0, n, [&](int64_t c, uint32_t b) __attribute__((always_inline)) {
-                        list_append(sh, bf_val(b) >= t_val, b, static_cast<int32_t>(c));
-                    });
-                    __syncthreads();
-                    const uint32_t nl = sh.listed;
-                    if (nl <= static_cast<uint32_t>(kCandMax))
+                    count[row] = static_cast<int32_t>(sh.found);
+                    nonfinite[row] = static_cast<int32_t>(sh.bad);
+                }
+                __syncthreads(); // the shared counters are reset for the next row
+            }
+        }
+
+        // ---- rows that fit a block's registers -----------------------------------
+
+        // A row of up to kRegColumns columns is read once, all loads in flight
+        // together, and stays in the registers of its block (20 vectors a thread)
+        // for both steps.  bf16 bits as signed 16-bit integers are in value order
+        // among positive values and sort every negative one below, so with a
+        // positive bound the packed-integer maximum does a dword pair in one
+        // instruction; a row whose bound is not positive is read again by
+        // select_reading.  Non-finite: the signed maximum reaches +inf's bits or the
+        // unsigned maximum -inf's.
+        //
+        // Bound for k <= kGroupK: the k-th largest of the 256 maxima of four threads
+        // each (k groups hold a logit at or above it; about 256 ln(256 / (256 - k))
+        // logits reach it: 21 for k = 20, 226 for k = 150).  Above that the k-th
+        // largest of the thread maxima, as in the other kernels.  The k-th largest
+        // of up to 512 values is found by every wave for itself, bit by bit with
+        // ballots (15 steps, no barrier), for the bound and for the short list.
+        //
+        // 64 rows of 151936: 11.0 us at k = 20 and 15.5 at k = 150, where slices and
+        // merge took 15.5 and 18.8 and one block a row that read twice 17.3 and 19.6;
+        // 256 rows of 151669: 17.6 against 29.7 and 27.8.  Beside the read (6 us at 64
+        // rows) it is the list that takes time, an LDS atomic a logit; listing by
+        // wave segments without atomics (readlane a vector) measured 14.3 and 19.7.
+        constexpr int kRegVecs = 20;
+        constexpr int64_t kRegColumns = int64_t{8} * kRegVecs * kSelBlock;
+        constexpr uint32_t kGroupK = 192;
+        constexpr int kRankSlots = 8; // list entries a lane holds
+        constexpr uint32_t kRankList = kRankSlots * kWave;
+
+        typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
+        typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+        __device__ __forceinline__ uint32_t max_i16x2(uint32_t a, uint32_t b)
+        {
+            return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(i16x2, a), __builtin_bit_cast(i16x2, b)));
+        }
+        __device__ __forceinline__ uint32_t max_u16x2(uint32_t a, uint32_t b)
+        {
+            return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+        }
+        // the larger half as a signed value
+        __device__ __forceinline__ int32_t top_i16(uint32_t m)
+        {
+            const int32_t lo = static_cast<int16_t>(m & 0xffffu), hi = static_cast<int32_t>(m) >> 16;
+            return lo > hi ? lo : hi;
+        }
+        __device__ __forceinline__ int32_t max_i32(int32_t a, int32_t b) { return a > b ? a : b; }
+
+        // The largest T > 0 that at least k of the wave's SLOTS values a lane reach,
+        // i.e. their k-th largest (positive 15-bit values), or 0: there are fewer
+        // than k positive ones.
+        template <int SLOTS>
+        __device__ __forceinline__ int32_t wave_kth(const int32_t (&val)[SLOTS], uint32_t k)
+        {
+            int32_t t = 0;
+#pragma unroll
+            for (int bit = 14; bit >= 0; --bit)
+            {
+                const int32_t cand = t | (1 << bit);
+                uint32_t reach = 0;
+#pragma unroll
+                for (int i = 0; i < SLOTS; ++i)
+                    reach += static_cast<uint32_t>(__popcll(__ballot(val[i] >= cand)));
+                t = reach >= k ? cand : t;
+            }
+            return t;
+        }
+
+        // The list entries at or above its k-th largest (k <= nl <= SLOTS waves'
+        // worth of lanes): each wave finds it and writes its own 64 entries.
+        template <int SLOTS>
+        __device__ __forceinline__ void emit_ranked(SelShared &sh, uint32_t nl, uint32_t k, int64_t row, const CandOut &co)
+        {
+            const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+            if (wave * kWave >= nl)
+                return;
+            int32_t val[SLOTS];
+#pragma unroll
+            for (int i = 0; i < SLOTS; ++i)
+                val[i] = i * kWave + lane < nl ? static_cast<int32_t>(sh.list_bits[i * kWave + lane]) : 0;
+            const int32_t kth = wave_kth<SLOTS>(val, k);
+            const bool in = threadIdx.x < nl;
+            const int32_t mine = in ? static_cast<int32_t>(sh.list_bits[threadIdx.x]) : 0;
+            const bool take = in && mine >= kth;
+            const uint64_t ballot = __ballot(take);
+            uint32_t base = 0;
+            if (lane == 0)
+                base = atomicAdd(&sh.found, static_cast<uint32_t>(__popcll(ballot)));
+            base = __builtin_amdgcn_readfirstlane(base);
+            const uint32_t slot = base + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(ballot >> 32),
+                                                                   __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(ballot), 0u));
+            if (take && slot < static_cast<uint32_t>(co.cap))
+            {
+                co.cand_index[row * co.cap + slot] = sh.list_index[threadIdx.x];
+                co.cand_logit[row * co.cap + slot] = static_cast<uint16_t>(mine);
+            }
+        }
+
+        __global__ __launch_bounds__(kSelBlock) void topk_row_kernel(const uint16_t *__restrict__ x, int64_t rows,
+                                                                     int64_t stride, int32_t n, uint32_t k, CandOut co,
+                                                                     int32_t *__restrict__ count,
+                                                                     int32_t *__restrict__ nonfinite)
+        {
+            __shared__ SelShared sh;
+            const int tid = threadIdx.x, lane = tid % kWave;
+            for (int64_t row = blockIdx.x; row < rows; row += gridDim.x)
+            {
+                const uint16_t *r = x + row * stride;
+                // the 16-byte aligned middle [first, first + 8 nv), up to seven columns on either side
+                const int32_t odd = static_cast<int32_t>((reinterpret_cast<uintptr_t>(r) / 2) % 8);
+                const int32_t first = odd == 0 ? 0 : 8 - odd < n ? 8 - odd : n;
+                const int32_t nv = (n - first) / 8;
+                const Vec8 *rv = reinterpret_cast<const Vec8 *>(r + first);
+                constexpr uint32_t kNone = 0x80008000u; // below every value, finite
+                Vec8 v[kRegVecs];
+#pragma unroll
+                for (int u = 0; u < kRegVecs; ++u)
+                {
+                    v[u] = Vec8{{kNone, kNone, kNone, kNone}};
+                    if (tid + u * kSelBlock < nv)
+                        v[u] = load8<false>(rv + tid + u * kSelBlock);
+                }
+                const int32_t side = tid < 8 ? tid : first + 8 * nv + tid - 8;
+                uint32_t side_bits = kNone & 0xffffu;
+                if (tid < 16 && (tid < 8 ? side < first : side < n))
+                    side_bits = r[side];
+                if (tid == 0)
+                {
+                    sh.found = 0u;
+                    sh.bad = 0u;
+                    sh.listed = 0u;
+                }
+                __syncthreads();
+                // 1. maxima and the non-finite flag
+                uint32_t mi = side_bits | (kNone & 0xffff0000u), mu = mi;
+#pragma unroll
+                for (int u = 0; u < kRegVecs; ++u)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
                     {
-                        // 3. exact k-th over the list (k <= nl: the bound holds)
-                        emit_list(sh, nl, k, row, co);
-                        exact = true;
+                        mi = max_i16x2(mi, v[u].d[j]);
+                        mu = max_u16x2(mu, v[u].d[j]);
+                    }
+                const int32_t tmax = top_i16(mi);
+                if (tmax >= 0x7f80 || (mu >> 16) >= 0xff80u || (mu & 0xffffu) >= 0xff80u)
+                    atomicOr(&sh.bad, 1u);
+                if (k <= kGroupK)
+                {
+                    int32_t g = tmax;
+                    g = max_i32(g, static_cast<int32_t>(dpp_u<kDppQuadXor1>(static_cast<uint32_t>(g))));
+                    g = max_i32(g, static_cast<int32_t>(dpp_u<kDppQuadXor2>(static_cast<uint32_t>(g))));
+                    if (lane % 4 == 0)
+                        sh.group_max[tid / 4] = g;
+                }
+                else
+                    sh.thread_max[tid] = tmax > 0 ? static_cast<uint32_t>(tmax) : 0u;
+                __syncthreads();
+                // 2. the bound, and the list of logits at or above it
+                bool exact = false;
+                const bool bad = sh.bad != 0u;
+                if (!bad)
+                {
+                    int32_t bound;
+                    if (k <= kGroupK)
+                    {
+                        int32_t g[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            g[i] = sh.group_max[i * kWave + lane];
+                        bound = wave_kth<4>(g, k);
+                    }
+                    else
+                        bound = static_cast<int32_t>(
+                            block_kth([&](int i) { return sh.thread_max[i]; }, kSelBlock, k, sh.hist, sh.sel));
+                    if (bound > 0)
+                    {
+                        auto append = [&](uint32_t bits, int32_t index) __attribute__((always_inline)) {
+                            const uint32_t pos = atomicAdd(&sh.listed, 1u);
+                            if (pos < static_cast<uint32_t>(kCandMax))
+                            {
+                                sh.list_bits[pos] = bits;
+                                sh.list_index[pos] = index;
+                            }
+                        };
+                        if (tmax >= bound)
+                        {
+                            if (static_cast<int16_t>(side_bits) >= bound)
+                                append(side_bits, side);
+#pragma unroll
+                            for (int u = 0; u < kRegVecs; ++u)
+                            {
+                                if (top_i16(max_i16x2(max_i16x2(v[u].d[0], v[u].d[1]), max_i16x2(v[u].d[2], v[u].d[3]))) < bound)
+                                    continue;
+                                const int32_t c = first + 8 * (tid + u * kSelBlock);
+#pragma unroll
+                                for (int e = 0; e < 8; ++e)
+                                {
+                                    const uint32_t b = e % 2 == 0 ? v[u].d[e / 2] & 0xffffu : v[u].d[e / 2] >> 16;
+                                    if (static_cast<int16_t>(b) >= bound)
+                                        append(b, c + e);
+                                }
+                            }
+                        }
+                        __syncthreads();
+                        const uint32_t nl = sh.listed;
+                        if (nl <= static_cast<uint32_t>(kCandMax))
+                        {
+                            // 3. the exact top k of the list (k <= nl: the bound holds)
+                            if (nl <= 2 * kWave)
+                                emit_ranked<2>(sh, nl, k, row, co);
+                            else if (nl <= kRankList)
+                                emit_ranked<kRankSlots>(sh, nl, k, row, co);
+                            else
+                                emit_list(sh, nl, k, row, co);
+                            exact = true;
+                        }
                     }
                 }
-                if (!exact)
-                    whole_row_select(r, n, k, row, co, sh);
                 __syncthreads();
+                if (!exact)
+                {
+                    if (bad || sh.listed > static_cast<uint32_t>(kCandMax))
+                        whole_row_select(r, n, k, row, co, sh);
+                    else
+                    {
+                        if (tid == 0)
+                            sh.listed = 0u;
+                        __syncthreads();
+                        select_reading(r, n, k, row, co, sh);
+                    }
+                    __syncthreads();
+                }
                 if (tid == 0)
                 {
                     count[row] = static_cast<int32_t>(sh.found);
@@ -581,6 +830,13 @@ extern "C" int q3k_topk_candidates_bf16(const uint16_t *logits, int64_t rows, in
         return set_error(Q3K_ERR_OVERFLOW, "top-k sizes overflow");
     const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const CandOut co{cap, cand_index, cand_logit};
+    const unsigned grid = static_cast<unsigned>(rows < 65535 ? rows : 65535);
+    if (search_size <= kRegColumns && k <= kSelBlock)
+    {
+        topk_row_kernel<<<dim3(grid), dim3(kSelBlock), 0, s>>>(logits, rows, row_stride, static_cast<int32_t>(search_size),
+                                                                static_cast<uint32_t>(k), co, count, nonfinite);
+        return check_launch("topk_candidates");
+    }
     const SlicePlan plan = plan_slices(rows, search_size, k);
     if (plan.slices > 1 && workspace != nullptr && workspace_bytes >= plan.bytes && aligned_to(workspace, 16))
     {
@@ -597,7 +853,6 @@ extern "C" int q3k_topk_candidates_bf16(const uint16_t *logits, int64_t rows, in
             logits, row_stride, search_size, static_cast<uint32_t>(k), w, co, count, nonfinite);
         return check_launch("topk_candidates");
     }
-    const unsigned grid = static_cast<unsigned>(rows < 65535 ? rows : 65535);
     topk_select_kernel<<<dim3(grid), dim3(kSelBlock), 0, s>>>(logits, rows, row_stride, search_size,
                                                                static_cast<uint32_t>(k), co, count, nonfinite);
     return check_launch("topk_candidates");
