@@ -10,11 +10,16 @@ IndexError, ``std::overflow_error`` -> OverflowError, HIP failures ->
 RuntimeError).
 
 There is no fallback: if the library is not built, :func:`load` raises.
+The wrappers that launch go through ``lib/q3k_calls.so``, which converts the
+usual arguments (ints, floats, buffer objects, tuples of strides) without
+ctypes' cost; anything else it hands back to ctypes.
 Device memory comes from :mod:`.hip` (the HIP runtime the library links).
 """
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import re
 
@@ -22,6 +27,7 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 REPO_DIR = os.path.dirname(PKG_DIR)
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libq3k.so")
+CALLS_PATH = os.path.join(LIB_DIR, "q3k_calls.so")
 RUNTIME_LIB_PATH = os.path.join(LIB_DIR, "libqwen3_runtime.so")
 BENCH_LIB_PATH = os.path.join(LIB_DIR, "libq3k_bench.so")
 ABI_HEADERS = [os.path.join(REPO_DIR, "include", "q3k_abi.h")]
@@ -97,6 +103,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_calls = None  # the module of lib/q3k_calls.so
 
 
 # name -> argtypes, in the order of include/q3k_bench.h (lib/libq3k_bench.so)
@@ -120,7 +127,7 @@ def declared_symbols(headers=None) -> list[str]:
 
 def load(path: str | None = None) -> ctypes.CDLL:
     """Load libq3k.so (RTLD_GLOBAL, so that :mod:`.hip` binds the same HIP runtime)."""
-    global _lib
+    global _lib, _calls
     if _lib is not None and path is None:
         return _lib
     lib_path = path or LIB_PATH
@@ -137,7 +144,13 @@ def load(path: str | None = None) -> ctypes.CDLL:
     lib.q3k_version.restype = ctypes.c_char_p
     lib.q3k_version.argtypes = []
     if path is None:
-        _lib = lib
+        if not os.path.exists(CALLS_PATH):
+            raise RuntimeError(f"{CALLS_PATH} is not built; run __graft_entry__.build()")
+        loader = importlib.machinery.ExtensionFileLoader("q3k_calls", CALLS_PATH)
+        spec = importlib.util.spec_from_file_location("q3k_calls", CALLS_PATH, loader=loader)
+        calls = importlib.util.module_from_spec(spec)
+        loader.exec_module(calls)
+        _lib, _calls = lib, calls
     return lib
 
 
@@ -166,9 +179,17 @@ def _check_bench(status: int) -> None:
 
 
 def _check(status: int) -> None:
-    if status != Q3K_OK:
+    if status:
         msg = load().q3k_last_error_string().decode()
         raise _ERRORS.get(status, Q3kError)(status, msg)
+
+
+def _fast():
+    """The launch entry points without ctypes (lib/q3k_calls.so): a status, or None for arguments they do not
+    convert."""
+    if _calls is None:
+        load()
+    return _calls
 
 
 def _ptr(x):
@@ -183,61 +204,99 @@ def version() -> str:
 
 
 def embedding(ids, T, table, V, H, out, stream=None):
-    _check(load().q3k_embedding_bf16(_ptr(ids), T, _ptr(table), V, H, _ptr(out), _ptr(stream)))
+    st = _fast().q3k_embedding_bf16(ids, T, table, V, H, out, stream)
+    if st is None:
+        st = load().q3k_embedding_bf16(_ptr(ids), T, _ptr(table), V, H, _ptr(out), _ptr(stream))
+    _check(st)
 
 
 def rms_norm(x, w, y, rows, N, eps, stream=None):
-    _check(load().q3k_rms_norm_bf16(_ptr(x), _ptr(w), _ptr(y), rows, N, eps, _ptr(stream)))
+    st = _fast().q3k_rms_norm_bf16(x, w, y, rows, N, eps, stream)
+    if st is None:
+        st = load().q3k_rms_norm_bf16(_ptr(x), _ptr(w), _ptr(y), rows, N, eps, _ptr(stream))
+    _check(st)
 
 
 def add_rms_norm(h, d, w, y, rows, N, eps, stream=None):
-    _check(load().q3k_add_rms_norm_bf16(_ptr(h), _ptr(d), _ptr(w), _ptr(y), rows, N, eps, _ptr(stream)))
+    st = _fast().q3k_add_rms_norm_bf16(h, d, w, y, rows, N, eps, stream)
+    if st is None:
+        st = load().q3k_add_rms_norm_bf16(_ptr(h), _ptr(d), _ptr(w), _ptr(y), rows, N, eps, _ptr(stream))
+    _check(st)
 
 
 def rms_norm_rows(x, w, y, count, first_row, row_stride, N, eps, stream=None):
-    _check(load().q3k_rms_norm_rows_bf16(_ptr(x), _ptr(w), _ptr(y), count, first_row, row_stride, N, eps, _ptr(stream)))
+    st = _fast().q3k_rms_norm_rows_bf16(x, w, y, count, first_row, row_stride, N, eps, stream)
+    if st is None:
+        st = load().q3k_rms_norm_rows_bf16(_ptr(x), _ptr(w), _ptr(y), count, first_row, row_stride, N, eps,
+                                           _ptr(stream))
+    _check(st)
 
 
 def add_rms_norm_rows(h, d, w, y, count, first_row, row_stride, N, eps, stream=None):
-    _check(load().q3k_add_rms_norm_rows_bf16(_ptr(h), _ptr(d), _ptr(w), _ptr(y), count, first_row, row_stride, N, eps,
-                                             _ptr(stream)))
+    st = _fast().q3k_add_rms_norm_rows_bf16(h, d, w, y, count, first_row, row_stride, N, eps, stream)
+    if st is None:
+        st = load().q3k_add_rms_norm_rows_bf16(_ptr(h), _ptr(d), _ptr(w), _ptr(y), count, first_row, row_stride, N,
+                                               eps, _ptr(stream))
+    _check(st)
 
 
 def embedding_rms_norm(ids, T, table, V, H, w, eps, hidden, y, stream=None):
-    _check(load().q3k_embedding_rms_norm_bf16(_ptr(ids), T, _ptr(table), V, H, _ptr(w), eps, _ptr(hidden), _ptr(y),
-                                              _ptr(stream)))
+    st = _fast().q3k_embedding_rms_norm_bf16(ids, T, table, V, H, w, eps, hidden, y, stream)
+    if st is None:
+        st = load().q3k_embedding_rms_norm_bf16(_ptr(ids), T, _ptr(table), V, H, _ptr(w), eps, _ptr(hidden), _ptr(y),
+                                                _ptr(stream))
+    _check(st)
 
 
 def add_inplace(d, s, n, stream=None):
-    _check(load().q3k_add_inplace_bf16(_ptr(d), _ptr(s), n, _ptr(stream)))
+    st = _fast().q3k_add_inplace_bf16(d, s, n, stream)
+    if st is None:
+        st = load().q3k_add_inplace_bf16(_ptr(d), _ptr(s), n, _ptr(stream))
+    _check(st)
 
 
 def silu_mul(g, u, out, n, stream=None):
-    _check(load().q3k_silu_mul_bf16(_ptr(g), _ptr(u), _ptr(out), n, _ptr(stream)))
+    st = _fast().q3k_silu_mul_bf16(g, u, out, n, stream)
+    if st is None:
+        st = load().q3k_silu_mul_bf16(_ptr(g), _ptr(u), _ptr(out), n, _ptr(stream))
+    _check(st)
 
 
 def rope(x, B, S, heads, D, cache, P, start, positions=None, stream=None):
-    _check(load().q3k_rope_bf16(_ptr(x), B, S, heads, D, _ptr(cache), P, start, _ptr(positions), _ptr(stream)))
+    st = _fast().q3k_rope_bf16(x, B, S, heads, D, cache, P, start, positions, stream)
+    if st is None:
+        st = load().q3k_rope_bf16(_ptr(x), B, S, heads, D, _ptr(cache), P, start, _ptr(positions), _ptr(stream))
+    _check(st)
 
 
 def rope_qk(q, k, B, S, Hq, Hkv, D, cache, P, start, positions=None, stream=None):
-    _check(load().q3k_rope_qk_bf16(_ptr(q), _ptr(k), B, S, Hq, Hkv, D, _ptr(cache), P, start, _ptr(positions),
-                                   _ptr(stream)))
+    st = _fast().q3k_rope_qk_bf16(q, k, B, S, Hq, Hkv, D, cache, P, start, positions, stream)
+    if st is None:
+        st = load().q3k_rope_qk_bf16(_ptr(q), _ptr(k), B, S, Hq, Hkv, D, _ptr(cache), P, start, _ptr(positions),
+                                     _ptr(stream))
+    _check(st)
 
 
 def qk_norm_rope(q, k, qw, kw, B, S, Hq, Hkv, D, eps, cache, P, start, positions=None, stream=None):
-    _check(load().q3k_qk_norm_rope_bf16(_ptr(q), _ptr(k), _ptr(qw), _ptr(kw), B, S, Hq, Hkv, D, eps,
-                                        _ptr(cache), P, start, _ptr(positions), _ptr(stream)))
+    st = _fast().q3k_qk_norm_rope_bf16(q, k, qw, kw, B, S, Hq, Hkv, D, eps, cache, P, start, positions, stream)
+    if st is None:
+        st = load().q3k_qk_norm_rope_bf16(_ptr(q), _ptr(k), _ptr(qw), _ptr(kw), B, S, Hq, Hkv, D, eps, _ptr(cache), P,
+                                          start, _ptr(positions), _ptr(stream))
+    _check(st)
 
 
 def gqa_attention(q, k_cache, v_cache, out, B, S, Hq, Hkv, D, cached, start, k_strides, v_strides, stream=None,
                   workspace=None, workspace_bytes=0):
     """k_strides / v_strides: 4 element strides (batch, position, head, dim) of the cache views."""
-    ks = (ctypes.c_int64 * 4)(*[int(x) for x in k_strides])
-    vs = (ctypes.c_int64 * 4)(*[int(x) for x in v_strides])
-    _check(load().q3k_gqa_attention_bf16(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), B, S, Hq, Hkv, D, cached,
-                                         start, ctypes.cast(ks, _p), ctypes.cast(vs, _p), _ptr(workspace),
-                                         workspace_bytes, _ptr(stream)))
+    st = _fast().q3k_gqa_attention_bf16(q, k_cache, v_cache, out, B, S, Hq, Hkv, D, cached, start, k_strides,
+                                        v_strides, workspace, workspace_bytes, stream)
+    if st is None:
+        ks = (ctypes.c_int64 * 4)(*[int(x) for x in k_strides])
+        vs = (ctypes.c_int64 * 4)(*[int(x) for x in v_strides])
+        st = load().q3k_gqa_attention_bf16(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), B, S, Hq, Hkv, D, cached,
+                                           start, ctypes.cast(ks, _p), ctypes.cast(vs, _p), _ptr(workspace),
+                                           workspace_bytes, _ptr(stream))
+    _check(st)
 
 
 def gqa_attention_workspace_bytes(B, S, Hq, Hkv, D, cached):
@@ -245,12 +304,18 @@ def gqa_attention_workspace_bytes(B, S, Hq, Hkv, D, cached):
 
 
 def argmax(x, out, rows, row_stride, search_size, stream=None, workspace=None, workspace_bytes=0):
-    _check(load().q3k_argmax_bf16(_ptr(x), _ptr(out), rows, row_stride, search_size, _ptr(workspace),
-                                  workspace_bytes, _ptr(stream)))
+    st = _fast().q3k_argmax_bf16(x, out, rows, row_stride, search_size, workspace, workspace_bytes, stream)
+    if st is None:
+        st = load().q3k_argmax_bf16(_ptr(x), _ptr(out), rows, row_stride, search_size, _ptr(workspace),
+                                    workspace_bytes, _ptr(stream))
+    _check(st)
 
 
 def argmax_noalloc(x, out, rows, row_stride, search_size, stream=None):
-    _check(load().q3k_argmax_bf16_noalloc(_ptr(x), _ptr(out), rows, row_stride, search_size, _ptr(stream)))
+    st = _fast().q3k_argmax_bf16_noalloc(x, out, rows, row_stride, search_size, stream)
+    if st is None:
+        st = load().q3k_argmax_bf16_noalloc(_ptr(x), _ptr(out), rows, row_stride, search_size, _ptr(stream))
+    _check(st)
 
 
 def argmax_workspace_bytes(rows, search_size):
@@ -259,9 +324,13 @@ def argmax_workspace_bytes(rows, search_size):
 
 def topk_candidates(logits, rows, row_stride, search_size, k, cap, count, cand_index, cand_logit, nonfinite,
                     stream=None, workspace=None, workspace_bytes=0):
-    _check(load().q3k_topk_candidates_bf16(_ptr(logits), rows, row_stride, search_size, k, cap, _ptr(count),
-                                           _ptr(cand_index), _ptr(cand_logit), _ptr(nonfinite), _ptr(workspace),
-                                           workspace_bytes, _ptr(stream)))
+    st = _fast().q3k_topk_candidates_bf16(logits, rows, row_stride, search_size, k, cap, count, cand_index,
+                                          cand_logit, nonfinite, workspace, workspace_bytes, stream)
+    if st is None:
+        st = load().q3k_topk_candidates_bf16(_ptr(logits), rows, row_stride, search_size, k, cap, _ptr(count),
+                                             _ptr(cand_index), _ptr(cand_logit), _ptr(nonfinite), _ptr(workspace),
+                                             workspace_bytes, _ptr(stream))
+    _check(st)
 
 
 def topk_workspace_bytes(rows, search_size, k):
@@ -269,15 +338,22 @@ def topk_workspace_bytes(rows, search_size, k):
 
 
 def kv_append(k, v, k_cache, v_cache, B, S, row_bytes, seq_cap, start, stream=None):
-    _check(load().q3k_kv_append(_ptr(k), _ptr(v), _ptr(k_cache), _ptr(v_cache), B, S, row_bytes, seq_cap, start,
-                                _ptr(stream)))
+    st = _fast().q3k_kv_append(k, v, k_cache, v_cache, B, S, row_bytes, seq_cap, start, stream)
+    if st is None:
+        st = load().q3k_kv_append(_ptr(k), _ptr(v), _ptr(k_cache), _ptr(v_cache), B, S, row_bytes, seq_cap, start,
+                                  _ptr(stream))
+    _check(st)
 
 
 def qk_norm_rope_kv_append(q, k, v, qw, kw, B, S, Hq, Hkv, D, eps, cache, P, start, k_cache, v_cache, seq_cap,
                            cache_start, positions=None, stream=None):
-    _check(load().q3k_qk_norm_rope_kv_append_bf16(_ptr(q), _ptr(k), _ptr(v), _ptr(qw), _ptr(kw), B, S, Hq, Hkv, D,
-                                                  eps, _ptr(cache), P, start, _ptr(positions), _ptr(k_cache),
-                                                  _ptr(v_cache), seq_cap, cache_start, _ptr(stream)))
+    st = _fast().q3k_qk_norm_rope_kv_append_bf16(q, k, v, qw, kw, B, S, Hq, Hkv, D, eps, cache, P, start, positions,
+                                                 k_cache, v_cache, seq_cap, cache_start, stream)
+    if st is None:
+        st = load().q3k_qk_norm_rope_kv_append_bf16(_ptr(q), _ptr(k), _ptr(v), _ptr(qw), _ptr(kw), B, S, Hq, Hkv, D,
+                                                    eps, _ptr(cache), P, start, _ptr(positions), _ptr(k_cache),
+                                                    _ptr(v_cache), seq_cap, cache_start, _ptr(stream))
+    _check(st)
 
 
 def build_rope_cache(P: int, D: int, theta: float):

@@ -6,6 +6,8 @@ Outputs (in-tree, git-ignored, shipped with the source tree to the GPU box):
                                compiled for gfx950 with hipcc.
 * ``lib/libq3k_bench.so``     the benchmark's measurement kernels
                                (``include/q3k_bench.h``), kept out of libq3k.so.
+* ``lib/q3k_calls.so``        the C entry points as Python callables
+                               (``csrc/python``), linked to libq3k.so.
 * ``lib/libqwen3_runtime.so`` the C++ ``qwen3::`` core tensor layer and the
                                ``qwen3::ops`` drop-in API, linked to libq3k.so.
 * ``tests/cpp/build/*``       C++ test executables (built only when their
@@ -27,6 +29,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 REPO_DIR = os.path.dirname(PKG_DIR)
@@ -126,6 +129,17 @@ def build_bench_kernels(verbose=False) -> str:
     return out
 
 
+def build_python_calls(verbose=False) -> str:
+    """lib/q3k_calls.so: the C entry points as Python callables (csrc/python/q3k_calls.cpp)."""
+    src = os.path.join(PKG_DIR, "csrc", "python", "q3k_calls.cpp")
+    out = os.path.join(LIB_DIR, "q3k_calls.so")
+    tmp = out + ".tmp"
+    _run(["g++", *CXX_FLAGS, "-fvisibility=hidden", f"-I{sysconfig.get_paths()['include']}", "-shared", src, "-o", tmp,
+          f"-L{LIB_DIR}", "-lq3k", "-Wl,-rpath,$ORIGIN"], verbose=verbose)
+    os.replace(tmp, out)
+    return out
+
+
 def build_runtime(verbose=False) -> str | None:
     sources = []
     for d in HOST_DIRS:
@@ -203,7 +217,8 @@ def build_benches(verbose=False) -> list[str]:
 def build_all(verbose=False) -> dict:
     if shutil.which(HIPCC) is None and not os.path.exists(HIPCC):
         raise RuntimeError(f"hipcc not found at {HIPCC}")
-    result = {"kernels": build_kernels(verbose), "bench_kernels": build_bench_kernels(verbose),
+    result = {"kernels": build_kernels(verbose), "python_calls": build_python_calls(verbose),
+              "bench_kernels": build_bench_kernels(verbose),
               "oracle": build_oracle(verbose)}
     result["runtime"] = build_runtime(verbose)
     result["cpp_tests"] = build_cpp_tests(verbose) if result["runtime"] else []
