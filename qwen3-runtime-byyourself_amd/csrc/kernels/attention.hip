@@ -235,11 +235,24 @@ namespace q3k
                             8 * (tj % 2);
         }
 
+        // The V^T fragment of P V step i (key chunk i / 4, dims 32 (i % 4) .. + 31):
+        // keys 16 (i / 4) + 8 t + 4 lg + 0..3 in elements 4 t .. 4 t + 3, the keys
+        // of the P^T elements this lane holds.
+        __device__ __forceinline__ bf16x8_t read_v(const unsigned char *v_lds, const int (&v_off)[kAttD / 32], int i)
+        {
+            const unsigned char *vp = v_lds + v_off[i % 4] + 16 * (i / 4) * kRowBytes;
+            const bf16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4_t *)(vp));
+            const bf16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4_t *)(vp + 8 * kRowBytes));
+            return __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+
         // S^T = K Q^T for the 32 HH keys of a tile (sacc[hh]: keys 32 hh .. + 31).
         // The K fragment reads run kAhead steps ahead of the MFMAs that use them.
-        template <int HH>
+        // When its own reads have run out it calls next(x), x < kAhead, for the
+        // reads of the product that follows.
+        template <int HH, typename Next>
         __device__ __forceinline__ void qk_tile(const unsigned char *k_lds, const bf16x8_t (&qf)[kAttD / 16], int li,
-                                                int lg, f32x16_t (&sacc)[HH])
+                                                int lg, f32x16_t (&sacc)[HH], Next next)
         {
             auto read_k = [&](int c, int hh) __attribute__((always_inline)) {
                 return *reinterpret_cast<const Vec8 *>(k_lds + (32 * hh + li) * kRowBytes +
@@ -261,6 +274,8 @@ namespace q3k
 #pragma unroll
                     for (int hh = 0; hh < HH; ++hh)
                         kq[(c + kAhead) % (kAhead + 1)][hh] = read_k(c + kAhead, hh);
+                if (c + kAhead >= kAttD / 16)
+                    next(c + kAhead - kAttD / 16);
                 __builtin_amdgcn_sched_barrier(0); // keep the reads ahead of these MFMAs
 #pragma unroll
                 for (int hh = 0; hh < HH; ++hh)
@@ -356,29 +371,18 @@ namespace q3k
 
         // O^T += V^T P^T for one tile: step i covers the 16-key chunk i / 4
         // (hh = i / 8, mm = (i / 4) % 2) and dims 32 (i % 4) .. + 31.  The
-        // transpose reads run kAhead steps ahead of the MFMAs that use them.
+        // transpose reads run kAhead steps ahead of the MFMAs that use them; the
+        // first kAhead are in vq already.
         template <int HH>
         __device__ __forceinline__ void pv_tile(const unsigned char *v_lds, const int (&v_off)[kAttD / 32],
                                                 const bf16x8_t (&phi)[HH][2], const bf16x8_t (&plo)[HH][2],
-                                                f32x16_t (&o)[kAttD / 32])
+                                                f32x16_t (&o)[kAttD / 32], bf16x8_t (&vq)[kAhead + 1])
         {
-            auto read_v = [&](int i) __attribute__((always_inline)) {
-                // keys 16 (i / 4) + 8 t + 4 lg + 0..3 in elements 4 t .. 4 t + 3:
-                // the keys of the P^T elements this lane holds
-                const unsigned char *vp = v_lds + v_off[i % 4] + 16 * (i / 4) * kRowBytes;
-                const bf16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4_t *)(vp));
-                const bf16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4_t *)(vp + 8 * kRowBytes));
-                return __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-            };
-            bf16x8_t vq[kAhead + 1];
-#pragma unroll
-            for (int i = 0; i < kAhead; ++i)
-                vq[i] = read_v(i);
 #pragma unroll
             for (int i = 0; i < 8 * HH; ++i)
             {
                 if (i + kAhead < 8 * HH)
-                    vq[(i + kAhead) % (kAhead + 1)] = read_v(i + kAhead);
+                    vq[(i + kAhead) % (kAhead + 1)] = read_v(v_lds, v_off, i + kAhead);
                 __builtin_amdgcn_sched_barrier(0); // keep the reads ahead of these MFMAs
                 const int dt = i % 4, hh = i / 8, mm = (i / 4) % 2;
                 o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vq[i % (kAhead + 1)], phi[hh][mm], o[dt], 0, 0, 0);
@@ -636,11 +640,15 @@ namespace q3k
                     // instead of competing for issue with the MFMAs (prefill 4%
                     // faster at config 4).
                     __builtin_amdgcn_s_setprio(1);
-                    qk_tile<HH>(k_cur + kw * kTileBytes, qf, li, lg, sacc);
+                    bf16x8_t vq[kAhead + 1];
+                    qk_tile<HH>(k_cur + kw * kTileBytes, qf, li, lg, sacc, [&](int x) __attribute__((always_inline)) {
+                        if constexpr (decltype(with_pv)::value)
+                            vq[x] = read_v(v_prev + kw * kTileBytes, v_off, x);
+                    });
                     if (key0 + kKeys - 1 > start + wave_s0 || wave_partial)
                         mask_tile<HH>(sacc, key0, lg, last_key, col_ok);
                     if constexpr (decltype(with_pv)::value)
-                        pv_tile<HH>(v_prev + kw * kTileBytes, v_off, phi, plo, o);
+                        pv_tile<HH>(v_prev + kw * kTileBytes, v_off, phi, plo, o, vq);
                     __builtin_amdgcn_s_setprio(0);
                     const float alpha = softmax_tile<HH>(sacc, scale2, m, l, phi, plo);
                     // o holds the tiles before this one at the previous reference
@@ -672,10 +680,12 @@ namespace q3k
             }
             if (wave_active && mine > 0)
             {
-                if ((mine - 1) % 2 == 0)
-                    pv_tile<HH>(v_a + kw * kTileBytes, v_off, phi, plo, o);
-                else
-                    pv_tile<HH>(v_b + kw * kTileBytes, v_off, phi, plo, o);
+                const unsigned char *v_last = ((mine - 1) % 2 == 0 ? v_a : v_b) + kw * kTileBytes;
+                bf16x8_t vq[kAhead + 1];
+#pragma unroll
+                for (int x = 0; x < kAhead; ++x)
+                    vq[x] = read_v(v_last, v_off, x);
+                pv_tile<HH>(v_last, v_off, phi, plo, o, vq);
             }
 
             const int64_t row = (b * a.S + s_col) * a.Hq + h_col;
@@ -776,7 +786,7 @@ namespace q3k
                 else
                     wait_loads<kL>();
                 f32x16_t sacc[1];
-                qk_tile<1>(kb + kw * kTileBytes, qf, li, lg, sacc);
+                qk_tile<1>(kb + kw * kTileBytes, qf, li, lg, sacc, [](int) __attribute__((always_inline)) {});
                 wait_loads<63>();
                 if (j + 2 < mine)
                     load_k(j + 2, kb);
@@ -793,7 +803,11 @@ namespace q3k
                     wait_loads<2 * kL>();
                 else
                     wait_loads<0>();
-                pv_tile<1>(vb + kw * kTileBytes, v_off, phi, plo, o);
+                bf16x8_t vq[kAhead + 1];
+#pragma unroll
+                for (int x = 0; x < kAhead; ++x)
+                    vq[x] = read_v(vb + kw * kTileBytes, v_off, x);
+                pv_tile<1>(vb + kw * kTileBytes, v_off, phi, plo, o, vq);
                 wait_loads<63>();
                 if (j + 2 < mine)
                     load_v(j + 2, vb);
