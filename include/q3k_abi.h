@@ -210,8 +210,9 @@ Q3K_API int q3k_gqa_attention_bf16(const uint16_t *q, const uint16_t *k_cache,
 
 /*
  * Workspace bytes that let q3k_gqa_attention_bf16 split this shape's key
- * range (0: it does not split).  A call may leave it unused where one launch
- * is the faster way (a few hundred keys).  No counterpart in the reference
+ * range (0: it does not split), and that of any shorter context: one of the
+ * size for the cache's length serves every step up to it.  A call may leave
+ * it unused where one launch is the faster way (a few hundred keys).  No counterpart in the reference
  * (its kernel is one block per query row).
  */
 Q3K_API int64_t q3k_gqa_attention_workspace_bytes(int64_t B, int64_t S,

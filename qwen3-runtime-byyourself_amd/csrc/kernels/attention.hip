@@ -1230,5 +1230,5 @@ extern "C" int64_t q3k_gqa_attention_workspace_bytes(int64_t B, int64_t S, int32
     if (B <= 0 || S <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || D != q3k::kAttD || cached < S ||
         B * S * Hq > INT32_MAX)
         return 0;
-    return q3k::plan_attention_split(B, S, Hq, Hkv, cached).bytes;
+    return q3k::attention_workspace_bytes(B, S, Hq, Hkv, cached);
 }

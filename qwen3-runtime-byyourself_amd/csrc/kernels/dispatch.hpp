@@ -84,6 +84,9 @@ namespace q3k
     // Decode slices of up to this many keys run as one-wave blocks.
     constexpr int32_t kAttMaxOneWaveSplitKeys = 2 * kAttKeyTile;
     constexpr int32_t kAttDecodeTile = 32; // keys of a decode wave's tile
+    // Most blocks a decode step's slices make: of 3593 shapes of up to 511 pairs and
+    // 32768 keys the estimate below wanted more for two.
+    constexpr int64_t kAttDecodeMaxBlocks = 2048;
 
     struct AttnSplit
     {
@@ -287,6 +290,8 @@ namespace q3k
             return best;
         for (const int slices : {2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64})
         {
+            if (slices > kAttDecodeMaxBlocks / pairs)
+                break;
             const int64_t keys = blocks_for(blocks_for(cached, slices), kAttDecodeTile) * kAttDecodeTile;
             if (keys >= cached || keys < 2 * kAttDecodeTile)
                 continue;
@@ -310,12 +315,40 @@ namespace q3k
         return best;
     }
 
-    // The key split the workspace is for.
+    // The key split of a call with a workspace.
     inline AttnSplit plan_attention_split(int64_t B, int64_t S, int32_t Hq, int32_t Hkv, int64_t cached)
     {
         if (S * (Hq / Hkv) <= kAttColsPerWave)
             return plan_attention_decode(B, S, Hq, Hkv, cached, true);
         return plan_attention_prefill(B, S, Hq, Hkv, cached, true);
+    }
+
+    // Workspace of the most slices a call of up to `cached` keys may be cut into: a
+    // caller that sizes it once for the length of its cache never has too little
+    // for a shorter context.  (The plan's own slices go up and down with the length:
+    // 64 sequences of 4 / 1 heads take 4 slices at 16384 keys and 16 at 1924.)
+    inline int64_t attention_workspace_bytes(int64_t B, int64_t S, int32_t Hq, int32_t Hkv, int64_t cached)
+    {
+        const int64_t pairs = B * Hkv, cols = S * (Hq / Hkv);
+        int64_t most, keys; // slices, and the fewest keys of one
+        if (cols <= kAttColsPerWave)
+        {
+            if (pairs >= kAttSplitTargetBlocks || cached < 2 * kAttKeyTile)
+                return 0;
+            most = kAttDecodeMaxBlocks / pairs;
+            keys = 2 * kAttDecodeTile;
+        }
+        else
+        {
+            const int64_t blocks = pairs * blocks_for(cols, attn_block_cols(1));
+            if (blocks > kAttSplitTargetBlocks / 2)
+                return 0;
+            most = kAttSplitTargetBlocks / blocks + 1;
+            keys = 2 * kAttKeyTile;
+        }
+        for (const int64_t bound : {static_cast<int64_t>(kAttMaxSplits), blocks_for(cached, keys)})
+            most = most < bound ? most : bound;
+        return most < 2 ? 0 : most * B * S * Hq * (kAttHeadDim + 2) * 4;
     }
 
     struct AttnPlan
