@@ -150,7 +150,7 @@ def load(path: str | None = None) -> ctypes.CDLL:
         spec = importlib.util.spec_from_file_location("q3k_calls", CALLS_PATH, loader=loader)
         calls = importlib.util.module_from_spec(spec)
         loader.exec_module(calls)
-        _lib, _calls = lib, calls
+        _calls, _lib = calls, lib  # _lib last: once it is set, a second thread takes both
     return lib
 
 
