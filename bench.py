@@ -340,9 +340,9 @@ def time_sampling(q3k, hip, synth, configs, c, stream):
             x, B, V, V, k, cap, cnt, ci, cv, bad, stream, workspace=ws_k, workspace_bytes=wk))], 50, 5)
         nb = B * V * 2
         out[f"argmax_b{B}_v{V}"] = {"ms": round(ms_a, 5), "bytes": nb, "GB/s": round(nb / (ms_a * 1e-3) / 1e9, 1),
-                                    "sliced": wa > 0}
+                                    "workspace_bytes": wa}
         out[f"topk{k}_candidates_b{B}_v{V}"] = {"ms": round(ms_k, 5), "bytes_read_2_passes": 2 * nb,
-                                                "logits_GB/s": round(nb / (ms_k * 1e-3) / 1e9, 1), "sliced": wk > 0}
+                                                "logits_GB/s": round(nb / (ms_k * 1e-3) / 1e9, 1), "workspace_bytes": wk}
         for buf in (x, ids, cnt, bad, ci, cv, ws_a, ws_k):
             if buf is not None:
                 buf.free()
