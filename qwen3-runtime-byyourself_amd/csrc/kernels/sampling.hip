@@ -415,14 +415,18 @@ namespace q3k
         // each (k groups hold a logit at or above it; about 256 ln(256 / (256 - k))
         // logits reach it: 21 for k = 20, 226 for k = 150).  Above that the k-th
         // largest of the thread maxima, as in the other kernels.  The k-th largest
-        // of up to 512 values is found by every wave for itself, bit by bit with
-        // ballots (15 steps, no barrier), for the bound and for the short list.
+        // of up to 512 values is found by a wave bit by bit with ballots (15 steps,
+        // no barrier): by one wave for the bound, by those that write for the short list.
         //
-        // 64 rows of 151936: 11.0 us at k = 20 and 15.5 at k = 150, where slices and
-        // merge took 15.5 and 18.8 and one block a row that read twice 17.3 and 19.6;
-        // 256 rows of 151669: 17.6 against 29.7 and 27.8.  Beside the read (6 us at 64
-        // rows) it is the list that takes time, an LDS atomic a logit; listing by
-        // wave segments without atomics (readlane a vector) measured 14.3 and 19.7.
+        // The list is made in two steps: vectors that hold a logit at or above the
+        // bound go to LDS with one atomic a wave, and all threads then test their
+        // columns.  An append a column, 160 in line, made the code 16500 lines and its
+        // fetching took as long as the read.
+        //
+        // 64 rows of 151936: 9.9 us at k = 20, 12.1 at k = 150, 14.8 at k = 600 (10.7,
+        // 15.2 and 19.4 with an append a column; 15.5 and 18.8 as slices and merge at k = 20
+        // and 150); 256 rows of 151669: 17.1 and 19.1 (17.7 and 21.9; 29.7 and 31.6).
+        // Listing by wave segments (readlane a vector) measured 14.3 and 19.7.
         constexpr int kRegVecs = 20;
         constexpr int64_t kRegColumns = int64_t{8} * kRegVecs * kSelBlock;
         constexpr uint32_t kGroupK = 192;
@@ -467,6 +471,31 @@ namespace q3k
             return t;
         }
 
+        // Sum of c (below 32) over the wave's lower lanes, and over all of them.
+        __device__ __forceinline__ uint32_t wave_prefix(uint32_t c, uint32_t *total)
+        {
+            uint32_t below = 0, all = 0;
+#pragma unroll
+            for (int bit = 0; bit < 5; ++bit)
+            {
+                const uint64_t b = __ballot((c >> bit & 1u) != 0u);
+                below += __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(b >> 32),
+                                                   __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(b), 0u))
+                         << bit;
+                all += static_cast<uint32_t>(__popcll(b)) << bit;
+            }
+            *total = all;
+            return below;
+        }
+
+        // A row's vectors that hold a logit at or above the bound.
+        struct HitVectors
+        {
+            Vec8 vec[kCandMax];
+            int32_t column[kCandMax];
+            uint32_t count;
+        };
+
         // The list entries at or above its k-th largest (k <= nl <= SLOTS waves'
         // worth of lanes): each wave finds it and writes its own 64 entries.
         template <int SLOTS>
@@ -497,12 +526,29 @@ namespace q3k
             }
         }
 
+        // The rows the register path leaves, out of line: inlined, their addresses
+        // took registers that the row needs.
+        __device__ __noinline__ void select_rest(const uint16_t *r, int64_t n, uint32_t k, int64_t row, CandOut co,
+                                                 SelShared &sh, bool whole)
+        {
+            if (whole)
+            {
+                whole_row_select(r, n, k, row, co, sh);
+                return;
+            }
+            if (threadIdx.x == 0)
+                sh.listed = 0u;
+            __syncthreads();
+            select_reading(r, n, k, row, co, sh);
+        }
+
         __global__ __launch_bounds__(kSelBlock) void topk_row_kernel(const uint16_t *__restrict__ x, int64_t rows,
                                                                      int64_t stride, int32_t n, uint32_t k, CandOut co,
                                                                      int32_t *__restrict__ count,
                                                                      int32_t *__restrict__ nonfinite)
         {
             __shared__ SelShared sh;
+            __shared__ HitVectors hits;
             const int tid = threadIdx.x, lane = tid % kWave;
             for (int64_t row = blockIdx.x; row < rows; row += gridDim.x)
             {
@@ -530,6 +576,7 @@ namespace q3k
                     sh.found = 0u;
                     sh.bad = 0u;
                     sh.listed = 0u;
+                    hits.count = 0u;
                 }
                 __syncthreads();
                 // 1. maxima and the non-finite flag
@@ -564,11 +611,19 @@ namespace q3k
                     int32_t bound;
                     if (k <= kGroupK)
                     {
-                        int32_t g[4];
+                        // one wave: side by side, the 16 waves' steps held each other up
+                        if (tid < kWave)
+                        {
+                            int32_t g[4];
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            g[i] = sh.group_max[i * kWave + lane];
-                        bound = wave_kth<4>(g, k);
+                            for (int i = 0; i < 4; ++i)
+                                g[i] = sh.group_max[i * kWave + lane];
+                            const int32_t t = wave_kth<4>(g, k);
+                            if (lane == 0)
+                                sh.bound = static_cast<uint32_t>(t);
+                        }
+                        __syncthreads();
+                        bound = static_cast<int32_t>(sh.bound);
                     }
                     else
                         bound = static_cast<int32_t>(
@@ -583,25 +638,49 @@ namespace q3k
                                 sh.list_index[pos] = index;
                             }
                         };
+                        // vectors that hold a logit at or above the bound
+                        uint32_t mask = 0;
                         if (tmax >= bound)
-                        {
-                            if (static_cast<int16_t>(side_bits) >= bound)
-                                append(side_bits, side);
 #pragma unroll
                             for (int u = 0; u < kRegVecs; ++u)
                             {
-                                if (top_i16(max_i16x2(max_i16x2(v[u].d[0], v[u].d[1]), max_i16x2(v[u].d[2], v[u].d[3]))) < bound)
-                                    continue;
-                                const int32_t c = first + 8 * (tid + u * kSelBlock);
-#pragma unroll
-                                for (int e = 0; e < 8; ++e)
-                                {
-                                    const uint32_t b = e % 2 == 0 ? v[u].d[e / 2] & 0xffffu : v[u].d[e / 2] >> 16;
-                                    if (static_cast<int16_t>(b) >= bound)
-                                        append(b, c + e);
-                                }
+                                const uint32_t m = max_i16x2(max_i16x2(v[u].d[0], v[u].d[1]), max_i16x2(v[u].d[2], v[u].d[3]));
+                                mask |= top_i16(m) >= bound ? 1u << u : 0u;
                             }
+                        uint32_t total;
+                        uint32_t pos = wave_prefix(static_cast<uint32_t>(__popc(mask)), &total);
+                        uint32_t base = 0;
+                        if (lane == 0 && total != 0)
+                            base = atomicAdd(&hits.count, total);
+                        pos += __builtin_amdgcn_readfirstlane(base);
+#pragma unroll
+                        for (int u = 0; u < kRegVecs; ++u)
+                            if ((mask >> u & 1u) != 0u)
+                            {
+                                if (pos < static_cast<uint32_t>(kCandMax))
+                                {
+                                    hits.vec[pos] = v[u];
+                                    hits.column[pos] = first + 8 * (tid + u * kSelBlock);
+                                }
+                                ++pos;
+                            }
+                        if (static_cast<int16_t>(side_bits) >= bound)
+                            append(side_bits, side);
+                        __syncthreads();
+                        // each of them has one at least: past kCandMax the list would overflow
+                        const uint32_t nh = hits.count;
+                        if (nh > static_cast<uint32_t>(kCandMax))
+                        {
+                            if (tid == 0)
+                                sh.listed = kCandMax + 1;
                         }
+                        else
+                            for (uint32_t i = tid; i < 8 * nh; i += kSelBlock)
+                            {
+                                const uint32_t bits = reinterpret_cast<const uint16_t *>(hits.vec)[i];
+                                if (static_cast<int16_t>(bits) >= bound)
+                                    append(bits, hits.column[i / 8] + static_cast<int32_t>(i % 8));
+                            }
                         __syncthreads();
                         const uint32_t nl = sh.listed;
                         if (nl <= static_cast<uint32_t>(kCandMax))
@@ -620,15 +699,7 @@ namespace q3k
                 __syncthreads();
                 if (!exact)
                 {
-                    if (bad || sh.listed > static_cast<uint32_t>(kCandMax))
-                        whole_row_select(r, n, k, row, co, sh);
-                    else
-                    {
-                        if (tid == 0)
-                            sh.listed = 0u;
-                        __syncthreads();
-                        select_reading(r, n, k, row, co, sh);
-                    }
+                    select_rest(r, n, k, row, co, sh, bad || sh.listed > static_cast<uint32_t>(kCandMax));
                     __syncthreads();
                 }
                 if (tid == 0)
