@@ -8,9 +8,8 @@
 // ~index in the low word, so "larger value, then smaller index" is a plain
 // unsigned max.  One block of 1024 threads per row (rows strided over the
 // grid): 128-bit loads of the row's aligned middle, a thread's maximum from the
-// plain bits as packed 16-bit integers (a key per thread, not per element; rows
-// without a positive value or with a NaN start over with a key per element), wave
-// and block maxima by DPP and through LDS.  When rows are longer than
+// bits as packed 16-bit integers (a key per thread, not per element), wave and
+// block maxima by DPP and through LDS.  When rows are longer than
 // kWholeRowColumns, too few to fill the GPU, and the caller gives a workspace,
 // each row is cut into slices of whole 8-column
 // vectors: one block per (row, slice) writes the slice's best key, and a
@@ -35,8 +34,6 @@ namespace q3k
             const uint32_t ord = (b & 0x8000u) ? (~b & 0xffffu) : (b | 0x8000u);
             return (static_cast<uint64_t>(ord) << 32) | (0xffffffffu - index);
         }
-
-        __device__ __forceinline__ uint64_t max_u64(uint64_t a, uint64_t b) { return a > b ? a : b; }
 
         // Maximum over the wave's lanes, in every lane: DPP within 16-lane rows,
         // permlane swaps across them (VALU only, no LDS round trip).
@@ -78,147 +75,178 @@ namespace q3k
             }
         };
 
-        // This thread's best key over columns [begin, end) of row r: any values.
         constexpr int kUnroll = 5;
-        __device__ uint64_t thread_best_any(const uint16_t *r, int64_t begin, int64_t end)
-        {
-            uint64_t best = 0; // below every candidate
-            const Middle mid(r, begin, end);
-            const Vec8 *rv = reinterpret_cast<const Vec8 *>(r + mid.first);
-            for (int64_t i = threadIdx.x; i < mid.count; i += kUnroll * kArgmaxBlock)
-            {
-                Vec8 v[kUnroll];
-#pragma unroll
-                for (int u = 0; u < kUnroll; ++u)
-                    if (i + u * kArgmaxBlock < mid.count)
-                        v[u] = load8<false>(rv + i + u * kArgmaxBlock);
-#pragma unroll
-                for (int u = 0; u < kUnroll; ++u)
-                    if (i + u * kArgmaxBlock < mid.count)
-                    {
-                        const uint32_t c = static_cast<uint32_t>(mid.first + 8 * (i + u * kArgmaxBlock));
-#pragma unroll
-                        for (int j = 0; j < 8; ++j)
-                            best = max_u64(best, argmax_key(j % 2 == 0 ? v[u].d[j / 2] & 0xffffu : v[u].d[j / 2] >> 16, c + j));
-                    }
-            }
-            const int64_t side = mid.side(threadIdx.x);
-            if (side >= 0)
-                best = max_u64(best, argmax_key(r[side], static_cast<uint32_t>(side)));
-            return best;
-        }
-
         typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
         __device__ __forceinline__ uint32_t max_i16x2(uint32_t a, uint32_t b)
         {
             return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(i16x2, a), __builtin_bit_cast(i16x2, b)));
         }
 
-        // This thread's best key over columns [begin, end) of row r when the range
-        // holds a positive finite or infinite value and no positive NaN (the bits
-        // are then in order as signed 16-bit integers: everything negative, NaN
-        // included, sorts below).  Returns the plain bits' maximum in *top: a block
-        // whose maximum is outside (0, +inf] starts over with thread_best_any.
+        // Two bf16 with NaN as -inf.
+        __device__ __forceinline__ uint32_t without_nan(uint32_t d)
+        {
+            const i16x2 inf = {0x7f80, 0x7f80};
+            const uint32_t nan = __builtin_bit_cast(uint32_t, (inf - __builtin_bit_cast(i16x2, d & 0x7fff7fffu)) >> 15);
+            return (nan & 0xff80ff80u) | (~nan & d);
+        }
+
+        // Largest of a vector's eight 16-bit integers.
+        __device__ __forceinline__ int32_t max_of(uint32_t d0, uint32_t d1, uint32_t d2, uint32_t d3)
+        {
+            const uint32_t m = max_i16x2(max_i16x2(d0, d1), max_i16x2(d2, d3));
+            const int32_t lo = static_cast<int16_t>(m & 0xffffu), hi = static_cast<int32_t>(m) >> 16;
+            return lo > hi ? lo : hi;
+        }
+
+        // The largest value a thread has scanned, in its scan's own integers, and the
+        // vector that holds its first occurrence.
+        struct Scan
+        {
+            int32_t best;
+            int32_t at;
+            Vec8 vec;
+            __device__ __forceinline__ void take(int32_t x, int32_t i, const Vec8 &v)
+            {
+                if (x > best)
+                {
+                    best = x;
+                    at = i;
+                    vec = v;
+                }
+            }
+        };
+
+        // 16 bits of bf16 as integers in order among positive values, everything else
+        // below: the plain bits, signed.
+        __device__ __forceinline__ int32_t positive_of(uint32_t bits)
+        {
+            return static_cast<int16_t>(without_nan(bits) & 0xffffu);
+        }
+        // In order among the others: 0x7fff less the magnitude's bits, so the zeros are
+        // 0x7fff, -inf 0x7f and NaN below.
+        __device__ __forceinline__ int32_t negative_of(uint32_t bits) { return static_cast<int32_t>(~bits & 0x7fffu); }
+
+        // This thread's best key over columns [begin, end) of row r, or 0 (below every
+        // candidate): the best of all threads' is the row's.
         //
         // The 16-byte aligned middle of the range goes kUnroll vectors a thread at a
         // time, all loaded before any is used; of the vectors seen only the one
-        // holding the first maximum is kept.  Two packed-max instructions do a
-        // dword pair; a 64-bit key per element made the kernel VALU-bound (64 x
-        // 151936: 7.5 us of kernel, 12 instructions an element).
-        __device__ __forceinline__ uint64_t thread_best(const uint16_t *r, int64_t begin, int64_t end, int32_t *top)
+        // holding the first maximum is kept.  A wave that sees a positive value in its
+        // first vectors scans for those alone: a packed instruction for two columns (a
+        // 64-bit key per element made the kernel VALU-bound, 64 x 151936: 7.5 us of
+        // kernel, 12 instructions an element).  A wave that sees none scans for both,
+        // and each of its threads takes the negative maximum if it finds nothing
+        // positive; where that is -inf all its columns are -inf or NaN, and the first
+        // of them is the one.  Nothing is read twice: a second pass with a key per
+        // element over rows without a positive value or with a NaN took as long again
+        // as one and a half reads (no positive value, 1 / 64 / 256 rows of 151936: 5.7 /
+        // 6.8 / 13.6 us, 19.7 / 21.2 / 30.0 with the second pass; ordinary rows 4.6 / 6.2 /
+        // 13.2 either way).
+        __device__ __forceinline__ uint64_t thread_best(const uint16_t *r, int64_t begin, int64_t end)
         {
             const Middle mid(r, begin, end);
-            const int64_t nv = mid.count;
+            const int32_t nv = static_cast<int32_t>(mid.count); // below 2^28
             const Vec8 *rv = reinterpret_cast<const Vec8 *>(r + mid.first);
-            int32_t best = INT32_MIN; // below every 16-bit value
-            int64_t at = 0;
-            Vec8 keep{};
-            for (int64_t i = threadIdx.x; i < nv; i += kUnroll * kArgmaxBlock)
+            int32_t tid = threadIdx.x;
+            __asm__ volatile("" : "+v"(tid)); // nothing of a row is kept in registers for the next one
+            const int64_t side = mid.side(tid);
+            Scan p{0, 0, {}}, n{-1, 0, {}};
+            bool negative = true; // the wave has seen no positive value in its first vectors
+            for (int32_t i0 = 0; i0 < nv; i0 += kUnroll * kArgmaxBlock)
             {
+                // past the end a thread reads the last vector once more
                 Vec8 v[kUnroll];
+                auto index = [&](int u) __attribute__((always_inline)) {
+                    const int32_t i = i0 + tid + u * kArgmaxBlock;
+                    return i < nv ? i : nv - 1;
+                };
 #pragma unroll
                 for (int u = 0; u < kUnroll; ++u)
-                    if (i + u * kArgmaxBlock < nv)
-                        v[u] = load8<false>(rv + i + u * kArgmaxBlock);
+                    v[u] = load8<false>(rv + index(u));
+                int32_t x[kUnroll], top = 0;
+                auto maxima = [&]() __attribute__((always_inline)) {
 #pragma unroll
-                for (int u = 0; u < kUnroll; ++u)
-                    if (i + u * kArgmaxBlock < nv)
+                    for (int u = 0; u < kUnroll; ++u)
                     {
-                        const uint32_t m = max_i16x2(max_i16x2(v[u].d[0], v[u].d[1]), max_i16x2(v[u].d[2], v[u].d[3]));
-                        const int32_t lo = static_cast<int16_t>(m & 0xffffu), hi = static_cast<int32_t>(m) >> 16;
-                        const int32_t mx = lo > hi ? lo : hi;
-                        if (mx > best)
-                        {
-                            best = mx;
-                            at = i + u * kArgmaxBlock;
-                            keep = v[u];
-                        }
+                        x[u] = max_of(v[u].d[0], v[u].d[1], v[u].d[2], v[u].d[3]);
+                        top = x[u] > top ? x[u] : top;
+                    }
+                };
+                maxima();
+                if (__ballot(top > p.best) != 0)
+                {
+                    if (__ballot(top > 0x7f80) != 0)
+                    {
+#pragma unroll
+                        for (int u = 0; u < kUnroll; ++u)
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                v[u].d[j] = without_nan(v[u].d[j]);
+                        top = 0;
+                        maxima();
+                    }
+#pragma unroll
+                    for (int u = 0; u < kUnroll; ++u)
+                        p.take(x[u], index(u), v[u]);
+                }
+                if (i0 == 0)
+                    negative = __ballot(p.best > 0) == 0;
+                if (negative)
+#pragma unroll
+                    for (int u = 0; u < kUnroll; ++u)
+                    {
+                        constexpr uint32_t kMagnitude = 0x7fff7fffu;
+                        n.take(max_of(~v[u].d[0] & kMagnitude, ~v[u].d[1] & kMagnitude, ~v[u].d[2] & kMagnitude,
+                                      ~v[u].d[3] & kMagnitude),
+                               index(u), v[u]);
                     }
             }
-            uint32_t index = 0;
-            if (best != INT32_MIN)
-            {
-                int e = 7;
+            // the column of a scan's best, the side column included
+            const uint32_t side_bits = side >= 0 ? r[side] : 0u;
+            auto column = [&](Scan &s, bool any, auto value) __attribute__((always_inline)) {
+                uint32_t at = 0;
+                if (any)
+                {
+                    int e = 7;
 #pragma unroll
-                for (int j = 7; j >= 0; --j)
-                {
-                    const int32_t x = static_cast<int16_t>(j % 2 == 0 ? keep.d[j / 2] & 0xffffu : keep.d[j / 2] >> 16);
-                    e = x == best ? j : e;
+                    for (int j = 7; j >= 0; --j)
+                        e = value(j % 2 == 0 ? s.vec.d[j / 2] & 0xffffu : s.vec.d[j / 2] >> 16) == s.best ? j : e;
+                    at = static_cast<uint32_t>(mid.first + 8 * static_cast<int64_t>(s.at) + e);
                 }
-                index = static_cast<uint32_t>(mid.first + 8 * at + e);
-            }
-            const int64_t side = mid.side(threadIdx.x);
-            if (side >= 0)
-            {
-                const int32_t x = static_cast<int16_t>(r[side]);
-                if (x > best || (x == best && static_cast<uint32_t>(side) < index))
+                const int32_t x = value(side_bits);
+                if (side >= 0 && (x > s.best || (x == s.best && static_cast<uint32_t>(side) < at)))
                 {
-                    best = x;
-                    index = static_cast<uint32_t>(side);
+                    s.best = x;
+                    at = static_cast<uint32_t>(side);
                 }
-            }
-            *top = best;
-            return best > 0 ? argmax_key(static_cast<uint32_t>(best), index) : 0;
+                return at;
+            };
+            const uint32_t p_at = column(p, p.best > 0, [](uint32_t b) __attribute__((always_inline)) { return positive_of(b); });
+            if (p.best > 0)
+                return argmax_key(static_cast<uint32_t>(p.best), p_at);
+            if (!negative)
+                return 0;
+            const uint32_t n_at = column(n, n.best >= 0, [](uint32_t b) __attribute__((always_inline)) { return negative_of(b); });
+            if (n.best > 0x7f)
+                return argmax_key(0x8000u + static_cast<uint32_t>(0x7fff - n.best), n_at);
+            if (n.best < 0)
+                return 0; // no columns
+            const int64_t first = mid.first + 8 * static_cast<int64_t>(tid < nv ? tid : nv - 1);
+            return argmax_key(0xff80u, static_cast<uint32_t>(nv > 0 && (side < 0 || first < side) ? first : side));
         }
 
-        struct ArgmaxShared
-        {
-            uint64_t key[kArgmaxBlock / kWave];
-            int32_t top[kArgmaxBlock / kWave];
-        };
-
         // The best key of columns [begin, end) of row r, in every thread of wave 0;
-        // the shared memory is free again when the call returns.
-        __device__ __forceinline__ uint64_t block_best(const uint16_t *r, int64_t begin, int64_t end, ArgmaxShared &sh)
+        // the shared memory (a key a wave) is free again when the call returns.
+        constexpr int kArgmaxWaves = kArgmaxBlock / kWave;
+        __device__ __forceinline__ uint64_t block_best(const uint16_t *r, int64_t begin, int64_t end, uint64_t *wave_key)
         {
-            constexpr int kWaves = kArgmaxBlock / kWave;
             const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-            int32_t top;
-            uint64_t best = wave_max(thread_best(r, begin, end, &top));
-            const int32_t wave_top = static_cast<int32_t>(wave_max(static_cast<uint32_t>(top) ^ 0x80000000u) ^ 0x80000000u);
+            uint64_t best = wave_max(thread_best(r, begin, end));
             if (lane == 0)
-            {
-                sh.key[wave] = best;
-                sh.top[wave] = wave_top;
-            }
-            __syncthreads();
-            const int32_t t = lane < kWaves ? sh.top[lane] : INT32_MIN;
-            const int32_t block_top = static_cast<int32_t>(wave_max(static_cast<uint32_t>(t) ^ 0x80000000u) ^ 0x80000000u);
-            if (block_top > 0 && block_top <= 0x7f80)
-            {
-                if (wave == 0)
-                    best = wave_max(lane < kWaves ? sh.key[lane] : uint64_t{0});
-                __syncthreads();
-                return best;
-            }
-            // no positive value, or a NaN
-            __syncthreads();
-            best = wave_max(thread_best_any(r, begin, end));
-            if (lane == 0)
-                sh.key[wave] = best;
+                wave_key[wave] = best;
             __syncthreads();
             if (wave == 0)
-                best = wave_max(lane < kWaves ? sh.key[lane] : uint64_t{0});
+                best = wave_max(lane < kArgmaxWaves ? wave_key[lane] : uint64_t{0});
             __syncthreads();
             return best;
         }
@@ -232,10 +260,10 @@ namespace q3k
                                                                       int32_t *__restrict__ out, int64_t rows,
                                                                       int64_t stride, int64_t n)
         {
-            __shared__ ArgmaxShared sh;
+            __shared__ uint64_t wave_key[kArgmaxWaves];
             for (int64_t row = blockIdx.x; row < rows; row += gridDim.x)
             {
-                const uint64_t best = block_best(x + row * stride, 0, n, sh);
+                const uint64_t best = block_best(x + row * stride, 0, n, wave_key);
                 if (threadIdx.x == 0)
                     out[row] = key_index(best);
             }
@@ -248,11 +276,11 @@ namespace q3k
                                                                             int64_t stride, int64_t n,
                                                                             int32_t slices, int64_t slice_len)
         {
-            __shared__ ArgmaxShared sh;
+            __shared__ uint64_t wave_key[kArgmaxWaves];
             const int32_t row = static_cast<int32_t>(blockIdx.x) / slices;
             const int64_t begin = (static_cast<int32_t>(blockIdx.x) % slices) * slice_len;
             const int64_t end = begin + slice_len < n ? begin + slice_len : n;
-            const uint64_t best = block_best(x + row * stride, begin, end, sh);
+            const uint64_t best = block_best(x + row * stride, begin, end, wave_key);
             if (threadIdx.x == 0)
                 part[blockIdx.x] = best;
         }

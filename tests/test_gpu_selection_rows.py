@@ -47,6 +47,88 @@ def test_argmax_row_edges(q3k, hip, oracle, synth, n, pad, offset):
     check_exact(name, O.get(np.int32, (rows,)).view(np.uint32), oracle.argmax(x, n).view(np.uint32))
 
 
+def _special_rows(synth, n):
+    """Rows whose maximum is not an ordinary positive value: -inf but for one column of either sign, NaN of both signs
+    over negatives, over -inf and over zeros, nothing but NaN and -inf, a largest value among infinities and NaN."""
+    neg = synth.normal_bf16(191, n, (n,), std=3.0) | 0x8000
+    x = np.full((10, n), 0xff80, np.uint16)
+    x[0, n // 2] = 0x3f80
+    x[1, n - 1] = 0xc040
+    x[2] = neg
+    x[2, :: 5] = 0x7fc0
+    x[3, n // 3:] = 0x7f81
+    x[4, : n // 3 + 1] = 0xffff
+    x[5] = 0x7fff
+    x[5, n // 2:] = 0xff80
+    x[6] = neg
+    x[6, n // 2:: 3] = 0x8000
+    x[6, n // 2 + n // 4:: 3] = 0x0000
+    x[6, :: 4] = 0xff81
+    x[7] = neg
+    x[7, n // 2] = 0x0001
+    x[7, -1] = 0x7fc0
+    x[8] = neg
+    x[8, n // 2:: 9] = 0x7f80
+    x[8, 0] = 0x7f81
+    x[9] = 0xff7f
+    return x
+
+
+@pytest.mark.parametrize("n", [1, 9, 100, 8200, 40961, 151936, 300001])
+@pytest.mark.parametrize("offset", [0, 6])
+def test_argmax_special_rows(q3k, hip, oracle, synth, n, offset):
+    name = f"argmax special rows n={n} offset={offset}"
+    announce(name)
+    x = _special_rows(synth, n)
+    rows = x.shape[0]
+    X, O = Guarded(hip, x, offset=offset), Guarded(hip, nbytes=rows * 4)
+    ws = q3k.argmax_workspace_bytes(rows, n)
+    W = Guarded(hip, nbytes=ws) if ws else None
+    q3k.argmax(X, O, rows, n, n, workspace=W, workspace_bytes=ws)
+    hip.synchronize()
+    assert O.guards_intact()
+    check_exact(name, O.get(np.int32, (rows,)).view(np.uint32), oracle.argmax(x, n).view(np.uint32))
+
+
+def _us(hip, stream, fn, calls=30):
+    """The shortest of five timings: other work on the machine only adds."""
+    best = None
+    for _ in range(5):
+        fn()
+        stream.synchronize()
+        e0, e1 = hip.Event(), hip.Event()
+        e0.record(stream)
+        for _ in range(calls):
+            fn()
+        e1.record(stream)
+        e1.synchronize()
+        us = e0.elapsed_ms(e1) * 1e3 / calls
+        best = us if best is None or us < best else best
+    return best
+
+
+def _kinds(synth, rows, n):
+    """Ordinary logits; the same without a positive value; shifted so that the largest is zero."""
+    x = np.broadcast_to(synth.normal_bf16(192, n, (8, n), std=3.0)[:, None], (8, rows // 8, n)).reshape(rows, n)
+    v = synth.bf16_to_f32(x)
+    return {"ordinary": x, "negative": x | 0x8000,
+            "shifted": synth.f32_to_bf16(np.ascontiguousarray(v - v.max(axis=1, keepdims=True)))}
+
+
+def test_argmax_time_without_positive_values(q3k, hip, synth):
+    """Rows of log-probabilities or of logits less their maximum take about as long as ordinary ones: 1.1 times here,
+    3.4 times when such rows were read again with a key per element."""
+    rows, n = 64, 151936
+    stream, us = hip.Stream(), {}
+    out = hip.DeviceBuffer(rows * 4)
+    for kind, x in _kinds(synth, rows, n).items():
+        X = hip.DeviceBuffer.from_array(x)
+        us[kind] = _us(hip, stream, lambda: q3k.argmax(X, out, rows, n, n, stream))
+        X.free()
+    print(f"[time] argmax {rows} x {n}: {us}", flush=True)
+    assert max(us["negative"], us["shifted"]) < 2.0 * us["ordinary"], us
+
+
 @pytest.mark.parametrize("n,ks", [(9, (1, 9)), (100, (1, 20, 100)), (8193, (20, 192, 193)), (20000, (1, 192, 1024, 1500)),
                                   (155649, (20, 193)), (163840, (1, 64, 192, 193, 1024)), (163841, (20, 1024)),
                                   (262145, (20, 300))])
