@@ -43,6 +43,17 @@ namespace q3k
         constexpr int kSelWaves = kSelBlock / kWave;
         constexpr int kCandMax = 4096;
 
+        // threadIdx.x, where it is used: addresses that follow from it, computed before
+        // the row loop, took registers that topk_row_kernel's row needs (a spill, and
+        // 600 rows of 151936 48.9 us instead of 46.7).
+        __device__ __forceinline__ int own_thread()
+        {
+            int t = threadIdx.x;
+            __asm__ volatile("" : "+v"(t));
+            __builtin_assume(t >= 0 && t < kSelBlock);
+            return t;
+        }
+
         // order-preserving key of a finite bf16 value; -0 and +0 share a key
         // (the reference compares the scores as doubles)
         __device__ __forceinline__ uint32_t sel_key(uint32_t b)
@@ -67,7 +78,7 @@ namespace q3k
         __device__ __forceinline__ void find_bin(const uint32_t *hist, uint32_t k, uint32_t *bin_out,
                                                  uint32_t *rank_out)
         {
-            const int lane = threadIdx.x % kWave;
+            const int lane = own_thread() % kWave;
             const int top = 255 - 4 * lane;
             uint32_t c[4];
 #pragma unroll
@@ -104,7 +115,7 @@ namespace q3k
         template <typename KeyAt>
         __device__ uint32_t block_kth(KeyAt key_at, int n, uint32_t k, uint32_t *hist, uint32_t *sel)
         {
-            const int tid = threadIdx.x;
+            const int tid = own_thread();
             if (tid < 256)
                 hist[tid] = 0u;
             __syncthreads();
@@ -407,7 +418,12 @@ namespace q3k
         // for both steps.  bf16 bits as signed 16-bit integers are in value order
         // among positive values and sort every negative one below, so with a
         // positive bound the packed-integer maximum does a dword pair in one
-        // instruction; a row whose bound is not positive is read again by
+        // instruction.  A row whose bound is not positive has fewer than k groups (or
+        // threads) with a positive value: by the unsigned minimum, under which the
+        // positive values come first and the negative ones in value order after them,
+        // it is bounded once more from the registers (rows of log-probabilities, 1 / 64 /
+        // 256 x 151936 at k = 20: 10.6 / 11.8 / 19.1 us; 20.8 / 22.1 / 108 when they were read
+        // again, twice).  Only a row too short for that is read again, by
         // select_reading.  Non-finite: the signed maximum reaches +inf's bits or the
         // unsigned maximum -inf's.
         //
@@ -423,9 +439,9 @@ namespace q3k
         // columns.  An append a column, 160 in line, made the code 16500 lines and its
         // fetching took as long as the read.
         //
-        // 64 rows of 151936: 9.9 us at k = 20, 12.1 at k = 150, 14.8 at k = 600 (10.7,
+        // 64 rows of 151936: 10.0 us at k = 20, 12.2 at k = 150, 15.0 at k = 600 (10.7,
         // 15.2 and 19.4 with an append a column; 15.5 and 18.8 as slices and merge at k = 20
-        // and 150); 256 rows of 151669: 17.1 and 19.1 (17.7 and 21.9; 29.7 and 31.6).
+        // and 150); 256 rows of 151669: 17.2 at k = 20 (17.7; 29.7).
         // Listing by wave segments (readlane a vector) measured 14.3 and 19.7.
         constexpr int kRegVecs = 20;
         constexpr int64_t kRegColumns = int64_t{8} * kRegVecs * kSelBlock;
@@ -450,23 +466,38 @@ namespace q3k
             return lo > hi ? lo : hi;
         }
         __device__ __forceinline__ int32_t max_i32(int32_t a, int32_t b) { return a > b ? a : b; }
-
-        // The largest T > 0 that at least k of the wave's SLOTS values a lane reach,
-        // i.e. their k-th largest (positive 15-bit values), or 0: there are fewer
-        // than k positive ones.
-        template <int SLOTS>
-        __device__ __forceinline__ int32_t wave_kth(const int32_t (&val)[SLOTS], uint32_t k)
+        __device__ __forceinline__ uint32_t min_u16x2(uint32_t a, uint32_t b)
         {
-            int32_t t = 0;
+            return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+        }
+        // the smaller half
+        __device__ __forceinline__ uint32_t low_u16(uint32_t m) { return (m & 0xffffu) < (m >> 16) ? m & 0xffffu : m >> 16; }
+        // bf16 bits as a signed integer in value order, -0 (-1) next below +0
+        __device__ __forceinline__ int32_t value_order(uint32_t bits)
+        {
+            return (bits & 0x8000u) != 0u ? static_cast<int16_t>(bits ^ 0x7fffu) : static_cast<int32_t>(bits);
+        }
+
+        // The largest T above low that at least k of the wave's SLOTS 16-bit values a
+        // lane reach, i.e. their k-th largest, or low: fewer than k lie above it.  low is 0
+        // (the values searched are positive) or kLowest.
+        constexpr int32_t kLowest = -0x8000;
+        template <int SLOTS>
+        __device__ __forceinline__ int32_t wave_kth(const int32_t (&val)[SLOTS], uint32_t k, int32_t low)
+        {
+            auto reach = [&](int32_t cand) __attribute__((always_inline)) {
+                uint32_t n = 0;
+#pragma unroll
+                for (int i = 0; i < SLOTS; ++i)
+                    n += static_cast<uint32_t>(__popcll(__ballot(val[i] >= cand)));
+                return n >= k;
+            };
+            int32_t t = low < 0 && reach(0) ? 0 : low;
 #pragma unroll
             for (int bit = 14; bit >= 0; --bit)
             {
                 const int32_t cand = t | (1 << bit);
-                uint32_t reach = 0;
-#pragma unroll
-                for (int i = 0; i < SLOTS; ++i)
-                    reach += static_cast<uint32_t>(__popcll(__ballot(val[i] >= cand)));
-                t = reach >= k ? cand : t;
+                t = reach(cand) ? cand : t;
             }
             return t;
         }
@@ -497,21 +528,25 @@ namespace q3k
         };
 
         // The list entries at or above its k-th largest (k <= nl <= SLOTS waves'
-        // worth of lanes): each wave finds it and writes its own 64 entries.
+        // worth of lanes; low as for wave_kth): each wave finds it and writes its own 64
+        // entries.
         template <int SLOTS>
-        __device__ __forceinline__ void emit_ranked(SelShared &sh, uint32_t nl, uint32_t k, int64_t row, const CandOut &co)
+        __device__ __forceinline__ void emit_ranked(SelShared &sh, uint32_t nl, uint32_t k, int64_t row, const CandOut &co,
+                                                    int32_t low)
         {
-            const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+            const uint32_t tid = own_thread();
+            const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
             if (wave * kWave >= nl)
                 return;
             int32_t val[SLOTS];
 #pragma unroll
             for (int i = 0; i < SLOTS; ++i)
-                val[i] = i * kWave + lane < nl ? static_cast<int32_t>(sh.list_bits[i * kWave + lane]) : 0;
-            const int32_t kth = wave_kth<SLOTS>(val, k);
-            const bool in = threadIdx.x < nl;
-            const int32_t mine = in ? static_cast<int32_t>(sh.list_bits[threadIdx.x]) : 0;
-            const bool take = in && mine >= kth;
+                val[i] = i * kWave + lane < nl ? value_order(sh.list_bits[i * kWave + lane]) : low;
+            int32_t kth = wave_kth<SLOTS>(val, k, low);
+            kth = kth == 0 ? -1 : kth; // +0 takes -0 too
+            const bool in = tid < nl;
+            const uint32_t mine = in ? sh.list_bits[tid] : 0u;
+            const bool take = in && value_order(mine) >= kth;
             const uint64_t ballot = __ballot(take);
             uint32_t base = 0;
             if (lane == 0)
@@ -521,7 +556,7 @@ namespace q3k
                                                                    __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(ballot), 0u));
             if (take && slot < static_cast<uint32_t>(co.cap))
             {
-                co.cand_index[row * co.cap + slot] = sh.list_index[threadIdx.x];
+                co.cand_index[row * co.cap + slot] = sh.list_index[tid];
                 co.cand_logit[row * co.cap + slot] = static_cast<uint16_t>(mine);
             }
         }
@@ -549,16 +584,16 @@ namespace q3k
         {
             __shared__ SelShared sh;
             __shared__ HitVectors hits;
-            const int tid = threadIdx.x, lane = tid % kWave;
             for (int64_t row = blockIdx.x; row < rows; row += gridDim.x)
             {
+                const int tid = own_thread(), lane = tid % kWave;
                 const uint16_t *r = x + row * stride;
                 // the 16-byte aligned middle [first, first + 8 nv), up to seven columns on either side
                 const int32_t odd = static_cast<int32_t>((reinterpret_cast<uintptr_t>(r) / 2) % 8);
                 const int32_t first = odd == 0 ? 0 : 8 - odd < n ? 8 - odd : n;
                 const int32_t nv = (n - first) / 8;
                 const Vec8 *rv = reinterpret_cast<const Vec8 *>(r + first);
-                constexpr uint32_t kNone = 0x80008000u; // below every value, finite
+                constexpr uint32_t kNone = 0xff7fff7fu; // an empty place: the lowest finite value
                 Vec8 v[kRegVecs];
 #pragma unroll
                 for (int u = 0; u < kRegVecs; ++u)
@@ -568,8 +603,9 @@ namespace q3k
                         v[u] = load8<false>(rv + tid + u * kSelBlock);
                 }
                 const int32_t side = tid < 8 ? tid : first + 8 * nv + tid - 8;
+                const bool has_side = tid < 16 && (tid < 8 ? side < first : side < n);
                 uint32_t side_bits = kNone & 0xffffu;
-                if (tid < 16 && (tid < 8 ? side < first : side < n))
+                if (has_side)
                     side_bits = r[side];
                 if (tid == 0)
                 {
@@ -589,26 +625,24 @@ namespace q3k
                         mi = max_i16x2(mi, v[u].d[j]);
                         mu = max_u16x2(mu, v[u].d[j]);
                     }
-                const int32_t tmax = top_i16(mi);
+                int32_t tmax = top_i16(mi);
                 if (tmax >= 0x7f80 || (mu >> 16) >= 0xff80u || (mu & 0xffffu) >= 0xff80u)
                     atomicOr(&sh.bad, 1u);
-                if (k <= kGroupK)
-                {
-                    int32_t g = tmax;
-                    g = max_i32(g, static_cast<int32_t>(dpp_u<kDppQuadXor1>(static_cast<uint32_t>(g))));
-                    g = max_i32(g, static_cast<int32_t>(dpp_u<kDppQuadXor2>(static_cast<uint32_t>(g))));
-                    if (lane % 4 == 0)
-                        sh.group_max[tid / 4] = g;
-                }
-                else
-                    sh.thread_max[tid] = tmax > 0 ? static_cast<uint32_t>(tmax) : 0u;
-                __syncthreads();
                 // 2. the bound, and the list of logits at or above it
-                bool exact = false;
-                const bool bad = sh.bad != 0u;
-                if (!bad)
-                {
-                    int32_t bound;
+                auto share_maxima = [&](int32_t low) __attribute__((always_inline)) {
+                    if (k <= kGroupK)
+                    {
+                        int32_t g = tmax;
+                        g = max_i32(g, static_cast<int32_t>(dpp_u<kDppQuadXor1>(static_cast<uint32_t>(g))));
+                        g = max_i32(g, static_cast<int32_t>(dpp_u<kDppQuadXor2>(static_cast<uint32_t>(g))));
+                        if (lane % 4 == 0)
+                            sh.group_max[tid / 4] = g;
+                    }
+                    else
+                        sh.thread_max[tid] = tmax > low ? static_cast<uint32_t>(tmax - low) : 0u;
+                    __syncthreads();
+                };
+                auto find_bound = [&](int32_t low) __attribute__((always_inline)) {
                     if (k <= kGroupK)
                     {
                         // one wave: side by side, the 16 waves' steps held each other up
@@ -618,82 +652,122 @@ namespace q3k
 #pragma unroll
                             for (int i = 0; i < 4; ++i)
                                 g[i] = sh.group_max[i * kWave + lane];
-                            const int32_t t = wave_kth<4>(g, k);
+                            const int32_t t = wave_kth<4>(g, k, low);
                             if (lane == 0)
                                 sh.bound = static_cast<uint32_t>(t);
                         }
                         __syncthreads();
-                        bound = static_cast<int32_t>(sh.bound);
+                        return static_cast<int32_t>(sh.bound);
                     }
-                    else
-                        bound = static_cast<int32_t>(
-                            block_kth([&](int i) { return sh.thread_max[i]; }, kSelBlock, k, sh.hist, sh.sel));
-                    if (bound > 0)
+                    return static_cast<int32_t>(
+                               block_kth([&](int i) { return sh.thread_max[i]; }, kSelBlock, k, sh.hist, sh.sel)) +
+                           low;
+                };
+                share_maxima(0);
+                bool exact = false;
+                const bool bad = sh.bad != 0u;
+                int32_t bound = 0, low = 0;
+                if (!bad)
+                    bound = find_bound(0);
+                if (__builtin_expect(!bad && bound <= 0, 0))
+                {
+                    // by the unsigned minima, a positive value counted as -0
+                    uint32_t mn = side_bits | (kNone & 0xffff0000u);
+#pragma unroll
+                    for (int u = 0; u < kRegVecs; ++u)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            mn = min_u16x2(mn, v[u].d[j]);
+                    mn = low_u16(mn);
+                    tmax = value_order(mn < 0x8000u ? 0x8000u : mn);
+                    low = kLowest;
+                    share_maxima(low);
+                    bound = find_bound(low);
+                }
+                if (bound > value_order(kNone & 0xffffu) && (low < 0 || bound > 0))
+                {
+                    // at or above the bound: the bits, or with a negative one the bits ^ 0x7fff, as signed integers
+                    const uint32_t flip = low < 0 ? 0x7fffu : 0u;
+                    auto reaches = [&](uint32_t bits) __attribute__((always_inline)) {
+                        return static_cast<int16_t>(bits ^ flip) >= bound;
+                    };
+                    auto append = [&](uint32_t bits, int32_t index) __attribute__((always_inline)) {
+                        const uint32_t pos = atomicAdd(&sh.listed, 1u);
+                        if (pos < static_cast<uint32_t>(kCandMax))
+                        {
+                            sh.list_bits[pos] = bits;
+                            sh.list_index[pos] = index;
+                        }
+                    };
+                    // vectors that hold a logit at or above the bound
+                    uint32_t mask = 0;
+                    if (tmax >= bound)
                     {
-                        auto append = [&](uint32_t bits, int32_t index) __attribute__((always_inline)) {
-                            const uint32_t pos = atomicAdd(&sh.listed, 1u);
-                            if (pos < static_cast<uint32_t>(kCandMax))
+                        if (__builtin_expect(low < 0, 0))
+                        {
+#pragma unroll
+                            for (int u = 0; u < kRegVecs; ++u)
                             {
-                                sh.list_bits[pos] = bits;
-                                sh.list_index[pos] = index;
+                                const uint32_t m = min_u16x2(min_u16x2(v[u].d[0], v[u].d[1]), min_u16x2(v[u].d[2], v[u].d[3]));
+                                mask |= reaches(low_u16(m)) ? 1u << u : 0u;
                             }
-                        };
-                        // vectors that hold a logit at or above the bound
-                        uint32_t mask = 0;
-                        if (tmax >= bound)
+                        }
+                        else
+                        {
 #pragma unroll
                             for (int u = 0; u < kRegVecs; ++u)
                             {
                                 const uint32_t m = max_i16x2(max_i16x2(v[u].d[0], v[u].d[1]), max_i16x2(v[u].d[2], v[u].d[3]));
                                 mask |= top_i16(m) >= bound ? 1u << u : 0u;
                             }
-                        uint32_t total;
-                        uint32_t pos = wave_prefix(static_cast<uint32_t>(__popc(mask)), &total);
-                        uint32_t base = 0;
-                        if (lane == 0 && total != 0)
-                            base = atomicAdd(&hits.count, total);
-                        pos += __builtin_amdgcn_readfirstlane(base);
+                        }
+                    }
+                    uint32_t total;
+                    uint32_t pos = wave_prefix(static_cast<uint32_t>(__popc(mask)), &total);
+                    uint32_t base = 0;
+                    if (lane == 0 && total != 0)
+                        base = atomicAdd(&hits.count, total);
+                    pos += __builtin_amdgcn_readfirstlane(base);
 #pragma unroll
-                        for (int u = 0; u < kRegVecs; ++u)
-                            if ((mask >> u & 1u) != 0u)
-                            {
-                                if (pos < static_cast<uint32_t>(kCandMax))
-                                {
-                                    hits.vec[pos] = v[u];
-                                    hits.column[pos] = first + 8 * (tid + u * kSelBlock);
-                                }
-                                ++pos;
-                            }
-                        if (static_cast<int16_t>(side_bits) >= bound)
-                            append(side_bits, side);
-                        __syncthreads();
-                        // each of them has one at least: past kCandMax the list would overflow
-                        const uint32_t nh = hits.count;
-                        if (nh > static_cast<uint32_t>(kCandMax))
+                    for (int u = 0; u < kRegVecs; ++u)
+                        if ((mask >> u & 1u) != 0u)
                         {
-                            if (tid == 0)
-                                sh.listed = kCandMax + 1;
+                            if (pos < static_cast<uint32_t>(kCandMax))
+                            {
+                                hits.vec[pos] = v[u];
+                                hits.column[pos] = first + 8 * (tid + u * kSelBlock);
+                            }
+                            ++pos;
                         }
+                    if (reaches(side_bits))
+                        append(side_bits, side);
+                    __syncthreads();
+                    // each of them has one at least: past kCandMax the list would overflow
+                    const uint32_t nh = hits.count;
+                    if (nh > static_cast<uint32_t>(kCandMax))
+                    {
+                        if (tid == 0)
+                            sh.listed = kCandMax + 1;
+                    }
+                    else
+                        for (uint32_t i = tid; i < 8 * nh; i += kSelBlock)
+                        {
+                            const uint32_t bits = reinterpret_cast<const uint16_t *>(hits.vec)[i];
+                            if (reaches(bits))
+                                append(bits, hits.column[i / 8] + static_cast<int32_t>(i % 8));
+                        }
+                    __syncthreads();
+                    const uint32_t nl = sh.listed;
+                    if (nl <= static_cast<uint32_t>(kCandMax))
+                    {
+                        // 3. the exact top k of the list (k <= nl: the bound holds)
+                        if (nl <= 2 * kWave)
+                            emit_ranked<2>(sh, nl, k, row, co, low);
+                        else if (nl <= kRankList)
+                            emit_ranked<kRankSlots>(sh, nl, k, row, co, low);
                         else
-                            for (uint32_t i = tid; i < 8 * nh; i += kSelBlock)
-                            {
-                                const uint32_t bits = reinterpret_cast<const uint16_t *>(hits.vec)[i];
-                                if (static_cast<int16_t>(bits) >= bound)
-                                    append(bits, hits.column[i / 8] + static_cast<int32_t>(i % 8));
-                            }
-                        __syncthreads();
-                        const uint32_t nl = sh.listed;
-                        if (nl <= static_cast<uint32_t>(kCandMax))
-                        {
-                            // 3. the exact top k of the list (k <= nl: the bound holds)
-                            if (nl <= 2 * kWave)
-                                emit_ranked<2>(sh, nl, k, row, co);
-                            else if (nl <= kRankList)
-                                emit_ranked<kRankSlots>(sh, nl, k, row, co);
-                            else
-                                emit_list(sh, nl, k, row, co);
-                            exact = true;
-                        }
+                            emit_list(sh, nl, k, row, co);
+                        exact = true;
                     }
                 }
                 __syncthreads();

@@ -163,3 +163,60 @@ def test_topk_row_edges(q3k, hip, oracle, synth, n, ks, pad, offset):
                 got = ids[r, :want.size]
                 check_exact(f"{name} row {r} ids", np.sort(got), np.sort(want))
                 check_exact(f"{name} row {r} logits", vals[r, :want.size], x[r, got])
+
+
+def _few_positive(synth, n, k):
+    """Rows with fewer than k positive logits: none; some; the k-th among zeros of both signs, among a few tied
+    negatives; zeros of both signs and nothing above."""
+    neg = synth.normal_bf16(193, n, (5, n), std=3.0) | 0x8000
+    rng = np.random.default_rng(n + k)
+    at = [rng.permutation(n) for _ in range(5)]
+    some = k // 2
+    x = neg
+    x[1, at[1][:some]] = 0x4000 + rng.integers(0, 200, some)
+    x[2, at[2][:some]] = 0x3f80
+    zeros = at[2][some:some + k]
+    x[2, zeros] = np.where(rng.integers(0, 2, zeros.size) == 1, 0x8000, 0)
+    x[3] = synth.f32_to_bf16(np.linspace(-4.0, -1.0, 64).astype(np.float32))[rng.integers(0, 64, n)]
+    x[4, at[4][: 2 * k]] = 0x8000
+    x[4, at[4][:some]] = 0x0000
+    return x
+
+
+@pytest.mark.parametrize("n,ks", [(9, (2, 9)), (900, (20, 120)), (3000, (20, 150)), (8193, (20, 192, 193, 1024)),
+                                  (151936, (1, 20, 64, 150, 600, 1024)), (163840, (20, 1000))])
+@pytest.mark.parametrize("pad,offset", [(0, 0), (3, 6)])
+def test_topk_few_positive_values(q3k, hip, oracle, synth, n, ks, pad, offset):
+    for k in ks:
+        x = np.concatenate([_few_positive(synth, n, k), np.full((5, pad), 0x42c8, np.uint16)], axis=1)
+        rows, stride, cap = 5, n + pad, 4096
+        name = f"topk few positive n={n} stride={stride} offset={offset} k={k}"
+        announce(name)
+        X = Guarded(hip, x, offset=offset)
+        C, F = Guarded(hip, nbytes=rows * 4), Guarded(hip, nbytes=rows * 4)
+        I, V = Guarded(hip, nbytes=rows * cap * 4), Guarded(hip, nbytes=rows * cap * 2)
+        q3k.topk_candidates(X, rows, stride, n, k, cap, C, I, V, F)
+        hip.synchronize()
+        assert all(b.guards_intact() for b in (C, F, I, V))
+        counts, flags = C.get(np.int32, (rows,)), F.get(np.int32, (rows,))
+        ids, vals = I.get(np.int32, (rows, cap)), V.get(np.uint16, (rows, cap))
+        for r in range(rows):
+            want = oracle.topk_set(x[r, :n], k)
+            assert flags[r] == 0 and counts[r] == want.size, (name, r, counts[r], want.size)
+            if want.size <= cap:
+                got = ids[r, :want.size]
+                check_exact(f"{name} row {r} ids", np.sort(got), np.sort(want))
+                check_exact(f"{name} row {r} logits", vals[r, :want.size], x[r, got])
+
+
+def test_topk_time_without_positive_values(q3k, hip, synth):
+    """As for argmax: 1.2 times here, 2.2 times when such rows were read again twice."""
+    rows, n, k, cap = 64, 151936, 20, 256
+    stream, us = hip.Stream(), {}
+    C, F, I, V = (hip.DeviceBuffer(rows * b) for b in (4, 4, 4 * cap, 2 * cap))
+    for kind, x in _kinds(synth, rows, n).items():
+        X = hip.DeviceBuffer.from_array(x)
+        us[kind] = _us(hip, stream, lambda: q3k.topk_candidates(X, rows, n, n, k, cap, C, I, V, F, stream))
+        X.free()
+    print(f"[time] topk {rows} x {n}, k = {k}: {us}", flush=True)
+    assert max(us["negative"], us["shifted"]) < 1.6 * us["ordinary"], us
