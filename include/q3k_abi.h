@@ -238,8 +238,9 @@ Q3K_API int q3k_argmax_bf16(const uint16_t *x, int32_t *out, int64_t rows,
 
 /*
  * Workspace bytes q3k_argmax_bf16 would use to slice these rows (0: it does
- * not slice).  No counterpart in the reference (its kernel is one block per
- * row).
+ * not slice: enough rows, or rows that one block each searches sooner, such as
+ * those of a Qwen3 vocabulary).  No counterpart in the reference (its kernel is
+ * one block per row).
  */
 Q3K_API int64_t q3k_argmax_workspace_bytes(int64_t rows, int64_t search_size);
 
@@ -250,10 +251,12 @@ Q3K_API int64_t q3k_argmax_workspace_bytes(int64_t rows, int64_t search_size);
  * each GPU it runs on until the process ends, instead of a caller
  * workspace.  Every input fits it (slicing needs fewer than 8 KiB); a plan
  * needing more returns Q3K_ERR_INVALID_ARGUMENT.  The call itself allocates
- * nothing.  Calls on one GPU share that array, so calls that overlap on one
- * GPU race.  The first call on each GPU looks up the array's device address
- * (a host-side query under a lock); make that call before capturing the
- * entry point into a HIP graph.  No counterpart in the reference.
+ * nothing.  Calls on one GPU whose rows are sliced (those that
+ * q3k_argmax_workspace_bytes gives a size for) share that array, so such calls
+ * that overlap on one GPU race.  The first of them on each GPU looks up the
+ * array's device address (a host-side query under a lock); make that call
+ * before capturing the entry point, with such rows, into a HIP graph.  No
+ * counterpart in the reference.
  */
 Q3K_API int q3k_argmax_bf16_noalloc(const uint16_t *x, int32_t *out, int64_t rows,
                   int64_t row_stride, int64_t search_size,
@@ -281,7 +284,8 @@ Q3K_API int q3k_topk_candidates_bf16(const uint16_t *logits, int64_t rows,
 
 /*
  * Workspace bytes q3k_topk_candidates_bf16 would use to cut these rows into
- * slices searched by separate blocks (0: it does not); the workspace (16-byte
+ * slices searched by separate blocks (0: it does not, e.g. for rows of a Qwen3
+ * vocabulary, which a block holds in its registers); the workspace (16-byte
  * aligned device memory, may be NULL) changes the speed, not the result, and
  * calls that share one must not overlap.  No counterpart in the reference
  * (its selection runs on the host).

@@ -321,7 +321,7 @@ namespace q3k
         SlicePlan plan_slices(int64_t rows, int64_t n)
         {
             SlicePlan p;
-            if (rows <= 0 || rows >= kTargetBlocks)
+            if (rows <= 0 || rows >= kTargetBlocks || n <= kWholeRowColumns)
                 return p;
             int64_t want = (kTargetBlocks + rows - 1) / rows;
             if (want > n / kMinSlice)
@@ -375,7 +375,7 @@ namespace q3k
         int launch_argmax(const uint16_t *x, int32_t *out, int64_t rows, int64_t row_stride, int64_t search_size,
                           const SlicePlan &plan, uint64_t *part, hipStream_t s)
         {
-            if (plan.slices > 1 && part != nullptr && search_size > kWholeRowColumns)
+            if (plan.slices > 1 && part != nullptr)
             {
                 argmax_slice_kernel<<<dim3(static_cast<unsigned>(rows * plan.slices)), dim3(kArgmaxBlock), 0, s>>>(
                     x, part, row_stride, search_size, plan.slices, plan.slice_len);

@@ -908,8 +908,9 @@ namespace q3k
             }
         }
 
-        // Rows are cut into slices when fewer than kTargetBlocks blocks would
-        // run (and k <= kSelBlock); a slice keeps at least kMinSlice logits.
+        // Rows that topk_row_kernel does not take are cut into slices when fewer than
+        // kTargetBlocks blocks would run (and k <= kSelBlock); a slice keeps at least
+        // kMinSlice logits.
         constexpr int64_t kTargetBlocks = 512;
         constexpr int64_t kMinSlice = 8 * kSelBlock;
         constexpr int kMaxSlices = kWave;
@@ -921,10 +922,12 @@ namespace q3k
             int64_t bytes = 0;
         };
 
+        bool fits_registers(int64_t n, int32_t k) { return n <= kRegColumns && k <= kSelBlock; }
+
         SlicePlan plan_slices(int64_t rows, int64_t n, int32_t k)
         {
             SlicePlan p;
-            if (rows <= 0 || rows >= kTargetBlocks || k <= 0 || k > kSelBlock)
+            if (rows <= 0 || rows >= kTargetBlocks || k <= 0 || k > kSelBlock || fits_registers(n, k))
                 return p;
             int64_t want = (kTargetBlocks + rows - 1) / rows;
             if (want > n / kMinSlice)
@@ -976,7 +979,7 @@ extern "C" int q3k_topk_candidates_bf16(const uint16_t *logits, int64_t rows, in
     const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const CandOut co{cap, cand_index, cand_logit};
     const unsigned grid = static_cast<unsigned>(rows < 65535 ? rows : 65535);
-    if (search_size <= kRegColumns && k <= kSelBlock)
+    if (fits_registers(search_size, k))
     {
         topk_row_kernel<<<dim3(grid), dim3(kSelBlock), 0, s>>>(logits, rows, row_stride, static_cast<int32_t>(search_size),
                                                                 static_cast<uint32_t>(k), co, count, nonfinite);

@@ -216,20 +216,25 @@ def test_argmax_argument_errors(q3k):
 
 
 def test_selection_workspace_plans(q3k):
-    """Argmax and top-k ask for a workspace only when the rows are too few to fill the GPU (and, for top-k, k fits
-    the bound step); the size covers one 8-byte key per slice, or a header and a list per slice."""
-    V = 151936
-    ws = q3k.argmax_workspace_bytes(64, V)
+    """Argmax and top-k ask for a workspace only when the rows are too few to fill the GPU and longer than one block
+    searches or holds (and, for top-k, k fits the bound step); the size covers one 8-byte key per slice, or a header
+    and a list per slice."""
+    V, L = 151936, 300000
+    ws = q3k.argmax_workspace_bytes(64, L)
     assert ws > 0 and ws % (64 * 8) == 0 and 2 <= ws // (64 * 8) <= 64
-    assert q3k.argmax_workspace_bytes(1, V) > 0
-    assert q3k.argmax_workspace_bytes(512, V) == 0        # enough rows: one block per row
+    assert q3k.argmax_workspace_bytes(1, L) > 0
+    assert q3k.argmax_workspace_bytes(512, L) == 0        # enough rows: one block per row
+    for rows in (1, 64, 511):
+        assert q3k.argmax_workspace_bytes(rows, V) == 0   # a Qwen3 vocabulary: one launch, nothing to hold
+        assert q3k.topk_workspace_bytes(rows, V, 20) == 0
     assert q3k.argmax_workspace_bytes(4, 10000) == 0      # a row too short to cut
-    assert q3k.argmax_workspace_bytes(0, V) == 0
-    tk = q3k.topk_workspace_bytes(64, V, 20)
+    assert q3k.argmax_workspace_bytes(0, L) == 0
+    tk = q3k.topk_workspace_bytes(64, L, 20)
     assert tk > 0 and tk % 64 == 0
-    assert q3k.topk_workspace_bytes(64, V, 1024) == tk    # the size does not depend on k up to the thread count
-    assert q3k.topk_workspace_bytes(64, V, 1025) == 0     # k above the thread count: whole-row select
-    assert q3k.topk_workspace_bytes(600, V, 20) == 0
+    assert q3k.topk_workspace_bytes(64, L, 1024) == tk    # the size does not depend on k up to the thread count
+    assert q3k.topk_workspace_bytes(64, L, 1025) == 0     # k above the thread count: whole-row select
+    assert q3k.topk_workspace_bytes(600, L, 20) == 0
+    assert q3k.topk_workspace_bytes(64, 163840, 20) == 0 and q3k.topk_workspace_bytes(64, 163841, 20) > 0
     IA = q3k.Q3K_ERR_INVALID_ARGUMENT
     fake = 256
     msg = _expect(q3k.topk_candidates, ValueError, IA, fake, 2, 100, 100, 5, 8, fake, fake, fake, fake, None, fake,

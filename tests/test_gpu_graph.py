@@ -24,7 +24,7 @@ def test_graph_replay_decode_step(q3k, hip, synth):
     replays, each bit-identical to the eager launches."""
     announce("graph replay: decode step")
     B, H, I, Hq, Hkv, P = 64, 4096, 12288, 32, 8, 4096
-    Bd, L, V = 4, 700, 20000   # attention over Bd sequences of L cached keys; argmax over [Bd, V]
+    Bd, L, V = 4, 700, 270000   # attention over Bd sequences of L cached keys; argmax over [Bd, V]
     rng = np.random.default_rng(5)
     arrays = {
         "h1": synth.normal_bf16(31, 1, (B, H)), "d1": synth.normal_bf16(31, 2, (B, H)),

@@ -2,7 +2,7 @@
 slice results live in a fixed device array held by the library), against
 q3k_argmax_bf16 with a caller workspace and against the oracle, bit for bit:
 several calls in a row on one GPU, each after the first with a smaller input
-(sliced rows, one long row, then enough rows to skip slicing), plus the
+(sliced rows, then rows searched whole), plus the
 ties-across-slices, NaN and -0 rows of the workspace form's tests.  The
 device's free memory is the same before and after each call."""
 import numpy as np
@@ -13,7 +13,7 @@ from gpu_util import Guarded, announce, check_exact
 pytestmark = pytest.mark.gpu
 
 # rows, columns: the first call is the largest; later ones are smaller
-CALLS = [(64, 151936), (9, 40000), (1, 151936), (2, 8192), (600, 2048)]
+CALLS = [(64, 300000), (9, 262145), (1, 300001), (64, 151936), (9, 40000), (1, 151936), (2, 8192), (600, 2048)]
 
 
 def _logits(synth, i, rows, N):
@@ -73,8 +73,8 @@ def test_noalloc_argmax_captured_in_graph(q3k, hip, oracle, synth):
     the GPU (made eagerly, before the capture) resolves the array's device address; the captured call then
     replays three times, each replay preceded by an eager call on other logits that overwrites the same array,
     and every replay's result equals the oracle's."""
-    rows, N = 9, 40000
-    rows2, N2 = 2, 151936
+    rows, N = 9, 270000
+    rows2, N2 = 2, 400000
     assert q3k.argmax_workspace_bytes(rows, N) > 0 and q3k.argmax_workspace_bytes(rows2, N2) > 0, "sliced shapes"
     announce(f"argmax noalloc in a graph: rows={rows} N={N}, eager rows={rows2} N={N2} between replays")
     x, x2 = _logits(synth, 10, rows, N), _logits(synth, 11, rows2, N2)
