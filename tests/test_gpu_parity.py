@@ -825,14 +825,21 @@ def _split_cases(cases, plan):
 
 
 ARGMAX_CASES = [(2, 513, 0, 0), (37, 1000, 0, 0), (64, 151936, 0, 0), (1, 151936, 151669, 0), (5, 1003, 0, 2),
-                (3, 4096, 77, 2), (700, 64, 0, 0), (9, 40000, 0, 0), (2, 70001, 0, 2)]
-ARGMAX_TIE_CASES = [(1, 151936, 3), (7, 50000, 2), (33, 20000, 5), (2, 151936, 256)]
+                (3, 4096, 77, 2), (700, 64, 0, 0), (9, 40000, 0, 0), (2, 70001, 0, 2),
+                # rows long enough to be cut into slices
+                (64, 262145, 0, 0), (1, 300001, 300000, 0), (9, 270000, 0, 0), (8, 400001, 0, 2)]
+ARGMAX_TIE_CASES = [(1, 151936, 3), (7, 50000, 2), (33, 20000, 5), (2, 151936, 256),
+                    (1, 600000, 3), (7, 270000, 2), (33, 262145, 5), (2, 300000, 256)]
 TOPK_CASES = [(8, 151936, 0, 20), (4, 151936, 151669, 1), (2, 151936, 0, 1024), (3, 5000, 0, 64), (2, 513, 500, 3),
               (2, 600, 0, 100),      # fewer than k threads hold logits: all listed
               (2, 20000, 0, 1500),   # k above the thread count: whole-row select
-              (1, 151936, 151669, 50), (6, 40000, 0, 700)]
+              (1, 151936, 151669, 50), (6, 40000, 0, 700),
+              # rows too long for a block's registers: cut into slices
+              (8, 163848, 0, 20), (4, 200000, 163841, 1), (2, 400000, 0, 1024), (1, 300001, 300000, 50),
+              (6, 180000, 0, 700), (300, 170000, 0, 20)]
 TOPK_TIE_CASES = [(1, 151936, 50, 16), (3, 50000, 7, 4), (17, 16385, 1, 64), (2, 151936, 300, 2048),
-                  (5, 40001, 700, 32)]
+                  (5, 40001, 700, 32), (1, 200000, 50, 16), (3, 170000, 7, 4), (17, 163841, 1, 64),
+                  (2, 300000, 300, 4096), (5, 180001, 700, 32)]
 
 
 @pytest.mark.parametrize("rows,N,search,offset,split", _split_cases(
