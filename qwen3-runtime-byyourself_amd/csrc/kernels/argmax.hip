@@ -9,12 +9,11 @@
 // unsigned max.  One block of 1024 threads per row (rows strided over the
 // grid): 128-bit loads of the row's aligned middle, a thread's maximum from the
 // bits as packed 16-bit integers (a key per thread, not per element), wave and
-// block maxima by DPP and through LDS.  When rows are longer than
-// kWholeRowColumns, too few to fill the GPU, and the caller gives a workspace,
-// each row is cut into slices of whole 8-column
-// vectors: one block per (row, slice) writes the slice's best key, and a
-// second kernel takes the maximum over the slices of each row (the key
-// order is total, so the result is the same).
+// block maxima by DPP and through LDS.  When rows are long (kWholeRowColumns),
+// too few to fill the GPU, and the caller gives a workspace, each row is cut
+// into slices of whole 8-column vectors: one block per (row, slice) writes the
+// slice's best key, and a second kernel takes the maximum over the slices of
+// each row (the key order is total, so the result is the same).
 #include "q3k_common.hpp"
 
 #include <mutex>
@@ -305,11 +304,17 @@ namespace q3k
         constexpr int64_t kMinSlice = 8 * kArgmaxBlock;
         constexpr int kMaxSlices = kWave;
 
-        // Rows up to this long are searched whole, a block each: one launch.  64 x
-        // 151936 took 6.3 us whole and 7.6 as slices and merge, 1 x 151936 4.7 and
-        // 4.7 (the second launch costs the host another 1.3), 256 x 151669 13.6 and
-        // 15.6.
+        // Rows up to kWholeRowColumns long are searched whole, a block each: one launch.
+        // Of at most kFewRows rows that holds up to kWholeFewRowsColumns only: their
+        // slices, on CUs that would idle, then take less than the second launch.  (Whole
+        // / slices in us, stream: 1 row of 200000 5.3 / 5.5, 230000 5.9 / 5.5, 262144 6.4 /
+        // 5.5; 8 of 200000 5.6 / 5.6, 262144 6.7 / 5.4; 32 of 200000 6.6 / 6.9, 230000 7.7 /
+        // 6.9.  40 of 230000 7.8 / 8.4, 262144 8.3 / 8.7, 300000 9.4 / 9.0; 64 of 151936 6.2 /
+        // 7.5, 262144 9.1 / 9.2, 300000 10.0 / 9.8; 256 of 151936 13.2 / 15.1, 262144 27.6 /
+        // 27.4.)
         constexpr int64_t kWholeRowColumns = int64_t{1} << 18;
+        constexpr int64_t kWholeFewRowsColumns = 5 * 8 * kUnroll * kArgmaxBlock; // 204800: five loads a thread
+        constexpr int64_t kFewRows = 32;
 
         struct SlicePlan
         {
@@ -321,7 +326,7 @@ namespace q3k
         SlicePlan plan_slices(int64_t rows, int64_t n)
         {
             SlicePlan p;
-            if (rows <= 0 || rows >= kTargetBlocks || n <= kWholeRowColumns)
+            if (rows <= 0 || rows >= kTargetBlocks || n <= (rows <= kFewRows ? kWholeFewRowsColumns : kWholeRowColumns))
                 return p;
             int64_t want = (kTargetBlocks + rows - 1) / rows;
             if (want > n / kMinSlice)

@@ -227,6 +227,9 @@ def test_selection_workspace_plans(q3k):
     for rows in (1, 64, 511):
         assert q3k.argmax_workspace_bytes(rows, V) == 0   # a Qwen3 vocabulary: one launch, nothing to hold
         assert q3k.topk_workspace_bytes(rows, V, 20) == 0
+    # whole rows up to 204800 columns of at most 32 rows, up to 2^18 of more
+    for rows, longest in ((1, 204800), (32, 204800), (33, 2**18), (511, 2**18)):
+        assert q3k.argmax_workspace_bytes(rows, longest) == 0 and q3k.argmax_workspace_bytes(rows, longest + 1) > 0
     assert q3k.argmax_workspace_bytes(4, 10000) == 0      # a row too short to cut
     assert q3k.argmax_workspace_bytes(0, L) == 0
     tk = q3k.topk_workspace_bytes(64, L, 20)
