@@ -55,10 +55,9 @@ namespace qwen3
         class SmallBlockCache
         {
         public:
-            static constexpr std::size_t kMaxBlock = std::size_t{4} << 20;  // larger sizes are not cached
+            static constexpr std::size_t kMaxBlock = std::size_t{4} << 20;  // larger Buffers are not cached
+            static constexpr std::size_t kMaxWorkspace = std::size_t{16} << 20;  // nor larger workspaces
             static constexpr std::size_t kMaxKeptPerDevice = std::size_t{64} << 20;
-
-            static bool cached(std::size_t bytes) { return bytes <= kMaxBlock; }
 
             // Size class: the next power of two, at least 512 bytes.
             static std::size_t size_class(std::size_t bytes)
@@ -131,9 +130,10 @@ namespace qwen3
             return *cache;
         }
 
-        void *allocate_device(std::size_t bytes, int index)
+        // Blocks of up to `most` bytes come from the cache and go back to it.
+        void *allocate_device(std::size_t bytes, int index, std::size_t most = SmallBlockCache::kMaxBlock)
         {
-            const bool small = SmallBlockCache::cached(bytes) && block_cache_enabled();
+            const bool small = bytes <= most && block_cache_enabled();
             const std::size_t alloc = small ? SmallBlockCache::size_class(bytes) : bytes;
             if (small && t_fresh_blocks == 0)
                 if (void *p = block_cache().take(index, alloc))
@@ -146,11 +146,11 @@ namespace qwen3
             return p;
         }
 
-        void free_device(void *p, std::size_t bytes, int index) noexcept
+        void free_device(void *p, std::size_t bytes, int index, std::size_t most = SmallBlockCache::kMaxBlock) noexcept
         {
             try
             {
-                if (SmallBlockCache::cached(bytes) && block_cache_enabled() &&
+                if (bytes <= most && block_cache_enabled() &&
                     block_cache().keep(index, SmallBlockCache::size_class(bytes), p))
                     return;
             }
@@ -212,6 +212,17 @@ namespace qwen3
 
     detail::FreshDeviceBlocks::FreshDeviceBlocks() noexcept { ++t_fresh_blocks; }
     detail::FreshDeviceBlocks::~FreshDeviceBlocks() { --t_fresh_blocks; }
+
+    detail::DeviceWorkspace::DeviceWorkspace(std::size_t bytes, int device)
+        : data_(bytes > 0 ? allocate_device(bytes, device, SmallBlockCache::kMaxWorkspace) : nullptr), bytes_(bytes),
+          device_(device)
+    {
+    }
+    detail::DeviceWorkspace::~DeviceWorkspace()
+    {
+        if (data_ != nullptr)
+            free_device(data_, bytes_, device_, SmallBlockCache::kMaxWorkspace);
+    }
 
     std::uint64_t device_allocation_count() noexcept { return g_device_allocations.load(std::memory_order_relaxed); }
 

@@ -3,6 +3,8 @@
 // src/ops/gqa_attention.cu:157-302 of the reference.
 #include "qwen3/ops/gqa_attention.h"
 
+#include "../core/block_cache.hpp"
+#include "../kernels/dispatch.hpp"
 #include "ops_common.hpp"
 
 #include <limits>
@@ -54,16 +56,20 @@ namespace qwen3::ops
             const std::int64_t B = query.shape()[0], S = query.shape()[1];
             const auto Hkv = static_cast<std::int32_t>(key_cache.shape()[2]);
             const auto D = static_cast<std::int32_t>(key_cache.shape()[3]);
-            // a launch too small for the GPU splits the key range; its slices need a workspace
-            const std::int64_t ws_bytes =
-                q3k_gqa_attention_workspace_bytes(B, S, num_query_heads, Hkv, D, key_cache.shape()[1]);
-            Tensor workspace = Tensor::empty(Shape{(ws_bytes + 3) / 4}, DType::Float32, query.device());
+            // A launch too small for the GPU splits the key range, and its slices need a workspace: of this call's
+            // own split, as it is taken anew for each call (the query of the C API covers every shorter context
+            // too, several times as much)
+            const q3k::AttnSplit split = q3k::plan_attention(B, S, num_query_heads, Hkv, D, start_position, ks, vs, true,
+                                                             std::numeric_limits<std::int64_t>::max(), true)
+                                             .split;
+            const std::int64_t ws_bytes = split.splits > 1 ? split.bytes : 0;
+            const qwen3::detail::DeviceWorkspace workspace(static_cast<std::size_t>(ws_bytes), query.device().index());
             detail::launch_on(query.device(), [&](q3k_stream_t stream) {
                 return q3k_gqa_attention_bf16(
                     detail::bf16_ptr(query), static_cast<const uint16_t *>(key_cache.data()),
                     static_cast<const uint16_t *>(value_cache.data()), detail::bf16_ptr(output), B, S,
                     num_query_heads, Hkv, D, key_cache.shape()[1], start_position, ks, vs,
-                    ws_bytes > 0 ? workspace.data() : nullptr, ws_bytes, stream);
+                    workspace.data(), ws_bytes, stream);
             });
         }
     } // namespace

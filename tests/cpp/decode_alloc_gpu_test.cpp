@@ -1,7 +1,7 @@
 // A decode step's selection and attention calls allocate no device memory
 // once warm: Sampler::sample (greedy, GPU top-k, whole-row), the
-// sample-into form, argmax_last_dimension and the key-split decode
-// attention, counted with qwen3::device_allocation_count() (hipMalloc calls
+// sample-into form, argmax_last_dimension and decode attention of one
+// sequence and of batches, counted with qwen3::device_allocation_count() (hipMalloc calls
 // made by Buffers).  Also prints the host latency per token of each call.
 #include "gpu_util.hpp"
 #include "qwen3/generation/sampler.h"
@@ -63,14 +63,28 @@ namespace
             steady(("Sampler top_k 20 into a tensor" + b).c_str(), 20, [&] { s.sample(logits, out); });
             steady(("Sampler top_k 0 (whole rows)" + b).c_str(), B == 1 ? 10 : 2, [&] { w.sample(logits, out); });
         }
-        // decode attention over a long cache: the key range is split, with a workspace
-        constexpr std::int64_t Hq = 32, Hkv = 8, D = 128, L = 4096;
-        Tensor q = test::to_gpu(test::values(Hq * D, 3, 1.0F), Shape{1, 1, Hq * D}, DType::BFloat16);
-        Tensor kc = test::to_gpu(test::values(L * Hkv * D, 4, 1.0F), Shape{1, L, Hkv, D}, DType::BFloat16);
-        Tensor vc = test::to_gpu(test::values(L * Hkv * D, 5, 1.0F), Shape{1, L, Hkv, D}, DType::BFloat16);
-        steady("grouped_query_attention decode B=1 L=4096", 20, [&] {
-            (void)qwen3::ops::grouped_query_attention(q, kc.view(), vc.view(), static_cast<std::int32_t>(Hq), L - 1);
-        });
+        // decode attention over a long cache: one sequence's keys are split, with a workspace; the batches after it
+        // are split into few slices, or not at all
+        struct Decode
+        {
+            std::int64_t B, L, Hq, Hkv;
+        };
+        for (const Decode &c : {Decode{1, 4096, 32, 8}, Decode{8, 2048, 32, 8}, Decode{16, 1024, 32, 8},
+                                Decode{32, 1024, 32, 8}, Decode{8, 2048, 40, 8}, Decode{32, 600, 40, 8},
+                                Decode{8, 2000, 64, 8}, Decode{34, 1200, 64, 8}, Decode{64, 2048, 8, 1}})
+        {
+            constexpr std::int64_t D = 128;
+            Tensor q = test::to_gpu(test::values(static_cast<std::size_t>(c.B * c.Hq * D), 3, 1.0F),
+                                    Shape{c.B, 1, c.Hq * D}, DType::BFloat16);
+            Tensor cache = Tensor::empty(Shape{c.B, c.L, c.Hkv, D}, DType::BFloat16, qwen3::Device::cuda(0));
+            QWEN3_HIP_CHECK(hipMemset(cache.data(), 0, cache.nbytes()));
+            const std::string what = "decode attention " + std::to_string(c.Hq) + "/" + std::to_string(c.Hkv) +
+                                     " B=" + std::to_string(c.B) + " L=" + std::to_string(c.L);
+            steady(what.c_str(), 20, [&] {
+                (void)qwen3::ops::grouped_query_attention(q, cache.view(), cache.view(),
+                                                          static_cast<std::int32_t>(c.Hq), c.L - 1);
+            });
+        }
     }
 } // namespace
 
