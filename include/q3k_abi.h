@@ -209,11 +209,14 @@ Q3K_API int q3k_gqa_attention_bf16(const uint16_t *q, const uint16_t *k_cache,
                           q3k_stream_t stream);
 
 /*
- * Workspace bytes that let q3k_gqa_attention_bf16 split this shape's key
- * range (0: it does not split), and that of any shorter context: one of the
- * size for the cache's length serves every step up to it.  A call may leave
- * it unused where one launch is the faster way (a few hundred keys).  No counterpart in the reference
- * (its kernel is one block per query row).
+ * Workspace bytes that let q3k_gqa_attention_bf16 split the key range of
+ * `cached` keys, or of any shorter context of the same B, S and heads (0: it
+ * splits none of them): one of the size for the cache's length serves every
+ * decode step up to it.  Another B or S may need more: a workspace held for
+ * several takes the largest of their sizes.  A call may leave it unused where one
+ * launch is the faster way (a few hundred keys).  For cached == S, a whole
+ * prefill, it is what that call uses.  No counterpart in the reference (its
+ * kernel is one block per query row).
  */
 Q3K_API int64_t q3k_gqa_attention_workspace_bytes(int64_t B, int64_t S,
                           int32_t Hq, int32_t Hkv, int32_t D, int64_t cached);

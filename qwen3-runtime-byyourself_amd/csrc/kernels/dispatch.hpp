@@ -323,13 +323,20 @@ namespace q3k
         return plan_attention_prefill(B, S, Hq, Hkv, cached, true);
     }
 
-    // Workspace of the most slices a call of up to `cached` keys may be cut into: a
-    // caller that sizes it once for the length of its cache never has too little
-    // for a shorter context.  (The plan's own slices go up and down with the length:
-    // 64 sequences of 4 / 1 heads take 4 slices at 16384 keys and 16 at 1924.)
+    // Workspace of the most slices a call of these B and S and up to `cached` keys may
+    // be cut into: a caller that sizes it once for the length of its cache never has
+    // too little for a shorter context.  (The plan's own slices go up and down with the
+    // length: 64 sequences of 4 / 1 heads take 4 slices at 16384 keys and 16 at 1924.)
+    // With no keys before the S positions there is no shorter context, and it is the
+    // call's own: 0 for a prefill of 2048 tokens of 16 / 8 heads, where the bound is 49 MiB.
     inline int64_t attention_workspace_bytes(int64_t B, int64_t S, int32_t Hq, int32_t Hkv, int64_t cached)
     {
         const int64_t pairs = B * Hkv, cols = S * (Hq / Hkv);
+        if (cached == S)
+        {
+            const AttnSplit split = plan_attention_split(B, S, Hq, Hkv, cached);
+            return split.splits > 1 ? split.bytes : 0;
+        }
         int64_t most, keys; // slices, and the fewest keys of one
         if (cols <= kAttColsPerWave)
         {

@@ -1,6 +1,6 @@
 // The attention workspace (csrc/kernels/dispatch.hpp): one sized for the cache's
 // length holds the split of every shorter context, and never shrinks as the
-// context grows.
+// context grows; a whole prefill's is what its launch uses.
 #include "../../qwen3-runtime-byyourself_amd/csrc/kernels/dispatch.hpp"
 #include "test_util.hpp"
 
@@ -29,6 +29,8 @@ namespace
                         const AttnSplit p = plan_attention_split(B, S, h[0], h[1], cached);
                         require(bytes >= before, what + ": less workspace than for a shorter context");
                         require(p.splits == 1 || bytes >= p.bytes, what + ": the split needs more than the workspace");
+                        require(cached > S || bytes == (p.splits > 1 ? p.bytes : 0),
+                                what + ": a whole prefill asks for what it does not use");
                         before = bytes;
                         split += p.splits > 1;
                     }
