@@ -94,7 +94,7 @@ namespace q3k
         int32_t split_keys = INT32_MAX;
         int32_t key_groups = 1; // groups of waves of a block that share its columns and divide its keys (1, 2 or 4)
         int32_t decode_waves = 0; // waves of a decode block (1, 2 or 4); 0: not the decode kernel
-        int64_t bytes = 0; // workspace of the best split (unnormalised O^T, max and sum of each slice, fp32), taken or not
+        int64_t bytes = 0; // workspace of the split (unnormalised O^T, max and sum of each slice, fp32); 0: splits == 1
     };
 
     // Columns of a block and keys of a step for each number of key groups: four
@@ -311,7 +311,6 @@ namespace q3k
         }
         if (can_split && best_split_us >= 0.0 && best_split_us < best_us)
             return best_split;
-        best.bytes = best_split.bytes;
         return best;
     }
 
@@ -333,10 +332,7 @@ namespace q3k
     {
         const int64_t pairs = B * Hkv, cols = S * (Hq / Hkv);
         if (cached == S)
-        {
-            const AttnSplit split = plan_attention_split(B, S, Hq, Hkv, cached);
-            return split.splits > 1 ? split.bytes : 0;
-        }
+            return plan_attention_split(B, S, Hq, Hkv, cached).bytes;
         int64_t most, keys; // slices, and the fewest keys of one
         if (cols <= kAttColsPerWave)
         {
@@ -361,7 +357,7 @@ namespace q3k
     struct AttnPlan
     {
         bool mfma = false;   // attn_mfma_kernel; otherwise attn_generic_kernel
-        int g_instance = 0;  // the compiled group size (1, 2, 4, 8, 16, 32), or 0: taken at run time
+        int g_instance = 0;  // the compiled group size (1, 2, 4, 8, 16, 32) of a whole-block prefill, or 0: taken at run time
         int waves = kAttWavesPerBlock; // waves that divide a block's columns or, in decode, its keys
         AttnSplit split;     // key groups; splits > 1: the key range is split and attn_combine_kernel merges
     };
@@ -385,7 +381,6 @@ namespace q3k
                  ks[2] % 8 == 0 && vs[0] % 8 == 0 && vs[1] % 8 == 0 && vs[2] % 8 == 0 && aligned;
         if (!p.mfma)
             return p;
-        p.g_instance = (G == 1 || G == 2 || G == 4 || G == 8 || G == 16 || G == 32) ? G : 0;
         p.split = plan_attention_split(B, S, Hq, Hkv, start + S);
         if (p.split.splits > 1 &&
             (p.split.splits > kAttMaxSplits || workspace_bytes < p.split.bytes || !workspace_aligned))
@@ -393,6 +388,8 @@ namespace q3k
                                                : plan_attention_prefill(B, S, Hq, Hkv, start + S, false);
         if (p.split.decode_waves > 0)
             p.waves = p.split.decode_waves;
+        else if (p.split.key_groups == 1 && (G == 1 || G == 2 || G == 4 || G == 8 || G == 16 || G == 32))
+            p.g_instance = G;
         return p;
     }
 } // namespace q3k

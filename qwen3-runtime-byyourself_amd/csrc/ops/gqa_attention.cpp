@@ -59,10 +59,9 @@ namespace qwen3::ops
             // A launch too small for the GPU splits the key range, and its slices need a workspace: of this call's
             // own split, as it is taken anew for each call (the query of the C API covers every shorter context
             // too, several times as much)
-            const q3k::AttnSplit split = q3k::plan_attention(B, S, num_query_heads, Hkv, D, start_position, ks, vs, true,
-                                                             std::numeric_limits<std::int64_t>::max(), true)
-                                             .split;
-            const std::int64_t ws_bytes = split.splits > 1 ? split.bytes : 0;
+            const std::int64_t ws_bytes = q3k::plan_attention(B, S, num_query_heads, Hkv, D, start_position, ks, vs, true,
+                                                              std::numeric_limits<std::int64_t>::max(), true)
+                                              .split.bytes;
             const qwen3::detail::DeviceWorkspace workspace(static_cast<std::size_t>(ws_bytes), query.device().index());
             detail::launch_on(query.device(), [&](q3k_stream_t stream) {
                 return q3k_gqa_attention_bf16(

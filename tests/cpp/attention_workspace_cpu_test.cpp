@@ -28,8 +28,9 @@ namespace
                         const int64_t bytes = attention_workspace_bytes(B, S, h[0], h[1], cached);
                         const AttnSplit p = plan_attention_split(B, S, h[0], h[1], cached);
                         require(bytes >= before, what + ": less workspace than for a shorter context");
-                        require(p.splits == 1 || bytes >= p.bytes, what + ": the split needs more than the workspace");
-                        require(cached > S || bytes == (p.splits > 1 ? p.bytes : 0),
+                        require((p.splits > 1) == (p.bytes > 0), what + ": a size without a split, or a split without");
+                        require(bytes >= p.bytes, what + ": the split needs more than the workspace");
+                        require(cached > S || bytes == p.bytes,
                                 what + ": a whole prefill asks for what it does not use");
                         before = bytes;
                         split += p.splits > 1;

@@ -84,7 +84,9 @@ namespace
                 const AttnSplit split = plan_attention_split(B, S, h.hq, h.hkv, L);
                 const AttnPlan p = plan_attention(B, S, h.hq, h.hkv, 128, start, st, st, true, split.bytes, true);
                 require(p.mfma, what + ": generic kernel chosen");
-                require(p.g_instance == want_g, what + ": group-size instance");
+                // the group size compiled in is that of whole-block prefills: decode and key groups take it at run time
+                require(p.g_instance == (decode || p.split.key_groups > 1 ? 0 : want_g), what + ": group-size instance");
+                require(decode == (p.split.decode_waves > 0), what + ": decode kernel");
                 require(p.split.splits == split.splits, what + ": the workspace the library asks for splits the keys");
                 if (decode)
                 {
