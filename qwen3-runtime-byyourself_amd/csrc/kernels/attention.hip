@@ -842,11 +842,6 @@ namespace q3k
         constexpr int kMaxSplits = kAttMaxSplits;
         constexpr int kCombineWaves = 4;
         constexpr int kCombineRound = kMaxSplits / kCombineWaves; // slices whose O^T a wave loads at once
-        // Up to this many rows a row takes a block (decode: its slices are many,
-        // their loads all in flight), above it a wave: 16384 rows of 4 slices took
-        // 13.0 us with a block each and 9.6 us with a wave each.
-        constexpr int64_t kCombineWideRows = 2048;
-
         struct CombineArgs
         {
             const float *part_o;
@@ -956,7 +951,7 @@ namespace q3k
         // itself, so a wave merges four rows with no exchange between lanes (1 x 512
         // tokens after 7680, 32 / 8 heads, 16384 rows of 4 slices: 96.1 us with the
         // attention, 98.5 with a wave a row; 260 after 4096: 37.0 and 39.1).
-        constexpr int kCombineFewSplits = 8;
+        constexpr int kCombineFewSplits = kAttLaneMergeSplits;
         constexpr int kCombineRows = kBlock / 16; // rows of a block
 
         __global__ __launch_bounds__(kBlock) void attn_combine_rows_kernel(CombineArgs a)
@@ -1078,16 +1073,23 @@ namespace q3k
                 const auto S = static_cast<unsigned>(a.S), batch = static_cast<unsigned>(B);
                 const auto heads = static_cast<unsigned>(a.Hq);
                 const dim3 threads(kCombineWaves * kWave);
-                if (S == 1)
-                    attn_combine_kernel<kCombineWaves, false><<<dim3(heads, 1, batch), threads, 0, stream>>>(c);
-                else if (a.rows <= kCombineWideRows)
-                    attn_combine_kernel<kCombineWaves, true><<<dim3(heads, S, batch), threads, 0, stream>>>(c);
-                else if (a.splits <= kCombineFewSplits)
+                switch (attn_merge(a.S, a.rows, a.splits))
+                {
+                case AttnMerge::BlockRow:
+                    if (S == 1)
+                        attn_combine_kernel<kCombineWaves, false><<<dim3(heads, 1, batch), threads, 0, stream>>>(c);
+                    else
+                        attn_combine_kernel<kCombineWaves, true><<<dim3(heads, S, batch), threads, 0, stream>>>(c);
+                    break;
+                case AttnMerge::LaneRow:
                     attn_combine_rows_kernel<<<dim3(static_cast<unsigned>(blocks_for(a.rows, kCombineRows))), dim3(kBlock), 0,
                                                stream>>>(c);
-                else
+                    break;
+                case AttnMerge::WaveRow:
                     attn_combine_kernel<1, true>
                         <<<dim3((heads + kCombineWaves - 1) / kCombineWaves, S, batch), threads, 0, stream>>>(c);
+                    break;
+                }
             }
             return check_launch("grouped_query_attention");
         }

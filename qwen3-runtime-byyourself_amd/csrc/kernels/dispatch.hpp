@@ -354,6 +354,27 @@ namespace q3k
         return most < 2 ? 0 : most * B * S * Hq * (kAttHeadDim + 2) * 4;
     }
 
+    // Which kernel merges the slices of the query rows.
+    enum class AttnMerge
+    {
+        BlockRow, // a block of four waves a row: few rows (decode), their slices many
+        LaneRow,  // 16 lanes a row: many rows of few slices
+        WaveRow   // a wave a row: many rows of more slices
+    };
+    // Up to this many rows a row takes a block (its loads all in flight), above it a
+    // wave or 16 lanes: 16384 rows of 4 slices took 13.0 us with a block each and 9.6 us
+    // with a wave each, and the whole launch 98.5 with those and 96.1 with 16 lanes.
+    constexpr int64_t kAttBlockMergeRows = 2048;
+    // Slices that a lane of the 16 holds at once.
+    constexpr int32_t kAttLaneMergeSplits = 8;
+
+    inline AttnMerge attn_merge(int64_t S, int64_t rows, int32_t splits)
+    {
+        if (S == 1 || rows <= kAttBlockMergeRows)
+            return AttnMerge::BlockRow;
+        return splits <= kAttLaneMergeSplits ? AttnMerge::LaneRow : AttnMerge::WaveRow;
+    }
+
     struct AttnPlan
     {
         bool mfma = false;   // attn_mfma_kernel; otherwise attn_generic_kernel

@@ -123,10 +123,36 @@ namespace
                 "an unaligned workspace used");
     }
 
+    // Which kernel merges the slices, at shapes that the GPU tests run.
+    void merge_cases()
+    {
+        using namespace q3k;
+        struct Case
+        {
+            int64_t B, S, start;
+            int32_t Hq, Hkv;
+            AttnMerge merge;
+            int32_t splits; // at least
+        };
+        const Case cases[] = {{1, 1, 4095, 32, 8, AttnMerge::BlockRow, 17},   {13, 1, 1278, 32, 8, AttnMerge::BlockRow, 2},
+                              {1, 7, 4090, 32, 8, AttnMerge::BlockRow, 17},   {1, 260, 4000, 32, 8, AttnMerge::LaneRow, 2},
+                              {1, 2048, 0, 4, 1, AttnMerge::LaneRow, 2},      {1, 1075, 0, 2, 1, AttnMerge::WaveRow, 9},
+                              {1, 167, 11748, 16, 8, AttnMerge::WaveRow, 16}, {1, 701, 11748, 4, 1, AttnMerge::WaveRow, 17}};
+        for (const Case &c : cases)
+        {
+            const std::string what = "merge of B " + std::to_string(c.B) + ", S " + std::to_string(c.S) + " after " +
+                                     std::to_string(c.start) + ", " + std::to_string(c.Hq) + "/" + std::to_string(c.Hkv);
+            const AttnSplit p = plan_attention_split(c.B, c.S, c.Hq, c.Hkv, c.start + c.S);
+            require(p.splits >= c.splits, what + ": slices");
+            require(attn_merge(c.S, c.B * c.S * c.Hq, p.splits) == c.merge, what + ": kernel");
+        }
+    }
+
     void body()
     {
         rope_cases();
         attention_cases();
+        merge_cases();
     }
 } // namespace
 

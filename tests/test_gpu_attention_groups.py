@@ -45,10 +45,11 @@ def test_gqa_attention_key_groups(q3k, hip, oracle, synth, B, S, start, Hq, Hkv)
 
 
 # chunks and prefills whose keys are split: slices that some query blocks do not reach, blocks with a single slice
-# (which write their result themselves), more slices than one merge round, rows for both merge shapes
+# (which write their result themselves); rows merged by a block each (few), by 16 lanes (many, of few slices) and by a
+# wave (many, of more: 9, 16 and, in two rounds, 22 slices)
 @pytest.mark.parametrize("B,S,start,Hq,Hkv", [
     (1, 2048, 0, 4, 1), (1, 7, 4090, 32, 8), (1, 70, 4000, 32, 8), (1, 260, 4000, 32, 8), (1, 600, 3000, 5, 1),
-    (1, 3000, 0, 2, 1), (1, 2, 8000, 8, 1)])
+    (1, 3000, 0, 2, 1), (1, 2, 8000, 8, 1), (1, 1075, 0, 2, 1), (1, 167, 11748, 16, 8), (1, 701, 11748, 4, 1)])
 def test_gqa_attention_key_groups_split(q3k, hip, oracle, synth, B, S, start, Hq, Hkv):
     name = f"gqa_attention groups, split, B={B} S={S} start={start} Hq={Hq} Hkv={Hkv}"
     announce(name)

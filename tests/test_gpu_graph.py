@@ -50,6 +50,7 @@ def test_graph_replay_decode_step(q3k, hip, synth):
     wk = q3k.topk_workspace_bytes(Bd, V, K)
     assert wa > 0 and wm > 0 and wk > 0, "the decode shapes should take the split and sliced paths"
     ws_a, ws_m, ws_k = hip.DeviceBuffer(wa), hip.DeviceBuffer(wm), hip.DeviceBuffer(wk)
+    ws_a.fill_bytes(0xA5)
     st = (L * Hkv * D, Hkv * D, D, 1)
     stream = hip.Stream()
     b = bufs
@@ -90,6 +91,7 @@ def test_graph_replay_decode_step(q3k, hip, synth):
     stream.synchronize()
     eager = results()
     assert not np.array_equal(eager["h1"], arrays["h1"]), "the step should have updated the residual"
+    assert (ws_a.download(np.uint8, (wa,)) != 0xA5).any(), "the decode attention should split its keys"
 
     reset()
     graph = hip.Graph(stream, step)

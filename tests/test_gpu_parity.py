@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 
 import kat
-from gpu_util import Guarded, announce, check_band, check_exact
+from gpu_util import GUARD_BYTE, Guarded, announce, check_band, check_exact
 
 pytestmark = pytest.mark.gpu
 EPS = 1e-6
@@ -632,10 +632,15 @@ def test_qk_norm_rope_kv_append(q3k, hip, oracle, synth, B, S, Hq, Hkv, D, Sc, c
 
 # ---------------------------------------------------------------- attention
 
+def written(workspace):
+    """Whether a launch has left anything in a Guarded workspace, which starts out as a fixed pattern."""
+    return bool((workspace.get(np.uint8, (workspace.n,)) != GUARD_BYTE).any())
+
+
 def run_attention(q3k, hip, q, store_k, store_v, B, S, Hq, start, offset=0, split=False):
     """q [B, S, Hq * D]; the caches are whole KvCache-like layers [Bcap, Scap, Hkv, D], read through the
     [B, start + S] view (strides of the storage), as KvCache::key_view hands them over.  With split, a workspace of
-    the size the library asks for lets it split the key range."""
+    the size the library asks for lets it split the key range, and it has to."""
     _, Scap, Hkv, D = store_k.shape
     Q, K, V = Guarded(hip, q, offset=offset), Guarded(hip, store_k, offset=offset), Guarded(hip, store_v, offset=offset)
     O = Guarded(hip, nbytes=q.nbytes, offset=offset)
@@ -648,6 +653,7 @@ def run_attention(q3k, hip, q, store_k, store_v, B, S, Hq, start, offset=0, spli
     hip.synchronize()
     assert all(b.guards_intact() for b in (Q, K, V, O) + ((W,) if W else ()))
     assert np.array_equal(Q.get(np.uint16, q.shape), q) and np.array_equal(K.get(np.uint16, store_k.shape), store_k)
+    assert W is None or written(W), "the launch did not split the keys"
     return O.get(np.uint16, q.shape)
 
 
@@ -980,16 +986,16 @@ def test_topk_candidates_ties(q3k, hip, oracle, synth, rows, N, k, levels, split
 
 
 @pytest.mark.parametrize("B,S,start,Hq,Hkv,cap", [(1, 1, 4095, 32, 8, 4096), (2, 5, 700, 32, 8, 800),
-                                                 (1, 1, 300, 64, 8, 320), (1, 3, 400, 16, 8, 420),
+                                                 (1, 1, 700, 64, 8, 720), (1, 3, 700, 16, 8, 720),
                                                  (4, 1, 1000, 32, 8, 1100), (1, 1, 1000, 8, 8, 1100),
-                                                 (1, 1, 500, 16, 8, 512), (2, 1, 900, 32, 2, 1000),
-                                                 (1, 1, 2000, 32, 1, 2100), (3, 1, 129, 32, 8, 200),
+                                                 (1, 1, 650, 16, 8, 700), (2, 1, 900, 32, 2, 1000),
+                                                 (1, 1, 2000, 32, 1, 2100), (13, 1, 1278, 32, 8, 1290),
                                                  (1, 1, 4095, 40, 8, 4096), (2, 3, 600, 40, 8, 700)])
 def test_gqa_attention_split_keys(q3k, hip, oracle, synth, B, S, start, Hq, Hkv, cap):
     """Decode with few sequences: the key range is split across blocks (the workspace the library asks for) and the
     slices merged; same band as the single-pass kernel.  Decode steps whose slices hold one or two tiles run as
-    one-wave blocks: covered for every group size G = Hq / Hkv from 1 to 32, and a cache of 130 keys (two slices,
-    the second a partial tile)."""
+    one-wave blocks: covered for every group size G = Hq / Hkv from 1 to 32, and 13 sequences of 1279 keys (two
+    slices, the second ending inside a tile)."""
     D = 128
     name = f"gqa_attention split B={B} S={S} start={start} Hq={Hq} Hkv={Hkv}"
     announce(name)
@@ -1037,7 +1043,7 @@ def test_prefill_then_decode_matches_one_shot(q3k, hip, oracle, synth):
         W = Guarded(hip, nbytes=ws) if ws else None
         q3k.gqa_attention(Qb, KC, VC, O, B, S, Hq, Hkv, D, start + S, start, st, st, workspace=W, workspace_bytes=ws)
         hip.synchronize()
-        assert O.guards_intact() and (W is None or W.guards_intact())
+        assert O.guards_intact() and (W is None or (W.guards_intact() and written(W)))
         return O.get(np.uint16, (B, S, Hq * D))
 
     # one prefill of all T tokens
