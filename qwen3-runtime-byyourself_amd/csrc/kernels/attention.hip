@@ -115,16 +115,6 @@ namespace q3k
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t *)lds_wave, 16, voffset, 0, 0, 0);
         }
 
-        // Renumbers workgroup ids so that the ids one XCD receives (id % kXcds
-        // == x, in dispatch order) become the contiguous range of the x-th
-        // share of the grid.
-        constexpr unsigned kXcds = 8;
-        __device__ __forceinline__ int xcd_contiguous(unsigned id, unsigned n)
-        {
-            const unsigned x = id % kXcds, k = id / kXcds, q = n / kXcds, r = n % kXcds;
-            return static_cast<int>(x < r ? x * (q + 1) + k : r * (q + 1) + (x - r) * q + k);
-        }
-
         // max / sum of x over lanes l and l ^ 32, in every lane (one VALU swap,
         // no LDS): after the swap one operand is x and the other its partner
         __device__ __forceinline__ float pair_max(float x)
