@@ -112,6 +112,67 @@ def test_bench_wrappers_refuse_buffers_smaller_than_the_call(q3k):
         q3k.bench_stream(big, big, big, small, 1 << 21)
 
 
+class _HandsBack:
+    """In place of the native calls: takes no argument at all, so that every wrapper goes through ctypes."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+class _Buffer:
+    def __init__(self, ptr):
+        self.ptr = ptr
+
+
+def _outcome(fn, args):
+    try:
+        return fn(*args)
+    except Exception as e:  # noqa: BLE001
+        return type(e), getattr(e, "status", None), str(e)
+
+
+def test_native_calls_take_what_ctypes_takes(q3k, monkeypatch):
+    """The wrappers' native calls convert ints, floats, None, buffer objects and tuples of strides themselves and hand
+    anything else back to ctypes: every wrapper has to end in the same result or the same exception either way.  No
+    call gets as far as a launch (no rows, negative rows, null pointers or another refused argument)."""
+    f, st = 256, (64, 64, 64, 1)
+    attn = (None, f, f, f, 1, 1, 2, 1, 128, 4, 3)
+    cases = [(q3k.rms_norm, a) for a in (
+        (None, None, None, 0, 128, 1e-6), (f, f, f, 4, 128, 0.0),
+        # an int or a bool for the epsilon, a bool, a numpy int or a float for a count
+        (f, f, f, 4, 128, 0), (f, f, f, 4, 128, -1), (f, f, f, -1, 128, True), (f, f, f, False, 128, 1e-6),
+        (f, f, f, np.int64(-1), 128, 1e-6), (f, f, f, 4.0, 128, 1e-6), (f, f, f, None, 128, 1e-6),
+        (f, f, f, 4, 128, np.float32(0.0)), (f, f, f, 4, 128, "1"),
+        # ints past the parameter's width
+        (f, f, f, 2**64 - 1, 128, 1e-6), (f, f, f, 2**64, 128, 1e-6), (f, f, f, -(2**63) - 1, 128, 1e-6),
+        # pointers: buffer objects, their .ptr anything, ctypes pointers, what is none
+        (_Buffer(None), f, f, 4, 128, 1e-6), (_Buffer(f), f, _Buffer(0), 4, 128, 1e-6),
+        (_Buffer(ctypes.c_void_p(None)), f, f, 4, 128, 1e-6), (ctypes.c_void_p(None), f, f, 4, 128, 1e-6),
+        (_Buffer("x"), f, f, 0, 128, 1e-6), ("x", f, f, 0, 128, 1e-6), (1.5, f, f, 0, 128, 1e-6),
+        (np.int64(0), f, f, 4, 128, 1e-6), (True, f, f, -1, 128, 1e-6), (object(), f, f, 0, 128, 1e-6))]
+    cases += [(q3k.gqa_attention, attn + a) for a in (
+        (st, st), (list(st), list(st)), (np.array(st), np.array(st)), (st, list(st)), (tuple(np.array(st)), st),
+        ((64, -64, 64, 1), st), ([64, -64, 64, 1], st), (st[:3], st), (st + (1,), st), (None, st), ("abcd", st),
+        (tuple(float(x) for x in st), st), ((2**63, 64, 64, 1), st))]
+    cases += [(q3k.embedding, ([], 0, f, 10, 8, f)), (q3k.embedding, (None, True, f, 10, 8, f)),
+              (q3k.add_rms_norm, (f, None, f, f, 4, 128, 1)), (q3k.rms_norm_rows, (None, f, f, 2, 0, 1, 128, 1)),
+              (q3k.add_rms_norm_rows, (f, None, f, f, 2, 0, 1, 128, 1)),
+              (q3k.embedding_rms_norm, (None, True, f, 10, 8, f, 1, f, f)), (q3k.add_inplace, (None, f, True)),
+              (q3k.silu_mul, (f, f, None, np.int32(8))), (q3k.rope, (f, 1, 3, 2, 8, f, 16, np.int64(-1))),
+              (q3k.rope_qk, (f, f, 1, 16, 2, 1, 8, f, 16, True, ctypes.c_void_p(None), None)),
+              (q3k.qk_norm_rope, (f, f, None, f, 1, 3, 2, 1, 8, 1, f, 16, 0)), (q3k.argmax, (f, f, 2, 100, np.int64(101))),
+              (q3k.argmax, (f, f, -1, 100, 100, None, f, True)), (q3k.argmax_noalloc, (f, f, True, 8, 9)),
+              (q3k.topk_candidates, (f, 2, 100, 100, True, 0, f, f, f, f)),
+              (q3k.kv_append, (None, f, f, f, True, 1, 16, 4, 0)),
+              (q3k.qk_norm_rope_kv_append, (f, f, f, None, f, 1, 3, 2, 1, 8, 1, f, 16, 0, f, f, 16, 0))]
+    native = [_outcome(fn, args) for fn, args in cases]
+    q3k.load()
+    monkeypatch.setattr(q3k, "_calls", _HandsBack())
+    for (fn, args), got in zip(cases, native):
+        want = _outcome(fn, args)
+        assert got == want, f"{fn.__name__}{args}: {got}, through ctypes {want}"
+
+
 def test_empty_inputs_are_no_ops(q3k):
     # zero work returns OK without a launch (no GPU needed)
     q3k.rms_norm(None, None, None, 0, 128, 1e-6)
