@@ -698,9 +698,9 @@ namespace q3k
         // two K and two V buffers with no barrier: a buffer is refilled as soon as
         // its products are issued, and a wave waits only for the tile it needs, so
         // about 1.5 tiles of K and V (24 KiB a wave) stay in flight throughout.  What
-        // bounds it is memory for many sequences (64 x 4096 keys of 32 / 8 heads: 184.7
-        // us, 5.8 TB/s; 193.0 with the four-wave prefill kernel, one of whose waves
-        // computed) and the latency of a launch, a tile and the merge for few (1 x 8191
+        // bounds it is memory for many sequences (64 x 4096 keys of 32 / 8 heads: 184.9
+        // us, 5.8 TB/s; 189.0 with the four-wave prefill kernel, one of whose waves
+        // computed, in alternating runs) and the latency of a launch, a tile and the merge for few (1 x 8191
         // of 16 / 8: 12.2 -> 11.4 us; 40 x 3000 of 16 / 8: 119 -> 88; 19 x 8548 of
         // 5 / 1: 27 -> 18; 1 x 250: 10.0 -> 6.7).
         template <int KW>
