@@ -17,6 +17,7 @@
 #include "q3k_common.hpp"
 
 #include <mutex>
+#include <type_traits>
 
 namespace q3k
 {
@@ -74,7 +75,7 @@ namespace q3k
             }
         };
 
-        constexpr int kUnroll = 5;
+        constexpr int kUnroll = 5; // most vectors a thread has in flight
         typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
         __device__ __forceinline__ uint32_t max_i16x2(uint32_t a, uint32_t b)
         {
@@ -128,7 +129,7 @@ namespace q3k
         // This thread's best key over columns [begin, end) of row r, or 0 (below every
         // candidate): the best of all threads' is the row's.
         //
-        // The 16-byte aligned middle of the range goes kUnroll vectors a thread at a
+        // The 16-byte aligned middle of the range goes UNROLL vectors a thread at a
         // time, all loaded before any is used; of the vectors seen only the one
         // holding the first maximum is kept.  A wave that sees a positive value in its
         // first vectors scans for those alone: a packed instruction for two columns (a
@@ -141,6 +142,7 @@ namespace q3k
         // as one and a half reads (no positive value, 1 / 64 / 256 rows of 151936: 5.7 /
         // 6.8 / 13.6 us, 19.7 / 21.2 / 30.0 with the second pass; ordinary rows 4.6 / 6.2 /
         // 13.2 either way).
+        template <int UNROLL>
         __device__ __forceinline__ uint64_t thread_best(const uint16_t *r, int64_t begin, int64_t end)
         {
             const Middle mid(r, begin, end);
@@ -149,23 +151,26 @@ namespace q3k
             int32_t tid = threadIdx.x;
             __asm__ volatile("" : "+v"(tid)); // nothing of a row is kept in registers for the next one
             const int64_t side = mid.side(tid);
+            if (__ballot(tid < nv || side >= 0) == 0)
+                return 0; // a short row: nothing for this wave
+            const uint32_t side_bits = side >= 0 ? r[side] : 0u; // beside the vectors
             Scan p{0, 0, {}}, n{-1, 0, {}};
             bool negative = true; // the wave has seen no positive value in its first vectors
-            for (int32_t i0 = 0; i0 < nv; i0 += kUnroll * kArgmaxBlock)
+            for (int32_t i0 = 0; i0 < nv; i0 += UNROLL * kArgmaxBlock)
             {
                 // past the end a thread reads the last vector once more
-                Vec8 v[kUnroll];
+                Vec8 v[UNROLL];
                 auto index = [&](int u) __attribute__((always_inline)) {
                     const int32_t i = i0 + tid + u * kArgmaxBlock;
                     return i < nv ? i : nv - 1;
                 };
 #pragma unroll
-                for (int u = 0; u < kUnroll; ++u)
+                for (int u = 0; u < UNROLL; ++u)
                     v[u] = load8<false>(rv + index(u));
-                int32_t x[kUnroll], top = 0;
+                int32_t x[UNROLL], top = 0;
                 auto maxima = [&]() __attribute__((always_inline)) {
 #pragma unroll
-                    for (int u = 0; u < kUnroll; ++u)
+                    for (int u = 0; u < UNROLL; ++u)
                     {
                         x[u] = max_of(v[u].d[0], v[u].d[1], v[u].d[2], v[u].d[3]);
                         top = x[u] > top ? x[u] : top;
@@ -177,7 +182,7 @@ namespace q3k
                     if (__ballot(top > 0x7f80) != 0)
                     {
 #pragma unroll
-                        for (int u = 0; u < kUnroll; ++u)
+                        for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
                             for (int j = 0; j < 4; ++j)
                                 v[u].d[j] = without_nan(v[u].d[j]);
@@ -185,14 +190,14 @@ namespace q3k
                         maxima();
                     }
 #pragma unroll
-                    for (int u = 0; u < kUnroll; ++u)
+                    for (int u = 0; u < UNROLL; ++u)
                         p.take(x[u], index(u), v[u]);
                 }
                 if (i0 == 0)
                     negative = __ballot(p.best > 0) == 0;
                 if (negative)
 #pragma unroll
-                    for (int u = 0; u < kUnroll; ++u)
+                    for (int u = 0; u < UNROLL; ++u)
                     {
                         constexpr uint32_t kMagnitude = 0x7fff7fffu;
                         n.take(max_of(~v[u].d[0] & kMagnitude, ~v[u].d[1] & kMagnitude, ~v[u].d[2] & kMagnitude,
@@ -201,7 +206,6 @@ namespace q3k
                     }
             }
             // the column of a scan's best, the side column included
-            const uint32_t side_bits = side >= 0 ? r[side] : 0u;
             auto column = [&](Scan &s, bool any, auto value) __attribute__((always_inline)) {
                 uint32_t at = 0;
                 if (any)
@@ -237,10 +241,11 @@ namespace q3k
         // The best key of columns [begin, end) of row r, in every thread of wave 0;
         // the shared memory (a key a wave) is free again when the call returns.
         constexpr int kArgmaxWaves = kArgmaxBlock / kWave;
+        template <int UNROLL>
         __device__ __forceinline__ uint64_t block_best(const uint16_t *r, int64_t begin, int64_t end, uint64_t *wave_key)
         {
             const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-            uint64_t best = wave_max(thread_best(r, begin, end));
+            uint64_t best = wave_max(thread_best<UNROLL>(r, begin, end));
             if (lane == 0)
                 wave_key[wave] = best;
             __syncthreads();
@@ -255,6 +260,7 @@ namespace q3k
             return static_cast<int32_t>(0xffffffffu - static_cast<uint32_t>(key));
         }
 
+        template <int UNROLL>
         __global__ __launch_bounds__(kArgmaxBlock) void argmax_kernel(const uint16_t *__restrict__ x,
                                                                       int32_t *__restrict__ out, int64_t rows,
                                                                       int64_t stride, int64_t n)
@@ -262,7 +268,7 @@ namespace q3k
             __shared__ uint64_t wave_key[kArgmaxWaves];
             for (int64_t row = blockIdx.x; row < rows; row += gridDim.x)
             {
-                const uint64_t best = block_best(x + row * stride, 0, n, wave_key);
+                const uint64_t best = block_best<UNROLL>(x + row * stride, 0, n, wave_key);
                 if (threadIdx.x == 0)
                     out[row] = key_index(best);
             }
@@ -270,6 +276,7 @@ namespace q3k
 
         // One block per (row, slice): part[row * slices + slice] = the best
         // key of columns [slice * slice_len, min(n, (slice + 1) * slice_len)).
+        template <int UNROLL>
         __global__ __launch_bounds__(kArgmaxBlock) void argmax_slice_kernel(const uint16_t *__restrict__ x,
                                                                             uint64_t *__restrict__ part,
                                                                             int64_t stride, int64_t n,
@@ -279,7 +286,7 @@ namespace q3k
             const int32_t row = static_cast<int32_t>(blockIdx.x) / slices;
             const int64_t begin = (static_cast<int32_t>(blockIdx.x) % slices) * slice_len;
             const int64_t end = begin + slice_len < n ? begin + slice_len : n;
-            const uint64_t best = block_best(x + row * stride, begin, end, wave_key);
+            const uint64_t best = block_best<UNROLL>(x + row * stride, begin, end, wave_key);
             if (threadIdx.x == 0)
                 part[blockIdx.x] = best;
         }
@@ -374,6 +381,27 @@ namespace q3k
             return Q3K_OK;
         }
 
+        // Calls launch with the vectors a thread has in flight over `columns`: no more than
+        // they take, up to kUnroll (past the end each further one costs a thread about
+        // twenty instructions: 64 rows of 1000 2.9 us, 3.3 with five; 1 of 20000 3.0 and
+        // 3.2; 600 of 1000 4.0, with the waves that have no columns going through the
+        // motions as well 5.1).
+        template <typename F>
+        void with_unroll(int64_t columns, F launch)
+        {
+            const int64_t vectors = (columns + 8 * kArgmaxBlock - 1) / (8 * kArgmaxBlock);
+            if (vectors <= 1)
+                launch(std::integral_constant<int, 1>{});
+            else if (vectors == 2)
+                launch(std::integral_constant<int, 2>{});
+            else if (vectors == 3)
+                launch(std::integral_constant<int, 3>{});
+            else if (vectors == 4)
+                launch(std::integral_constant<int, 4>{});
+            else
+                launch(std::integral_constant<int, kUnroll>{});
+        }
+
         // Launches for checked arguments: the sliced kernels when `part`
         // (8-byte aligned, room for plan.bytes) is given and the plan slices,
         // else one block per row.
@@ -382,15 +410,21 @@ namespace q3k
         {
             if (plan.slices > 1 && part != nullptr)
             {
-                argmax_slice_kernel<<<dim3(static_cast<unsigned>(rows * plan.slices)), dim3(kArgmaxBlock), 0, s>>>(
-                    x, part, row_stride, search_size, plan.slices, plan.slice_len);
+                with_unroll(plan.slice_len, [&](auto unroll) {
+                    argmax_slice_kernel<decltype(unroll)::value>
+                        <<<dim3(static_cast<unsigned>(rows * plan.slices)), dim3(kArgmaxBlock), 0, s>>>(
+                            x, part, row_stride, search_size, plan.slices, plan.slice_len);
+                });
                 const int64_t per_block = kBlock / kWave;
                 argmax_merge_kernel<<<dim3(static_cast<unsigned>((rows + per_block - 1) / per_block)), dim3(kBlock), 0,
                                       s>>>(part, out, rows, plan.slices);
                 return check_launch("argmax_last_dimension");
             }
             const unsigned grid = static_cast<unsigned>(rows < 65535 ? rows : 65535);
-            argmax_kernel<<<dim3(grid), dim3(kArgmaxBlock), 0, s>>>(x, out, rows, row_stride, search_size);
+            with_unroll(search_size, [&](auto unroll) {
+                argmax_kernel<decltype(unroll)::value>
+                    <<<dim3(grid), dim3(kArgmaxBlock), 0, s>>>(x, out, rows, row_stride, search_size);
+            });
             return check_launch("argmax_last_dimension");
         }
 

@@ -8,7 +8,7 @@ from gpu_util import Guarded, announce, check_exact
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [1, 7, 8, 9, 15, 100, 8191, 8193, 20000, 155649, 163840, 163841, 204800, 204801, 262144, 262145, 300001]
+SIZES = [1, 7, 8, 9, 15, 100, 520, 8191, 8193, 16384, 16385, 20000, 24577, 32769, 155649, 163840, 163841, 204800, 204801, 262144, 262145, 300001]
 
 
 def _rows(synth, n, stride):
