@@ -11,8 +11,8 @@
 //
 // Rows of up to 163840 columns (every Qwen3 vocabulary) with k up to 1024: one
 // block of 1024 threads a row reads it once into its registers (topk_row_kernel,
-// below).  Longer rows, and k above 1024: one block per row (rows strided over the grid),
-// two reads of the row:
+// below).  Other rows (longer, k above 1024, or too short for k): one block per
+// row (rows strided over the grid), two reads of the row:
 //   1. each thread's largest logit (16-byte loads when the row is aligned)
 //      and the non-finite flag;
 //   2. T = the k-th largest of those 1024 maxima.  The k threads whose maxima
@@ -27,7 +27,7 @@
 // each wave counts into its own histogram.  A row with a non-finite logit is
 // flagged (the reference throws for it).
 //
-// With few of those rows and a caller workspace, each row is cut into slices: one
+// With few long ones and a caller workspace, each row is cut into slices: one
 // block per (row, slice) finds the slice's bound and lists its logits at or
 // above it (steps 1-2 on the slice), and one block per row keeps the listed
 // logits at or above the largest slice bound and finishes with step 3 (or
@@ -76,9 +76,9 @@ namespace q3k
         // keys above each lane's bins, and the first lane whose bins reach k
         // walks its four bins and writes the result.
         __device__ __forceinline__ void find_bin(const uint32_t *hist, uint32_t k, uint32_t *bin_out,
-                                                 uint32_t *rank_out)
+                                                 uint32_t *rank_out, int tid)
         {
-            const int lane = own_thread() % kWave;
+            const int lane = tid % kWave;
             const int top = 255 - 4 * lane;
             uint32_t c[4];
 #pragma unroll
@@ -113,9 +113,8 @@ namespace q3k
         // k-th largest (1 <= k <= n) of the 16-bit keys key_at(0 .. n - 1),
         // block-wide, by two 8-bit radix passes over one shared histogram
         template <typename KeyAt>
-        __device__ uint32_t block_kth(KeyAt key_at, int n, uint32_t k, uint32_t *hist, uint32_t *sel)
+        __device__ uint32_t block_kth(KeyAt key_at, int n, uint32_t k, uint32_t *hist, uint32_t *sel, int tid)
         {
-            const int tid = own_thread();
             if (tid < 256)
                 hist[tid] = 0u;
             __syncthreads();
@@ -123,7 +122,7 @@ namespace q3k
                 atomicAdd(&hist[key_at(i) >> 8], 1u);
             __syncthreads();
             if (tid < kWave)
-                find_bin(hist, k, &sel[0], &sel[1]);
+                find_bin(hist, k, &sel[0], &sel[1], tid);
             __syncthreads();
             const uint32_t hi = sel[0], rank = sel[1];
             if (tid < 256)
@@ -139,7 +138,7 @@ namespace q3k
             if (tid < kWave)
             {
                 uint32_t unused;
-                find_bin(hist, rank, &sel[2], &unused);   // the low byte
+                find_bin(hist, rank, &sel[2], &unused, tid);   // the low byte
             }
             __syncthreads();
             if (tid == 0)
@@ -261,11 +260,11 @@ namespace q3k
         // The list entries at or above its k-th largest (k <= nl <= kCandMax)
         // go to the row's candidates, counted in sh.found.
         __device__ __forceinline__ void emit_list(SelShared &sh, uint32_t nl, uint32_t k, int64_t row,
-                                                  const CandOut &co)
+                                                  const CandOut &co, int tid)
         {
             const uint32_t kth = block_kth([&](int i) { return sel_key(sh.list_bits[i]); }, static_cast<int>(nl), k,
-                                           sh.hist, sh.sel);
-            for (int i = threadIdx.x; i < static_cast<int>(nl); i += kSelBlock)
+                                           sh.hist, sh.sel, tid);
+            for (int i = tid; i < static_cast<int>(nl); i += kSelBlock)
             {
                 const uint32_t b = sh.list_bits[i];
                 if (sel_key(b) >= kth)
@@ -310,7 +309,7 @@ namespace q3k
             merge();
             __syncthreads();
             if (tid < kWave)
-                find_bin(sh.hist, k, &sh.sel[0], &sh.sel[1]);
+                find_bin(sh.hist, k, &sh.sel[0], &sh.sel[1], tid);
             clear();
             __syncthreads();
             const uint32_t hi = sh.sel[0], rank = sh.sel[1];
@@ -325,7 +324,7 @@ namespace q3k
             if (tid < kWave)
             {
                 uint32_t unused;
-                find_bin(sh.hist, rank, &sh.sel[2], &unused);
+                find_bin(sh.hist, rank, &sh.sel[2], &unused, tid);
             }
             __syncthreads();
             if (tid == 0)
@@ -350,7 +349,8 @@ namespace q3k
         // logits: every logit is then taken), and its key in *key.
         __device__ __forceinline__ float maxima_bound(SelShared &sh, uint32_t k, uint32_t *key)
         {
-            const uint32_t t_key = block_kth([&](int i) { return sh.thread_max[i]; }, kSelBlock, k, sh.hist, sh.sel);
+            const uint32_t t_key = block_kth([&](int i) { return sh.thread_max[i]; }, kSelBlock, k, sh.hist, sh.sel,
+                                             threadIdx.x);
             *key = t_key;
             return t_key == 0u ? -__builtin_huge_valf() : bf_val(key_bits(t_key));
         }
@@ -376,7 +376,7 @@ namespace q3k
                 if (nl <= static_cast<uint32_t>(kCandMax))
                 {
                     // 3. exact k-th over the list (k <= nl: the bound holds)
-                    emit_list(sh, nl, k, row, co);
+                    emit_list(sh, nl, k, row, co, threadIdx.x);
                     exact = true;
                 }
             }
@@ -423,8 +423,8 @@ namespace q3k
         // positive values come first and the negative ones in value order after them,
         // it is bounded once more from the registers (rows of log-probabilities, 1 / 64 /
         // 256 x 151936 at k = 20: 10.6 / 11.8 / 19.1 us; 20.8 / 22.1 / 108 when they were read
-        // again, twice).  Only a row too short for that is read again, by
-        // select_reading.  Non-finite: the signed maximum reaches +inf's bits or the
+        // again, twice).  Only a row whose bound is the lowest finite value is read again,
+        // by select_reading.  Non-finite: the signed maximum reaches +inf's bits or the
         // unsigned maximum -inf's.
         //
         // Bound for k <= kGroupK: the k-th largest of the 256 maxima of four threads
@@ -445,6 +445,10 @@ namespace q3k
         // Listing by wave segments (readlane a vector) measured 14.3 and 19.7.
         constexpr int kRegVecs = 20;
         constexpr int64_t kRegColumns = int64_t{8} * kRegVecs * kSelBlock;
+        // A row that fits five vectors a thread goes through no more (64 rows of 20000,
+        // k = 20 / 150 / 300: 5.8 / 7.3 / 8.9 us, 8.3 / 9.8 / 11.4 with twenty).
+        constexpr int kShortRegVecs = 5;
+        constexpr int64_t kShortRegColumns = int64_t{8} * kShortRegVecs * kSelBlock;
         constexpr uint32_t kGroupK = 192;
         constexpr int kRankSlots = 8; // list entries a lane holds
         constexpr uint32_t kRankList = kRankSlots * kWave;
@@ -577,6 +581,7 @@ namespace q3k
             select_reading(r, n, k, row, co, sh);
         }
 
+        template <int VECS>
         __global__ __launch_bounds__(kSelBlock) void topk_row_kernel(const uint16_t *__restrict__ x, int64_t rows,
                                                                      int64_t stride, int32_t n, uint32_t k, CandOut co,
                                                                      int32_t *__restrict__ count,
@@ -594,9 +599,9 @@ namespace q3k
                 const int32_t nv = (n - first) / 8;
                 const Vec8 *rv = reinterpret_cast<const Vec8 *>(r + first);
                 constexpr uint32_t kNone = 0xff7fff7fu; // an empty place: the lowest finite value
-                Vec8 v[kRegVecs];
+                Vec8 v[VECS];
 #pragma unroll
-                for (int u = 0; u < kRegVecs; ++u)
+                for (int u = 0; u < VECS; ++u)
                 {
                     v[u] = Vec8{{kNone, kNone, kNone, kNone}};
                     if (tid + u * kSelBlock < nv)
@@ -618,7 +623,7 @@ namespace q3k
                 // 1. maxima and the non-finite flag
                 uint32_t mi = side_bits | (kNone & 0xffff0000u), mu = mi;
 #pragma unroll
-                for (int u = 0; u < kRegVecs; ++u)
+                for (int u = 0; u < VECS; ++u)
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
                     {
@@ -660,7 +665,8 @@ namespace q3k
                         return static_cast<int32_t>(sh.bound);
                     }
                     return static_cast<int32_t>(
-                               block_kth([&](int i) { return sh.thread_max[i]; }, kSelBlock, k, sh.hist, sh.sel)) +
+                               block_kth([&](int i) { return sh.thread_max[i]; }, kSelBlock, k, sh.hist, sh.sel,
+                                         own_thread())) +
                            low;
                 };
                 share_maxima(0);
@@ -674,7 +680,7 @@ namespace q3k
                     // by the unsigned minima, a positive value counted as -0
                     uint32_t mn = side_bits | (kNone & 0xffff0000u);
 #pragma unroll
-                    for (int u = 0; u < kRegVecs; ++u)
+                    for (int u = 0; u < VECS; ++u)
 #pragma unroll
                         for (int j = 0; j < 4; ++j)
                             mn = min_u16x2(mn, v[u].d[j]);
@@ -706,7 +712,7 @@ namespace q3k
                         if (__builtin_expect(low < 0, 0))
                         {
 #pragma unroll
-                            for (int u = 0; u < kRegVecs; ++u)
+                            for (int u = 0; u < VECS; ++u)
                             {
                                 const uint32_t m = min_u16x2(min_u16x2(v[u].d[0], v[u].d[1]), min_u16x2(v[u].d[2], v[u].d[3]));
                                 mask |= reaches(low_u16(m)) ? 1u << u : 0u;
@@ -715,7 +721,7 @@ namespace q3k
                         else
                         {
 #pragma unroll
-                            for (int u = 0; u < kRegVecs; ++u)
+                            for (int u = 0; u < VECS; ++u)
                             {
                                 const uint32_t m = max_i16x2(max_i16x2(v[u].d[0], v[u].d[1]), max_i16x2(v[u].d[2], v[u].d[3]));
                                 mask |= top_i16(m) >= bound ? 1u << u : 0u;
@@ -729,7 +735,7 @@ namespace q3k
                         base = atomicAdd(&hits.count, total);
                     pos += __builtin_amdgcn_readfirstlane(base);
 #pragma unroll
-                    for (int u = 0; u < kRegVecs; ++u)
+                    for (int u = 0; u < VECS; ++u)
                         if ((mask >> u & 1u) != 0u)
                         {
                             if (pos < static_cast<uint32_t>(kCandMax))
@@ -766,7 +772,7 @@ namespace q3k
                         else if (nl <= kRankList)
                             emit_ranked<kRankSlots>(sh, nl, k, row, co, low);
                         else
-                            emit_list(sh, nl, k, row, co);
+                            emit_list(sh, nl, k, row, co, own_thread());
                         exact = true;
                     }
                 }
@@ -894,7 +900,7 @@ namespace q3k
                 const uint32_t nl = sh.listed;
                 if (nl <= static_cast<uint32_t>(kCandMax))
                 {
-                    emit_list(sh, nl, k, row, co);
+                    emit_list(sh, nl, k, row, co, threadIdx.x);
                     exact = true;
                 }
             }
@@ -908,9 +914,27 @@ namespace q3k
             }
         }
 
-        // Rows that topk_row_kernel does not take are cut into slices when fewer than
-        // kTargetBlocks blocks would run (and k <= kSelBlock); a slice keeps at least
-        // kMinSlice logits.
+        // Rows a block could hold in its registers; they are never cut into slices.
+        bool fits_registers(int64_t n, int32_t k) { return n <= kRegColumns && k <= kSelBlock; }
+
+        // Those that topk_row_kernel takes.  Its bound needs k groups of four threads with a
+        // vector each (k <= kGroupK); without them it would read the row again (64 rows of
+        // 1000 at k = 150 12.6 us, 9.2 in topk_select_kernel).  With them it is the faster one
+        // for small k (1000 columns at k = 20 5.6 us against 7.9); for larger k the radix
+        // steps, twice for a row with few positive logits, weigh more than the second read
+        // of a short row.  Ordinary rows / rows without a positive value, in us, against the
+        // same in topk_select_kernel: 64 x 8000 at k = 150 7.2 / 8.5 and 8.5 / 8.1, 12000
+        // 7.4 / 8.6 and 9.4 / 9.0; at k = 300 8000 8.7 / 11.6 and 8.9 / 8.4, 16000 8.8 / 11.7 and
+        // 10.6 / 10.2 (rows off 16 bytes 8.8 and 12.4), 24000 8.9 / 11.8 and 11.7 / 11.3.
+        bool takes_registers(int64_t n, int32_t k)
+        {
+            // 32 k: the columns of k groups' vectors, and up to seven on either side
+            const int64_t least = k <= 64 ? 32 * int64_t{k} + 14 : k <= static_cast<int32_t>(kGroupK) ? 12 * kSelBlock : 16 * kSelBlock;
+            return fits_registers(n, k) && n >= least;
+        }
+
+        // Rows longer than that are cut into slices when fewer than kTargetBlocks blocks
+        // would run (and k <= kSelBlock); a slice keeps at least kMinSlice logits.
         constexpr int64_t kTargetBlocks = 512;
         constexpr int64_t kMinSlice = 8 * kSelBlock;
         constexpr int kMaxSlices = kWave;
@@ -921,8 +945,6 @@ namespace q3k
             int64_t slice_len = 0;
             int64_t bytes = 0;
         };
-
-        bool fits_registers(int64_t n, int32_t k) { return n <= kRegColumns && k <= kSelBlock; }
 
         SlicePlan plan_slices(int64_t rows, int64_t n, int32_t k)
         {
@@ -979,10 +1001,15 @@ extern "C" int q3k_topk_candidates_bf16(const uint16_t *logits, int64_t rows, in
     const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const CandOut co{cap, cand_index, cand_logit};
     const unsigned grid = static_cast<unsigned>(rows < 65535 ? rows : 65535);
-    if (fits_registers(search_size, k))
+    if (takes_registers(search_size, k))
     {
-        topk_row_kernel<<<dim3(grid), dim3(kSelBlock), 0, s>>>(logits, rows, row_stride, static_cast<int32_t>(search_size),
-                                                                static_cast<uint32_t>(k), co, count, nonfinite);
+        const auto n = static_cast<int32_t>(search_size);
+        if (search_size <= kShortRegColumns)
+            topk_row_kernel<kShortRegVecs><<<dim3(grid), dim3(kSelBlock), 0, s>>>(
+                logits, rows, row_stride, n, static_cast<uint32_t>(k), co, count, nonfinite);
+        else
+            topk_row_kernel<kRegVecs><<<dim3(grid), dim3(kSelBlock), 0, s>>>(
+                logits, rows, row_stride, n, static_cast<uint32_t>(k), co, count, nonfinite);
         return check_launch("topk_candidates");
     }
     const SlicePlan plan = plan_slices(rows, search_size, k);

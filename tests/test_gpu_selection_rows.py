@@ -129,7 +129,11 @@ def test_argmax_time_without_positive_values(q3k, hip, synth):
     assert max(us["negative"], us["shifted"]) < 2.0 * us["ordinary"], us
 
 
-@pytest.mark.parametrize("n,ks", [(9, (1, 9)), (100, (1, 20, 100)), (8193, (20, 192, 193)), (20000, (1, 192, 1024, 1500)),
+# the shortest rows that the register kernel takes (32 k + 14 columns up to k = 64, 12288, above k = 192 16384) and the
+# ones below, the longest row of five vectors a thread (40960)
+@pytest.mark.parametrize("n,ks", [(9, (1, 9)), (45, (1,)), (46, (1, 2)), (100, (1, 20, 100)), (653, (20,)), (654, (20, 21)),
+                                  (2061, (64,)), (2062, (64, 65)), (12287, (65, 192)), (12288, (65, 192, 193)), (8193, (20, 192, 193)), (20000, (1, 192, 1024, 1500)),
+                                  (16383, (193, 1024)), (16384, (193, 1024)), (40960, (20, 193)), (40961, (20, 193)),
                                   (155649, (20, 193)), (163840, (1, 64, 192, 193, 1024)), (163841, (20, 1024)),
                                   (262145, (20, 300))])
 @pytest.mark.parametrize("pad,offset", [(0, 0), (3, 6)])
