@@ -381,25 +381,25 @@ namespace q3k
             return Q3K_OK;
         }
 
-        // Calls launch with the vectors a thread has in flight over `columns`: no more than
-        // they take, up to kUnroll (past the end each further one costs a thread about
-        // twenty instructions: 64 rows of 1000 2.9 us, 3.3 with five; 1 of 20000 3.0 and
-        // 3.2; 600 of 1000 4.0, with the waves that have no columns going through the
-        // motions as well 5.1).
+        // Calls launch with the vectors a thread has in flight over `columns`: up to kUnroll,
+        // as many as fill the fewest rounds (past the end each further one costs a thread
+        // about twenty instructions: 64 rows of 1000 2.9 us, 3.3 with five; 1 of 20000 3.0
+        // and 3.2; 42 of 86600, three rounds of four, 4.5 and 4.7 with five; 600 of 1000
+        // 4.0, with the waves that have no columns going through the motions as well 5.1).
         template <typename F>
         void with_unroll(int64_t columns, F launch)
         {
+            static_assert(kUnroll == 5, "instances");
             const int64_t vectors = (columns + 8 * kArgmaxBlock - 1) / (8 * kArgmaxBlock);
-            if (vectors <= 1)
-                launch(std::integral_constant<int, 1>{});
-            else if (vectors == 2)
-                launch(std::integral_constant<int, 2>{});
-            else if (vectors == 3)
-                launch(std::integral_constant<int, 3>{});
-            else if (vectors == 4)
-                launch(std::integral_constant<int, 4>{});
-            else
-                launch(std::integral_constant<int, kUnroll>{});
+            const int64_t rounds = (vectors + kUnroll - 1) / kUnroll;
+            switch ((vectors + rounds - 1) / rounds)
+            {
+            case 1: return launch(std::integral_constant<int, 1>{});
+            case 2: return launch(std::integral_constant<int, 2>{});
+            case 3: return launch(std::integral_constant<int, 3>{});
+            case 4: return launch(std::integral_constant<int, 4>{});
+            default: return launch(std::integral_constant<int, 5>{});
+            }
         }
 
         // Launches for checked arguments: the sliced kernels when `part`
