@@ -320,7 +320,7 @@ namespace q3k
         // 7.5, 262144 9.1 / 9.2, 300000 10.0 / 9.8; 256 of 151936 13.2 / 15.1, 262144 27.6 /
         // 27.4.)
         constexpr int64_t kWholeRowColumns = int64_t{1} << 18;
-        constexpr int64_t kWholeFewRowsColumns = 5 * 8 * kUnroll * kArgmaxBlock; // 204800: five loads a thread
+        constexpr int64_t kWholeFewRowsColumns = 5 * 8 * kUnroll * kArgmaxBlock; // 204800: five rounds of loads
         constexpr int64_t kFewRows = 32;
 
         struct SlicePlan
