@@ -235,8 +235,13 @@ namespace q3k
     // beside the others, so uneven CUs cost; one, two or four waves a block put
     // four, two or one block on a CU; start and end take 2.7 us with one wave, 3.3
     // with two and 4.5 with four (the groups' merge), another round of short blocks
-    // 2 us, the merge launch 3.8 us with its share of the host.
-    inline double attn_decode_us(int64_t pairs, int64_t cached, int waves, int64_t split_keys)
+    // 2 us, the merge launch 3.8 us with its share of the host.  Of more than 8 columns
+    // (several positions) the slices' fp32 results count too, 17 KB for 32 columns beside
+    // 33 KB of 64 keys: the first 12 MB written and read hide behind the slices, the rest
+    // goes at 6 TB/s (3 x 4 positions after 1843, 64 / 8 heads: 15.3 us in the slices taken
+    // without it, 13.3 with; over 220 shapes of 2 to 16 positions 0.7% less, none more
+    // than 2% slower, where counting every byte at 5 TB/s made 23 of them so).
+    inline double attn_decode_us(int64_t pairs, int64_t cols, int64_t cached, int waves, int64_t split_keys)
     {
         const int64_t keys = split_keys < cached ? split_keys : cached;
         const int64_t slices = blocks_for(cached, keys);
@@ -261,7 +266,12 @@ namespace q3k
         if (more > 0 && round_us(slots) < 20.0)
             us += 2.0 * static_cast<double>(more);
         if (slices > 1)
+        {
             us += 3.8 + 0.006 * static_cast<double>(slices);
+            const double moved = static_cast<double>(blocks * cols) * (2 * (kAttHeadDim + 2) * 4);
+            if (cols > 8 && moved > 12.0e6)
+                us += (moved - 12.0e6) / 6.0e6;
+        }
         return us;
     }
 
@@ -273,14 +283,14 @@ namespace q3k
     // 3000 of 16 / 8 105 us whole and 88 in three slices of four-wave blocks.
     inline AttnSplit plan_attention_decode(int64_t B, int64_t S, int32_t Hq, int32_t Hkv, int64_t cached, bool can_split)
     {
-        const int64_t pairs = B * Hkv;
+        const int64_t pairs = B * Hkv, cols = S * (Hq / Hkv);
         AttnSplit best, best_split;
         double best_us = -1.0, best_split_us = -1.0;
         for (const int waves : {4, 2, 1})
         {
             if (waves == 1 && cached > kAttDecodeTile)
                 continue;
-            const double us = attn_decode_us(pairs, cached, waves, cached);
+            const double us = attn_decode_us(pairs, cols, cached, waves, cached);
             if (best_us >= 0.0 && us >= best_us)
                 continue;
             best_us = us;
@@ -299,7 +309,7 @@ namespace q3k
             {
                 if ((waves == 1) != (keys <= kAttMaxOneWaveSplitKeys))
                     continue;
-                const double us = attn_decode_us(pairs, cached, waves, keys);
+                const double us = attn_decode_us(pairs, cols, cached, waves, keys);
                 if (best_split_us >= 0.0 && us >= best_split_us)
                     continue;
                 best_split_us = us;

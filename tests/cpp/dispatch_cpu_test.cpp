@@ -148,10 +148,26 @@ namespace
         }
     }
 
+    // The slices of several positions' columns: their fp32 results are half the keys' bytes at 64 keys a slice, so
+    // there are fewer of them than for one position's
+    void slice_cases()
+    {
+        using namespace q3k;
+        for (const int64_t start : {1843, 3932})
+        {
+            const AttnSplit one = plan_attention_split(3, 1, 64, 8, start + 1);
+            const AttnSplit four = plan_attention_split(3, 4, 64, 8, start + 4);
+            const std::string what = "3 sequences after " + std::to_string(start) + ", 64/8";
+            require(one.splits > 1 && four.splits > 1, what + ": not split");
+            require(3 * four.splits <= 2 * one.splits, what + ": as many slices for 32 columns as for 8");
+        }
+    }
+
     void body()
     {
         rope_cases();
         attention_cases();
+        slice_cases();
         merge_cases();
     }
 } // namespace
